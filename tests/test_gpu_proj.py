@@ -118,3 +118,14 @@ def test_attention_rows_feed_the_projection():
     want = O.proj_bf16(xb, w, t=S, k=H * D, n=n, x_dtype=O.BF16)
     mag = O.proj_bf16(abs_bits(xb), abs_bits(w), t=S, k=H * D, n=n, x_dtype=O.BF16)
     assert_sum_close(y.cpu().numpy(), want, 2 * H * D * U * mag, "attention -> proj")
+
+
+@pytest.mark.parametrize("t", [1, 2, 15, 16, 17, 32, 33, 63, 64])
+@pytest.mark.parametrize("k,n,ldx,ldy", [(64, 1, 0, 0), (576, 49, 584, 60), (4160, 130, 0, 0)])
+@pytest.mark.parametrize("xd,split", [(O.BF16, 0), (O.F32, 0), (O.F32, 1)], ids=["bf16", "f32", "split"])
+def test_few_rows(t, k, n, ldx, ldy, xd, split):
+    """proj_few: blocks of 16 rows of x (1, 2 and 4 of them, the last one partial), one K chunk, a few more than the
+    waves take together, many; part blocks of columns."""
+    got, want, mag = run_proj(np.random.default_rng(t + k), t, k, n, xd, split, ldx, ldy)
+    assert_sum_close(got[:, :n], want[:, :n], (4 if split else 2) * k * U * mag[:, :n], "proj")
+    assert (got[:, n:] == SENTINEL).all(), "a column past n was written"
