@@ -99,7 +99,9 @@ const char* mako_last_error(void);
  * the prefill kernel, one launch with no workspace. Heads of 256 take one launch with no workspace, or past its
  * offsets first write V as f16 V^T tiles into a workspace. mako_attn_fwd keeps that workspace itself, per (device, stream),
  * allocated stream-ordered the first time a call needs it (or more of it) and held until mako_attn_release(stream);
- * under graph capture a call that would grow it fails with MAKO_EWORKSPACE.
+ * under graph capture a call that would grow it fails with MAKO_EWORKSPACE. Prefill calls of heads of 64 and 128 whose
+ * query rows leave compute units idle split their keys in up to 128 MiB of that workspace; where it cannot be had
+ * (a capture, no memory) they run unsplit.
  */
 int mako_attn_fwd(const mako_attn_args* a, uint32_t dim, mako_dtype in, mako_dtype out, const void* q,
                   const void* k, const void* v, void* o, float* lse, void* stream);
@@ -107,8 +109,9 @@ int mako_attn_fwd(const mako_attn_args* a, uint32_t dim, mako_dtype in, mako_dty
 /*
  * mako_attn_fwd with the caller's workspace, for callers that own their scratch (the reference's Runtime owns it as
  * named scratch buffers: src/gpu/runtime.cpp:117-125; TransformerRuntime::attention passes scratch("attn_fwd")).
- * It allocates nothing; MAKO_EWORKSPACE when workspace_bytes is below mako_attn_fwd_workspace(a, dim) (0 for the
- * prefill routes: workspace may then be NULL). The workspace's contents do not matter before or after a call;
+ * It allocates nothing; MAKO_EWORKSPACE when workspace_bytes is below mako_attn_fwd_workspace(a, dim), except
+ * on the prefill routes, which run with any workspace or NULL (the query gives 0, or the bytes to split the keys with;
+ * with less they run unsplit). The workspace's contents do not matter before or after a call;
  * calls that overlap in time need separate workspaces.
  */
 size_t mako_attn_fwd_workspace(const mako_attn_args* a, uint32_t dim);

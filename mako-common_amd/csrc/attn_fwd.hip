@@ -628,11 +628,13 @@ int launch_attn_splitk(const mako_attn_args* a, mako_dtype in, mako_dtype out, c
                        const void* v, void* o, float* lse, hipStream_t s, const Workspace& work);
 
 // flash_fwd_r64 (attn_fwd64.hip): heads of 128 and 64 with 64 rows a wave; 1 launched, 0 when a size does not fit
-// its offsets. flash_fwd_d256: heads of 256; the same, or -1 when its workspace could not be had (the error
+// its offsets; fwd64_workspace: the bytes it can split the call's keys with (it also runs without). flash_fwd_d256: heads of 256; the same, or -1 when its workspace could not be had (the error
 // recorded); d256_workspace: the bytes it needs.
 template <class T, class TO, int D>
 int launch_fwd64(const mako_attn_args* a, float scale_log2, const void* q, const void* k, const void* v, void* o,
-                 float* lse, hipStream_t s);
+                 float* lse, hipStream_t s, const Workspace& work);
+template <int D>
+size_t fwd64_workspace(const mako_attn_args* a);
 size_t d256_workspace(const mako_attn_args* a);
 // flash_fwd_r32 (attn_fwd_r32.hip): heads of 256 with 32 rows a wave, staged from K and V's rows (no workspace);
 // 1 launched, 0 when a size does not fit its offsets (flash_fwd_d256 then takes the call).
@@ -661,8 +663,8 @@ bool launch_d(const mako_attn_args* a, uint32_t dim, const FwdParams& p, dim3 gr
               const Workspace& work)
 {
     if (!force_fallback()) {
-        const int r = dim == 128 ? launch_fwd64<T, TO, 128>(a, p.scale_log2, p.q, p.k, p.v, p.o, p.lse, s)
-                      : dim == 64 ? launch_fwd64<T, TO, 64>(a, p.scale_log2, p.q, p.k, p.v, p.o, p.lse, s)
+        const int r = dim == 128 ? launch_fwd64<T, TO, 128>(a, p.scale_log2, p.q, p.k, p.v, p.o, p.lse, s, work)
+                      : dim == 64 ? launch_fwd64<T, TO, 64>(a, p.scale_log2, p.q, p.k, p.v, p.o, p.lse, s, work)
                       : launch_fwd_r32<T, TO>(a, p.scale_log2, p.q, p.k, p.v, p.o, p.lse, s)
                           ? 1
                           : launch_fwd_d256<T, TO>(a, p.scale_log2, p.q, p.k, p.v, p.o, p.lse, s, nullptr, &work);
@@ -726,12 +728,15 @@ int attn_check(const mako_attn_args* a, uint32_t dim, mako_dtype in, mako_dtype 
 }
 
 // The workspace a dense call needs: the split-K partials (heads of 128, a few rows) or, for heads of 256 past
-// flash_fwd_r32's offsets (sized for an f32 output, the larger), flash_fwd_d256's V^T images; the prefill kernels
-// for heads of 64 and 128, and flash_fwd_r32, need none.
+// flash_fwd_r32's offsets (sized for an f32 output, the larger), flash_fwd_d256's V^T images; flash_fwd_r32 needs none.
+// The prefill kernel for heads of 64 and 128 needs none either, but takes fwd64_workspace to split the keys of calls
+// whose items leave CUs idle.
 size_t attn_fwd_workspace(const mako_attn_args* a, uint32_t dim)
 {
     if (dim == 128 && splitk_takes(a, dim))
         return splitk_workspace(a);
+    if ((dim == 64 || dim == 128) && a->kv_heads && a->heads && a->heads % a->kv_heads == 0)
+        return dim == 128 ? fwd64_workspace<128>(a) : fwd64_workspace<64>(a);
     return dim == 256 && !r32_fits(a, 4) ? d256_workspace(a) : 0;
 }
 

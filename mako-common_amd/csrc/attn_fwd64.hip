@@ -29,10 +29,15 @@
 // group at a time), so the K / V an XCD streams stays in its L2. The grid is persistent, one workgroup a CU, each
 // walking a fixed list of its XCD's items (heavy and light in turn for causal rows), so no CU idles on the
 // workgroup dispatcher between items (measured 3.5 us a handover with a grid of one workgroup an item).
+#include <algorithm>
+#include <type_traits>
+
 #include "fwd64_common.hpp"
 
 namespace mako {
 namespace {
+
+constexpr uint32_t kSplitBlocks = 128;  // query blocks a split call has at most: two a lane (SPLIT's item lookup)
 
 struct Fwd64Params {
     const void* q;
@@ -47,14 +52,47 @@ struct Fwd64Params {
     uint32_t n_items;    // n_hg x n_qblk workgroup items
 };
 
+// flash_fwd_r64's parameters with SPLIT: also tiles a piece at most; the pieces' results, po [pieces][n_q][heads][D]
+// normalised f32 and pl [pieces][heads][n_q] natural-log sums; and ends[i], the pieces a head group has in its last
+// i + 1 query blocks (past its n_qblk: 0xffff).
+struct SplitParams : Fwd64Params {
+    uint32_t piece_tiles;
+    float* po;
+    float* pl;
+    uint16_t ends[kSplitBlocks];
+};
+template <bool SPLIT>
+using R64Params = std::conditional_t<SPLIT, SplitParams, Fwd64Params>;
+
 // Keys row position pos sees are [0, lim(pos)).
 __device__ __forceinline__ uint32_t lim_of(uint32_t pos, uint32_t n_k, uint32_t block)
 {
     return pos >= block ? n_k : min(n_k, pos + 1);
 }
 
-template <class T, class TO, int D>
-__global__ __launch_bounds__(256, 1) void flash_fwd_r64(const Fwd64Params p)
+// The pieces an item's keys are cut into when the grid is split: np = ceil(nt / piece_tiles) nearly equal runs of
+// tiles, piece i from tile start(i) up to start(i + 1). The last ones start no later than the last tile that every row
+// of the item sees a key of, so no row is fully masked in the tile its piece starts with.
+struct Pieces {
+    uint32_t nt, np, tmax;
+    __host__ __device__ Pieces(uint32_t n_tiles, uint32_t first_row_keys, uint32_t piece_tiles)
+        : nt(n_tiles), np((n_tiles + piece_tiles - 1) / piece_tiles), tmax((first_row_keys - 1) / 64)
+    {
+    }
+    __host__ __device__ uint32_t start(uint32_t i) const
+    {
+        const uint32_t t = i * nt / np;
+        return i >= np ? nt : t < tmax ? t : tmax;
+    }
+};
+
+// With SPLIT a workgroup takes pieces of items: an item's keys are cut into pieces (Pieces), a piece leaves a normalised
+// f32 result and its log-sum, and merge_pieces combines them; an item of one piece is stored as without SPLIT. The
+// pieces are dealt as the items are. The grid holds no idle workgroups: past one a CU the dispatcher makes a workgroup
+// wait for its turn's shader engine even beside free CUs (192 pieces in a grid of 288: 35 us, alone 21).
+// For calls whose items do not fill the chip or whose longest item would run on alone (split_plan).
+template <class T, class TO, int D, bool SPLIT>
+__global__ __launch_bounds__(256, 1) void flash_fwd_r64(const R64Params<SPLIT> p)
 {
     using L = R64<D>;
     __shared__ __attribute__((aligned(1024))) unsigned char lds[L::kLdsBytes];
@@ -71,12 +109,26 @@ __global__ __launch_bounds__(256, 1) void flash_fwd_r64(const Fwd64Params p)
     const bool by_xcd = G % 8 == 0;
     const uint32_t g8 = G / 8, bx = b % 8, bk = b / 8;
     for (uint32_t round = 0;; ++round) {
+    // Item -> (head group, query block); with SPLIT the piece too.
+    uint32_t hg, qb, piece = 0;
+    if constexpr (SPLIT) {
+        // the list of a set of `per` head groups (an XCD's, or all): blocks of rows heaviest first, for each of them
+        // its pieces, for each piece the head groups
+        const bool xcd_list = by_xcd && p.n_hg % 8 == 0;
+        const uint32_t j = xcd_list ? round * g8 + (round % 2 == 0 ? bk : g8 - 1 - bk) : b + round * G;
+        const uint32_t per = xcd_list ? p.n_hg / 8 : p.n_hg;
+        const uint16_t e0 = p.ends[lane], e1 = p.ends[lane + 64];
+        const uint32_t qi = __popcll(__ballot(e0 * per <= j)) + __popcll(__ballot(e1 * per <= j));
+        if (qi >= p.n_qblk)
+            break;
+        const uint32_t r = j - (qi ? p.ends[qi - 1] * per : 0u);
+        qb = p.n_qblk - 1 - qi;
+        hg = (xcd_list ? bx + 8 * (r % per) : r % per);
+        piece = r / per;
+    } else {
     const uint32_t item = by_xcd ? bx + 8 * (round * g8 + (round % 2 == 0 ? bk : g8 - 1 - bk)) : b + round * G;
     if (item >= p.n_items)
         break;
-
-    // Item -> (head group, query block).
-    uint32_t hg, qb;
     const uint32_t id = item;
     if (p.n_hg % 8 == 0) {
         const uint32_t x = id % 8, kx = id / 8, per = p.n_hg / 8;
@@ -91,21 +143,34 @@ __global__ __launch_bounds__(256, 1) void flash_fwd_r64(const Fwd64Params p)
         hg = id % p.n_hg;
         qb = p.n_qblk - 1 - id / p.n_hg;
     }
+    }
     const uint32_t h = hg * p.hq + w % p.hq;
     const uint32_t kvh = hg * p.hq / p.group;
     const uint32_t wg_q0 = qb * p.rows_wg;
     const uint32_t q0 = wg_q0 + (w / p.hq) * 64;  // this wave's first row
 
     const uint32_t wg_last = p.q_pos0 + min(wg_q0 + p.rows_wg, p.n_q) - 1;
-    const uint32_t n_keys = wg_last >= p.block ? p.n_k : min(p.n_k, wg_last + 1);
+    uint32_t n_keys = wg_last >= p.block ? p.n_k : min(p.n_k, wg_last + 1);
+    // the piece's first key: limits and counts below are relative to it
+    uint32_t ks = 0;
+    bool partial = false;
+    if constexpr (SPLIT) {
+        const Pieces pc((n_keys + 63) / 64, lim_of(p.q_pos0 + wg_q0, p.n_k, p.block), p.piece_tiles);
+        if (pc.start(piece) >= pc.start(piece + 1))
+            continue;  // an empty piece (prefix-causal rows: most of the keys lie past the first row's)
+        partial = pc.np > 1;
+        ks = 64 * pc.start(piece);
+        n_keys = min(n_keys, 64 * pc.start(piece + 1)) - ks;
+    }
     const bool live = q0 < p.n_q;
     const uint32_t w_last = p.q_pos0 + min(q0 + 64, p.n_q) - 1;
-    const uint32_t w_keys = !live ? 0u : (w_last >= p.block ? p.n_k : min(p.n_k, w_last + 1));
+    const uint32_t w_lim = !live ? 0u : (w_last >= p.block ? p.n_k : min(p.n_k, w_last + 1));
+    const uint32_t w_keys = SPLIT && live ? min(n_keys, w_lim - ks) : w_lim;
     const uint32_t nt = (n_keys + 63) / 64, ntw = (w_keys + 63) / 64;
     const uint32_t p0 = p.q_pos0 + q0;
-    const uint32_t lmin = lim_of(p0, p.n_k, p.block);
-    const uint32_t lim0 = lim_of(p0 + c32, p.n_k, p.block) - 8 * g;
-    const uint32_t lim1 = lim_of(p0 + 32 + c32, p.n_k, p.block) - 8 * g;
+    const uint32_t lmin = lim_of(p0, p.n_k, p.block) - ks;
+    const uint32_t lim0 = lim_of(p0 + c32, p.n_k, p.block) - ks - 8 * g;
+    const uint32_t lim1 = lim_of(p0 + 32 + c32, p.n_k, p.block) - ks - 8 * g;
 
     // LDS: the K images, then the V images.
     const uint32_t lbase = (uint32_t)reinterpret_cast<uintptr_t>(lds);
@@ -138,24 +203,33 @@ __global__ __launch_bounds__(256, 1) void flash_fwd_r64(const Fwd64Params p)
     // row R at c ^ (R % 8)). ew: where the lane's pieces of row c32 go (with the lane's part of the chunk index and
     // the swizzle; the stream xors in the rest); er: the first whole-row chunk it reads back (lane l: row l / lpr,
     // chunk l % lpr, lpr = lanes a row); og: where that chunk goes in o; ogs: o bytes of one read's rows.
-    constexpr uint32_t so = sizeof(TO), orow = D * so, lpr = orow / 16;
+    const uint32_t so = SPLIT && partial ? 4u : (uint32_t)sizeof(TO), orow = D * so, lpr = orow / 16;
+    const uint32_t width = SPLIT && partial ? p.heads * D : p.width;
     const uint32_t obase = lbase + w * 64 * orow;
     const uint32_t ew = so == 4 ? obase + c32 * orow + 16 * ((c32 & 7u) ^ g)
                                 : obase + c32 * orow + 8 * g + 16 * (c32 & 7u);
     const uint32_t er = obase + (lane / lpr) * orow + 16 * ((lane % lpr) ^ (lane / lpr));
-    const uint32_t og = (q0 + lane / lpr) * p.width * so + h * orow + 16 * (lane % lpr);
-    const uint32_t ogs = __builtin_amdgcn_readfirstlane((64 / lpr) * p.width * so);
+    const uint32_t og = (q0 + lane / lpr) * width * so + h * orow + 16 * (lane % lpr);
+    const uint32_t ogs = __builtin_amdgcn_readfirstlane((64 / lpr) * width * so);
     const uint32_t lo0 = q0 + c32 < p.n_q ? (h * p.n_q + q0 + c32) * 4 : 0xffffffffu;
     const uint32_t lo1 = q0 + 32 + c32 < p.n_q ? (h * p.n_q + q0 + 32 + c32) * 4 : 0xffffffffu;
     const uint32_t swp = (lane ^ 32) * 4;
 
     const u32x4 qrs = rsrc_of(static_cast<const T*>(p.q) + (size_t)h * p.q_pad * D, p.n_q * 2 * D);
-    const u32x4 krs = rsrc_of(static_cast<const T*>(p.k) + (size_t)kvh * p.k_pad * D, n_keys * 2 * D);
-    const u32x4 vrs = rsrc_of(static_cast<const T*>(p.vs) + (size_t)kvh * p.k_pad * D, n_keys * 2 * D);
-    const u32x4 ors = rsrc_of(p.o, p.n_q * p.width * so);
-    const u32x4 lrs = rsrc_of(p.lse, p.lse ? p.heads * p.n_q * 4 : 0);
+    const u32x4 krs = rsrc_of(static_cast<const T*>(p.k) + ((size_t)kvh * p.k_pad + ks) * D, n_keys * 2 * D);
+    const u32x4 vrs = rsrc_of(static_cast<const T*>(p.vs) + ((size_t)kvh * p.k_pad + ks) * D, n_keys * 2 * D);
+    void* out = p.o;
+    float* lse = p.lse;
+    if constexpr (SPLIT) {
+        if (partial) {
+            out = p.po + (size_t)piece * p.n_q * width;
+            lse = p.pl + (size_t)piece * p.heads * p.n_q;
+        }
+    }
+    const u32x4 ors = rsrc_of(out, p.n_q * width * so);
+    const u32x4 lrs = rsrc_of(lse, lse ? p.heads * p.n_q * 4 : 0);
     // scalar operands, made wave-uniform explicitly (the asm reads them from scalar registers)
-    const uint32_t has_lse = __builtin_amdgcn_readfirstlane(p.lse ? 1u : 0u);
+    const uint32_t has_lse = __builtin_amdgcn_readfirstlane(lse ? 1u : 0u);
     const float c = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(uint32_t, p.scale_log2)));
     const uint32_t s_nt = __builtin_amdgcn_readfirstlane(nt), s_ntw = __builtin_amdgcn_readfirstlane(ntw);
     const uint32_t s_lmin = __builtin_amdgcn_readfirstlane(lmin);
@@ -175,33 +249,73 @@ __global__ __launch_bounds__(256, 1) void flash_fwd_r64(const Fwd64Params p)
       [skww] "s"(skww), [svww] "s"(svww)                                                                          \
     : MAKO_FWD64_CLOBBERS, "vcc", "scc", "memory"
 
+#define MAKO_FWD64_STREAM(NAME, OUT16)                                                                            \
+    do {                                                                                                        \
+        if (__is_same(TO, float) || (SPLIT && partial))                                                         \
+            asm volatile(NAME##_F32 MAKO_FWD64_OPERANDS);                                                       \
+        else                                                                                                    \
+            asm volatile(NAME##_##OUT16 MAKO_FWD64_OPERANDS);                                                   \
+    } while (0)
+
     if constexpr (D == 64) {
-        if constexpr (__is_same(T, __bf16)) {
-            if constexpr (__is_same(TO, float))
-                asm volatile(MAKO_FWD64_D64_ASM_BF16_F32 MAKO_FWD64_OPERANDS);
-            else
-                asm volatile(MAKO_FWD64_D64_ASM_BF16_BF16 MAKO_FWD64_OPERANDS);
-        } else {
-            if constexpr (__is_same(TO, float))
-                asm volatile(MAKO_FWD64_D64_ASM_F16_F32 MAKO_FWD64_OPERANDS);
-            else
-                asm volatile(MAKO_FWD64_D64_ASM_F16_F16 MAKO_FWD64_OPERANDS);
-        }
+        if constexpr (__is_same(T, __bf16))
+            MAKO_FWD64_STREAM(MAKO_FWD64_D64_ASM_BF16, BF16);
+        else
+            MAKO_FWD64_STREAM(MAKO_FWD64_D64_ASM_F16, F16);
     } else if constexpr (__is_same(T, __bf16)) {
-        if constexpr (__is_same(TO, float))
-            asm volatile(MAKO_FWD64_ASM_BF16_F32 MAKO_FWD64_OPERANDS);
-        else
-            asm volatile(MAKO_FWD64_ASM_BF16_BF16 MAKO_FWD64_OPERANDS);
+        MAKO_FWD64_STREAM(MAKO_FWD64_ASM_BF16, BF16);
     } else {
-        if constexpr (__is_same(TO, float))
-            asm volatile(MAKO_FWD64_ASM_F16_F32 MAKO_FWD64_OPERANDS);
-        else
-            asm volatile(MAKO_FWD64_ASM_F16_F16 MAKO_FWD64_OPERANDS);
+        MAKO_FWD64_STREAM(MAKO_FWD64_ASM_F16, F16);
     }
     // every wave's stream has ended (its LDS reads landed) before the next item's staging overwrites LDS
     asm volatile("s_barrier" ::: "memory");
     }
+#undef MAKO_FWD64_STREAM
 #undef MAKO_FWD64_OPERANDS
+}
+
+// The rows of items with more than one piece, from query row row0 on: the pieces' normalised rows weighted by
+// exp(their log-sum - the largest). D / 4 lanes a (row, head), four head dims each; bound by the read of the pieces.
+template <class TO, int D>
+__global__ __launch_bounds__(256) void merge_pieces(const SplitParams p, uint32_t row0)
+{
+    const uint32_t t = blockIdx.x * (1024 / D) + threadIdx.x / (D / 4), d = 4 * (threadIdx.x % (D / 4));
+    const uint32_t row = row0 + t / p.heads, h = t % p.heads;
+    if (row >= p.n_q)
+        return;
+    const uint32_t wg_q0 = row / p.rows_wg * p.rows_wg, last = p.q_pos0 + min(wg_q0 + p.rows_wg, p.n_q) - 1;
+    const Pieces pc((lim_of(last, p.n_k, p.block) + 63) / 64, lim_of(p.q_pos0 + wg_q0, p.n_k, p.block), p.piece_tiles);
+    const float* pl = p.pl + (size_t)h * p.n_q + row;
+    const float* po = p.po + ((size_t)row * p.heads + h) * D + d;
+    const size_t ls = (size_t)p.heads * p.n_q, os = ls * D;
+    constexpr uint32_t U = 4;  // pieces whose loads are in flight together
+    float mx = -INFINITY, sum = 0.0f;
+    f32x4 acc = f32x4{};
+    for (uint32_t i0 = 0; i0 < pc.np; i0 += U) {
+        float l[U];
+        f32x4 v[U];
+        #pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {  // (an empty piece wrote nothing)
+            const bool has = i0 + u < pc.np && pc.start(i0 + u) < pc.start(i0 + u + 1);
+            l[u] = has ? pl[(i0 + u) * ls] : -INFINITY;
+            v[u] = has ? *reinterpret_cast<const f32x4*>(po + (i0 + u) * os) : f32x4{};
+        }
+        #pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            const float m = fmaxf(mx, l[u]);
+            if (m == -INFINITY)
+                continue;
+            const float a = exp2_fast((mx - m) * kLog2e), b = exp2_fast((l[u] - m) * kLog2e);
+            sum = sum * a + b;
+            acc = acc * a + v[u] * b;
+            mx = m;
+        }
+    }
+    const float inv = sum != 0.0f ? 1.0f / sum : 0.0f;
+    store4<TO>(static_cast<TO*>(p.o) + (size_t)row * p.width + (size_t)h * D + d, acc[0] * inv, acc[1] * inv,
+               acc[2] * inv, acc[3] * inv);
+    if (p.lse && d == 0)
+        p.lse[(size_t)h * p.n_q + row] = sum != 0.0f ? mx + __log2f(sum) * kLn2 : -INFINITY;
 }
 
 // Heads of 256 (Qwen3.5's gated attention): flash_fwd_d256. The parallelism of the usual shapes (16 query heads,
@@ -535,12 +649,106 @@ bool d256_fits(const mako_attn_args* a)
            (uint64_t)a->q_pad * 512 < (1ull << 31) && n_qblk <= 65535;
 }
 
-// Launches flash_fwd_r64 for heads of D (128 or 64) on stream s: one launch, no workspace (K and V are staged from
-// their rows). Returns 1 when launched, 0 (launching nothing) when a size does not fit the kernel's 32-bit buffer
-// offsets (the caller then uses flash_fwd).
+namespace {
+
+// How a call's keys are split over workgroups (pieces 1: they are not).
+struct SplitPlan {
+    uint32_t piece_tiles = 0, pieces = 1;
+    uint32_t row0 = 0;  // the first query row of an item with more than one piece
+    size_t o_bytes = 0, bytes = 0;
+};
+
+// The 64-key tiles the items of query block qb walk.
+uint32_t item_tiles(const mako_attn_args* a, uint32_t rows_wg, uint32_t qb)
+{
+    const uint32_t last = a->q_pos0 + std::min((qb + 1) * rows_wg, a->n_q) - 1;
+    return ((last >= a->block ? a->n_k : std::min(a->n_k, last + 1)) + 63) / 64;
+}
+
+// An estimate in microseconds, from this kernel's times: a workgroup takes kTileUs a tile of 64 keys on an otherwise
+// idle chip and kFullUs more where every CU works (the clock drops), kWgUs around them (dispatch, prologue, epilogue)
+// and kTurnUs for each further piece; the merge kMergeUs and its read of the pieces. A plan must gain 15 %.
+// Measured at 32 / 8 heads of 128, unsplit and split: 333 rows over 9333 keys 174 -> 61 us, 100 over 32868 591 -> 70,
+// 17 over 3017 61 -> 20, 1000 over 10000 188 -> 140; 8 / 2 heads, causal 2048 rows 43 -> 28. Not split: causal 1531
+// rows of 32 heads (192 items of 1 to 24 tiles: the chip's clock and the merge take back what the shorter path gives);
+// causal 4096 rows (512 items, heavy and light in turn).
+template <int D>
+SplitPlan split_plan(const mako_attn_args* a, uint32_t cus)
+{
+    constexpr double kTileUs = D == 128 ? 1.25 : 0.8, kFullUs = D == 128 ? 0.5 : 0.2, kWgUs = 8, kTurnUs = 3;
+    constexpr double kMergeUs = 5;
+    constexpr size_t kMaxBytes = 128u << 20;
+    SplitPlan best;
+    const uint32_t group = a->heads / a->kv_heads;
+    const uint32_t hq = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
+    const uint32_t rows_wg = 256 / hq, n_hg = a->heads / hq, n_qblk = (a->n_q + rows_wg - 1) / rows_wg;
+    const uint64_t n_items = (uint64_t)n_hg * n_qblk;
+    if (!cus || !a->n_k || !a->n_q || n_items > 4ull * cus || n_qblk > kSplitBlocks ||
+        (uint64_t)a->q_pos0 + a->n_q + 256 > 0xffffffffull)
+        return best;
+    const auto tiles = [&](uint32_t qb) { return item_tiles(a, rows_wg, qb); };
+    const uint32_t nt = tiles(n_qblk - 1);
+    const bool even = 2 * tiles(0) > nt;
+    uint64_t total = 0;
+    for (uint32_t qb = 0; qb < n_qblk; ++qb)
+        total += (uint64_t)n_hg * tiles(qb);
+    // the busiest CU's tiles: whole rounds of equal items, or a CU's share
+    const auto path = [&](uint64_t n, double longest) {
+        return even ? (double)((n + cus - 1) / cus) * longest : std::max(longest, (double)total / cus);
+    };
+    const double full_us = kFullUs * total / cus;
+    double best_us = 0.85 * (kTileUs * path(n_items, nt) + full_us + kWgUs);
+    for (uint32_t np = 2; np <= 16 && nt / np >= 6; ++np) {
+        SplitPlan s;
+        s.piece_tiles = (nt + np - 1) / np;
+        s.pieces = np;
+        s.o_bytes = ((size_t)np * a->n_q * a->heads * D * 4 + 255) / 256 * 256;
+        s.bytes = s.o_bytes + (size_t)np * a->heads * a->n_q * 4;
+        if (s.bytes > kMaxBytes)
+            break;
+        uint64_t n = 0, merged = 0;  // pieces; pieces' rows the merge reads
+        s.row0 = a->n_q;
+        for (uint32_t qb = 0; qb < n_qblk; ++qb) {
+            const uint32_t k = (tiles(qb) + s.piece_tiles - 1) / s.piece_tiles;
+            n += (uint64_t)n_hg * k;
+            if (k > 1) {
+                merged += (uint64_t)k * rows_wg * a->heads;
+                s.row0 = std::min(s.row0, qb * rows_wg);
+            }
+        }
+        // (the lists deal equal pieces evenly; of unequal ones a second round would put two long ones on a CU)
+        if (!even && n > cus)
+            continue;
+        const double us = kTileUs * path(n, s.piece_tiles) + full_us + kWgUs + kTurnUs * (double)((n - 1) / cus) +
+                          kMergeUs + merged * D * 4.0 / 4.5e6;
+        if (us < best_us) {
+            best_us = us;
+            best = s;
+        }
+    }
+    return best;
+}
+
+}  // namespace
+
+// The bytes flash_fwd_r64's split grid keeps its pieces in for this call (0: it runs unsplit). Only an offer: with
+// less, or none, the call runs unsplit.
+template <int D>
+size_t fwd64_workspace(const mako_attn_args* a)
+{
+    const SplitPlan s = split_plan<D>(a, device_cus());
+    return s.pieces > 1 ? s.bytes : 0;
+}
+template size_t fwd64_workspace<128>(const mako_attn_args*);
+template size_t fwd64_workspace<64>(const mako_attn_args*);
+
+// Launches flash_fwd_r64 for heads of D (128 or 64) on stream s: one launch with no workspace (K and V are staged from
+// their rows), or the split grid and its merge where split_plan finds it faster and work has the memory (a stream that
+// captures, or a caller without a workspace, keeps the one launch). Returns 1 when launched, 0 (launching nothing) when
+// a size does not fit the kernel's 32-bit buffer offsets (the caller then uses flash_fwd).
 template <class T, class TO, int D>
 int launch_fwd64(const mako_attn_args* a, float scale_log2, const void* q, const void* k, const void* v, void* o,
-                 float* lse, hipStream_t s)
+                 float* lse, hipStream_t s, const Workspace& work)
 {
     const uint32_t group = a->heads / a->kv_heads;
     const uint32_t hq = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
@@ -548,18 +756,41 @@ int launch_fwd64(const mako_attn_args* a, float scale_log2, const void* q, const
     const uint32_t n_qblk = (a->n_q + rows_wg - 1) / rows_wg;
     if (!fwd64_fits<D>(a, sizeof(TO)))
         return 0;
-    const uint32_t n_vt = (a->n_k + 63) / 64;
-    const uint32_t n_items = a->heads / hq * n_qblk;
+    const uint32_t n_vt = (a->n_k + 63) / 64, n_hg = a->heads / hq, n_items = n_hg * n_qblk;
+    const uint32_t cus = device_cus();
+    const SplitPlan sp = split_plan<D>(a, cus);
+    char* ws = nullptr;
+    // (a caller's workspace for another route of the call may be short or unaligned: no error here)
+    if (sp.pieces > 1 && !(work.given && (work.bytes < sp.bytes || reinterpret_cast<uintptr_t>(work.ptr) % 16)))
+        ws = static_cast<char*>(work.get(sp.bytes, s));
     const Fwd64Params p{q, k, v, o, lse, a->n_q, a->q_pad, a->n_k, a->k_pad, a->heads, a->kv_heads, a->q_pos0,
-                        a->block, a->width, scale_log2, group, hq, rows_wg, n_qblk, a->heads / hq, n_vt, n_items};
-    const uint32_t grid = std::min<uint32_t>(n_items, std::max<uint32_t>(1, device_cus()));
-    hipLaunchKernelGGL((flash_fwd_r64<T, TO, D>), dim3(grid), dim3(256), 0, s, p);
+                        a->block, a->width, scale_log2, group, hq, rows_wg, n_qblk, n_hg, n_vt, n_items};
+    if (ws) {
+        SplitParams ps;
+        static_cast<Fwd64Params&>(ps) = p;
+        ps.piece_tiles = sp.piece_tiles;
+        ps.po = reinterpret_cast<float*>(ws);
+        ps.pl = reinterpret_cast<float*>(ws + sp.o_bytes);
+        uint32_t n = 0;
+        for (uint32_t i = 0; i < kSplitBlocks; ++i) {
+            if (i < n_qblk)
+                n += (item_tiles(a, rows_wg, n_qblk - 1 - i) + sp.piece_tiles - 1) / sp.piece_tiles;
+            ps.ends[i] = i < n_qblk ? (uint16_t)n : 0xffff;
+        }
+        hipLaunchKernelGGL((flash_fwd_r64<T, TO, D, true>), dim3(std::min(n * n_hg, cus)), dim3(256), 0, s, ps);
+        const uint64_t rows = (uint64_t)(a->n_q - sp.row0) * a->heads, per = 1024 / D;
+        hipLaunchKernelGGL((merge_pieces<TO, D>), dim3((uint32_t)((rows + per - 1) / per)), dim3(256), 0, s, ps,
+                           sp.row0);
+        return 1;
+    }
+    const uint32_t grid = std::min<uint32_t>(n_items, std::max<uint32_t>(1, cus));
+    hipLaunchKernelGGL((flash_fwd_r64<T, TO, D, false>), dim3(grid), dim3(256), 0, s, p);
     return 1;
 }
 
 #define MAKO_FWD64_INSTANCE(T, TO, D)                                                                            \
     template int launch_fwd64<T, TO, D>(const mako_attn_args*, float, const void*, const void*, const void*, void*, \
-                                        float*, hipStream_t);
+                                        float*, hipStream_t, const Workspace&);
 MAKO_FWD64_INSTANCE(__bf16, float, 128)
 MAKO_FWD64_INSTANCE(__bf16, __bf16, 128)
 MAKO_FWD64_INSTANCE(_Float16, float, 128)

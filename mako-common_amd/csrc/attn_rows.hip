@@ -30,7 +30,7 @@ int launch_fwd_r32(const mako_attn_args* a, float scale_log2, const void* q, con
                    float* lse, hipStream_t s);
 template <class T, class TO, int D>
 int launch_fwd64(const mako_attn_args* a, float scale_log2, const void* q, const void* k, const void* v, void* o,
-                 float* lse, hipStream_t s);
+                 float* lse, hipStream_t s, const Workspace& work);
 template <class T, class TO>
 int launch_fwd_d256(const mako_attn_args* a, float scale_log2, const void* q, const void* k, const void* v, void* o,
                     float* lse, hipStream_t s, const void* vt_ready, const Workspace* work);
@@ -108,7 +108,7 @@ int launch_rows(const mako_attn_args* t, const HeadsParams& pq, const HeadsParam
     else if constexpr (D == 256)
         r = launch_fwd_r32<T, TO>(t, sl2, pq.y, pk.y, pvt.y, o, lse, s);
     else
-        r = launch_fwd64<T, TO, D>(t, sl2, pq.y, pk.y, pvt.y, o, lse, s);
+        r = launch_fwd64<T, TO, D>(t, sl2, pq.y, pk.y, pvt.y, o, lse, s, images);
     if (r <= 0)  // (the route was chosen where the kernel fits and its images are given)
         return fail(MAKO_EHIP, "attention from rows: the attention kernel refused a checked call");
     return check_launch("attention from rows");
