@@ -22,6 +22,14 @@
 // Items (head, query tile) go head-major, with every head on one XCD at a time when the heads are a multiple of 8
 // (the head's K / V then stay in that XCD's L2), and the query tiles from the last (dense tiles, which see every key)
 // to the first.
+//
+// Padding is not computed. Cubes cut by the video's edge hold few valid rows in runs of 16 (the last frame layer: one
+// run of four), so a tile of 32 keys is two groups of 16 consecutive keys with a valid one, from anywhere in the
+// sequence, and a workgroup's query rows are those with an output, packed. 56 heads, 9 frames of 34 x 60 patches, 948
+// dense rows: 53 -> 43 thousand tiles a head, 4.33 -> 3.6 ms; one frame (16 of 64 rows valid) 901 -> 511 us with the
+// selection; no padding (4 frames of 32 x 32) 273 -> 276 us. Groups of 8 keys would save another 6 % of the first
+// case's tiles, at four sources a tile. The loop is bound by its chain of barrier, scores, softmax and P V (MFMA a
+// third busy at two waves a SIMD).
 #include "fwd64_common.hpp"
 
 namespace mako {
@@ -33,7 +41,9 @@ constexpr uint32_t kLKRow = 2 * kLD + 16;         // 272: LDS bytes of a K image
 constexpr uint32_t kLKImg = 9 * 1024;             // the K image (8704 bytes) and what its ninth 1 KiB piece spills
 constexpr uint32_t kLVImg = kLKeys * 2 * kLD;     // 8 KiB: the V image
 constexpr uint32_t kLBuf = kLKImg + kLVImg + 64;  // and the tile's 32 validity bytes
-constexpr uint32_t kLMaxSel = 256;                 // list entries a query tile (two cube tiles each)
+constexpr uint32_t kLMaxSel = 256;                 // list entries a query tile
+constexpr uint32_t kLGroup = 16;                  // keys a group: a tile is two groups from anywhere
+constexpr uint32_t kLList = 514;                  // groups held at a time (a scan's 512 and one carried over)
 constexpr float kLRescale = 8.0f;
 
 struct ListsParams {
@@ -136,8 +146,8 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     using E = Elem<_Float16>;
     using V8 = f16x8;
     __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kLBuf];
-    __shared__ uint32_t lst[2 * kLMaxSel];  // the first keys of the cube tiles visited, in list order
-    __shared__ uint32_t lcnt[2];
+    __shared__ __attribute__((aligned(8))) uint32_t lst[kLList];  // the groups visited, in order: K / V byte offsets
+    __shared__ uint32_t lcnt[2], lcut;  // lcut: the last group crosses the end of the dense rows
 
     const uint32_t tid = threadIdx.x, lane = tid & 63;
     const uint32_t w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -153,15 +163,31 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             return;
     }
     const uint32_t kvh = h / p.group;
-    const uint32_t q0 = qt * 64 + 32 * w, row = q0 + c32;  // this wave's first row, this lane's row
-    const bool live = q0 < p.n_q;
-
-    // The tiles: a cube tile's selected cubes (two tiles each), then its dense rows; a later tile's keys [0, n_k).
+    // The keys: a cube tile's selected cubes, then its dense rows; a later tile's keys [0, n_k). The list's first
+    // entries, its length and the tile's row map are loaded together, Q and the first validity bytes after them: two
+    // round trips before the first tile's.
     const bool cube = qt < p.n_cubes;
     const uint16_t* my_sel = p.sel + ((size_t)h * p.n_cubes + (cube ? qt : 0u)) * p.max_sel;
+    const int32_t map_l = qt * 64 + lane < p.n_q ? p.map[qt * 64 + lane] : -1;
+    const uint32_t sel_first = cube && tid < p.max_sel ? my_sel[tid] : 0u;
     const uint32_t ns = cube ? min(uniform_u16(p.nsel, (size_t)h * p.n_cubes + qt), p.max_sel) : 0u;
     const uint32_t dlo = cube ? p.dense0 : 0u, dhi = cube ? p.dense1 : p.n_k;
-    const uint32_t nd = dhi > dlo ? (dhi - dlo + kLKeys - 1) / kLKeys : 0u;
+    const uint32_t nd = dhi > dlo ? (dhi - dlo + 63) / 64 : 0u;
+    // The rows: those of the tile's 64 that have an output (the others, a partly filled cube's padding, are not
+    // computed), packed in order, 32 a wave; a lane past the last one computes a row of zeros and stores nothing.
+    uint32_t row, n_rows;
+    {
+        const bool has = map_l >= 0;
+        const uint64_t bal = __ballot(has);
+        n_rows = (uint32_t)__builtin_popcountll(bal);
+        const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
+        // lane rank of `packed` gets the lane of the rank-th such row (the others are pushed behind, in any order)
+        const uint32_t at = has ? rank : n_rows + lane - rank;
+        const int packed = __builtin_amdgcn_ds_permute((int)(4 * at), (int)lane);
+        row = qt * 64 + (uint32_t)__builtin_amdgcn_ds_bpermute((int)(4 * (32 * w + c32)), packed);
+    }
+    const bool stores = 32 * w + c32 < n_rows;
+    const uint32_t row_lo = __builtin_amdgcn_readfirstlane(row);  // this wave's first row
 
     // Sources: the kv head's k_pad rows of K and V, the k_pad validity bytes (offsets past them load zeros).
     u32x4 krs = rsrc_of(static_cast<const _Float16*>(p.k) + (size_t)kvh * p.k_pad * kLD, p.k_pad * 2 * kLD);
@@ -177,48 +203,55 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // slot_of(R) of the tile), chunk (that % 272) / 16; chunk 16 (the row's padding) and rows past 31 (the spill of
     // piece 8) load any bytes of the tile. Wave w DMAs pieces 4 w .. 4 w + 3 and piece 8 (both waves: the same bytes
     // to the same place). V image piece i: keys 4 i .. 4 i + 3, lane l's slot holds the unit lv_unit places there.
+    // slot_of keeps a row's 16, so rows 0 .. 15 come from the tile's first group and 16 .. 31 from its second: pieces
+    // 0 .. 3 are the first group's, 5 .. 8 the second's, piece 4 holds row 15's end and rows 16 .. 18. Offsets are
+    // within the group.
     auto kd_of = [&](uint32_t i) {
         const uint32_t b = 1024 * i + 16 * lane, r = b / kLKRow, ch = b % kLKRow / 16;
-        return r < kLKeys && ch < 16 ? slot_of(r) * (2 * kLD) + 16 * ch : 0u;
+        return r < kLKeys && ch < 16 ? (slot_of(r) % kLGroup) * (2 * kLD) + 16 * ch : 0u;
     };
     uint32_t kd[5], vd[4];
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
         kd[m] = kd_of(4 * w + m);
-        vd[m] = 1024 * (4 * w + m) + lv_src(lane);
+        vd[m] = 1024 * m + lv_src(lane);
     }
     kd[4] = kd_of(8);
+    const bool second = 1024 * 4 + 16 * lane >= kLGroup * kLKRow;  // piece 4's lane is the second group's
     const uint32_t lbase = __builtin_amdgcn_readfirstlane((uint32_t)reinterpret_cast<uintptr_t>(lds));
     // A tile's K image and validity bytes, and its V image, into buffer buf.
-    auto dma_k = [&](uint32_t j0, uint32_t buf) __attribute__((always_inline)) {
+    // (ta, tb: the tile's groups; the wave's own is ta for wave 0 and tb for wave 1)
+    auto dma_k = [&](uint32_t ta, uint32_t tb, uint32_t buf) __attribute__((always_inline)) {
         const uint32_t kb = lbase + buf * kLBuf;
-        const uint32_t so = __builtin_amdgcn_readfirstlane(j0 * 2 * kLD);
+        const uint32_t so = w == 0 ? ta : tb;
+        if (w == 0)
+            dma16_at(kb, kd[0], so, krs);
+        else
+            dma16_at(kb + 1024 * 4, kd[0] + (second ? tb : ta), 0, krs);
 #pragma unroll
-        for (int m = 0; m < 4; ++m)
+        for (int m = 1; m < 4; ++m)
             dma16_at(kb + 1024 * (4 * w + m), kd[m], so, krs);
-        dma16_at(kb + 1024 * 8, kd[4], so, krs);
+        dma16_at(kb + 1024 * 8, kd[4], tb, krs);
         if (w == 0 && lane < 2)
-            dma16_at(kb + kLKImg + kLVImg, 16 * lane, j0, brs);
+            dma16_at(kb + kLKImg + kLVImg, (lane ? tb : ta) / (2 * kLD), 0, brs);
     };
-    auto dma_v = [&](uint32_t j0, uint32_t buf) __attribute__((always_inline)) {
+    auto dma_v = [&](uint32_t ta, uint32_t tb, uint32_t buf) __attribute__((always_inline)) {
         const uint32_t vb = lbase + buf * kLBuf + kLKImg;
-        const uint32_t so = __builtin_amdgcn_readfirstlane(j0 * 2 * kLD);
+        const uint32_t so = w == 0 ? ta : tb;
 #pragma unroll
         for (int m = 0; m < 4; ++m)
             dma16_at(vb + 1024 * (4 * w + m), vd[m], so, vrs);
     };
 
-    // Q: the B operand, lane (c32, g) holds row q0 + c32, head dims 16 kk + 8 g .. + 7 (rows past n_q load as 0).
+    // Q: the B operand, lane (c32, g) holds its row's head dims 16 kk + 8 g .. + 7 (no row: an offset past the end,
+    // zeros).
     V8 qreg[8];
     {
         const auto qrs = buffer_rsrc(static_cast<const _Float16*>(p.q) + (size_t)h * p.q_pad * kLD, p.n_q * 2 * kLD);
-        const uint32_t off = (row * kLD + 8 * g) * 2;
+        const uint32_t off = ((stores ? row : p.n_q) * kLD + 8 * g) * 2;
 #pragma unroll
         for (int kk = 0; kk < 8; ++kk)
             qreg[kk] = __builtin_bit_cast(V8, buffer_load16(qrs, off + 32 * kk));
-#pragma unroll
-        for (int kk = 0; kk < 8; ++kk)
-            settle(qreg[kk]);
     }
     // V^T reads: in each 16-lane group G, lane 4 j + y addresses head dims 16 (G % 2) + 4 y .. + 3 of key 8 (G / 2)
     // + j (+ 4 for the second read, + 16 for keys 16 .. 31) of 32-dim block db, and receives those dims' values for
@@ -230,53 +263,98 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int d4 = 0; d4 < 4; ++d4)
         vbase[d4] = (8 * g + gj) * (2 * kLD) + 32 * lv_unit(2 * d4 + gg, gj) + 8 * gy;
 
-    // The tile sequence: the cube tiles of the list that hold a valid key (not the padding halves of partly
-    // filled cubes) and, causal, start at or before the workgroup's last row, then the dense tiles. The cube tiles
-    // are found once, before the loop: thread i takes candidate i of each 128 (list entry i / 2, half i % 2), reads
-    // its 32 validity bytes, and the kept ones are packed in order into lst (ballot, then each lane's rank). The
-    // loop then reads one LDS word a tile instead of two dependent scalar loads a candidate.
+    // The key sequence: the groups of 16 keys of the listed cubes, then of the dense rows, that hold a valid key (not
+    // the padding of partly filled cubes) and, causal, start at or before the workgroup's last row; a tile is two
+    // consecutive ones, wherever they lie. A scan finds the groups of 128 blocks of 64 keys (a cube, or 64 dense rows)
+    // at once: thread i reads the 64 validity bytes of block i and the kept groups are packed in order into lst
+    // (ballots, then each lane's rank); the next scan runs when the groups are used up (dense query tiles, which see
+    // every key; long lists), an odd last group going to the front of the new ones.
     const uint32_t wg_last = qt * 64 + 63;
-    uint32_t ncl = 0;
-    for (uint32_t r0 = 0; r0 < 2 * ns; r0 += 128) {
-        const uint32_t r = r0 + tid;
-        bool keep = false;
-        uint32_t j0 = 0;
-        if (r < 2 * ns) {
-            j0 = (uint32_t)my_sel[r >> 1] * 64 + kLKeys * (r & 1);
-            const u32x4 a = *reinterpret_cast<const u32x4*>(p.valid + j0);
-            const u32x4 b = *reinterpret_cast<const u32x4*>(p.valid + j0 + 16);
-            keep = ((a[0] | a[1]) | (a[2] | a[3]) | (b[0] | b[1]) | (b[2] | b[3])) != 0 && (!CAUSAL || j0 <= wg_last);
+    const uint32_t n_blk = ns + nd;
+    uint32_t blk = 0, used = 0, held = 0;  // the next block to scan; groups of lst taken, and held
+    auto scan = [&]() __attribute__((always_inline)) {
+        __syncthreads();  // both waves are done with lst
+        uint32_t n = 0;
+        if (used < held) {
+            const uint32_t carry = lst[used];
+            __syncthreads();
+            if (tid == 0)
+                lst[0] = carry;
+            n = 1;
         }
-        const uint64_t bal = __ballot(keep);
+        const uint32_t i = blk + tid;
+        uint32_t keep = 0, j0 = 0, hi = 0;
+        if (i < n_blk) {
+            const bool listed = i < ns;
+            j0 = listed ? (blk ? (uint32_t)my_sel[i] : sel_first) * 64 : dlo + 64 * (i - ns);
+            hi = listed ? j0 + 64 : min(dhi, j0 + 64);
+            u32x4 f[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                f[k] = j0 + kLGroup * k < hi ? *reinterpret_cast<const u32x4*>(p.valid + j0 + kLGroup * k) : u32x4{};
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (((f[k][0] | f[k][1]) | (f[k][2] | f[k][3])) != 0 && (!CAUSAL || j0 + kLGroup * k <= wg_last))
+                    keep |= 1u << k;
+        }
+        uint64_t bal[4];
+        uint32_t total = 0, rank = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            bal[k] = __ballot((keep >> k) & 1u);
+            total += (uint32_t)__builtin_popcountll(bal[k]);
+            rank += __builtin_amdgcn_mbcnt_hi((uint32_t)(bal[k] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal[k], 0u));
+        }
         if (lane == 0)
-            lcnt[w] = (uint32_t)__builtin_popcountll(bal);
+            lcnt[w] = total;
         __syncthreads();
-        const uint32_t base = ncl + (w == 1 ? lcnt[0] : 0u);
-        const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
-        if (keep)
-            lst[base + rank] = j0;
-        ncl += lcnt[0] + lcnt[1];
-        __syncthreads();  // lcnt is rewritten by the next round; lst is complete after the last
-    }
-    ncl = __builtin_amdgcn_readfirstlane(ncl);
-    const uint32_t ntl = ncl + nd;
-    auto next_tile = [&](uint32_t& r, uint32_t& j0, uint32_t& hi) __attribute__((always_inline)) {
-        if (r >= ntl)
-            return false;
-        if (r < ncl) {
-            j0 = __builtin_amdgcn_readfirstlane(lst[r]);
-            hi = (j0 | 63u) + 1;  // the cube's end
-        } else {
-            j0 = dlo + kLKeys * (r - ncl);
-            hi = dhi;
-            if (CAUSAL && j0 > wg_last)  // the dense tiles ascend: none after this one either
+        uint32_t at = n + (w == 1 ? lcnt[0] : 0u) + rank;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if ((keep >> k) & 1u) {
+                const uint32_t j = j0 + kLGroup * k;
+                lst[at++] = j * (2 * kLD);
+                if (j + kLGroup > hi)
+                    lcut = 1;
+            }
+        held = __builtin_amdgcn_readfirstlane(n + lcnt[0] + lcnt[1]);
+        used = 0;
+        blk += 128;
+        __syncthreads();  // lst is complete
+    };
+    // The next tile's groups; both waves make the same calls, so they scan together. When the last tile is taken,
+    // last_mask gets the keys it has (an odd tile's second group, and past the end of the dense rows, none).
+    uint32_t last_mask = 0xffffffffu;
+    if (tid == 0)
+        lcut = 0;
+    auto next_tile = [&](uint32_t& ja, uint32_t& jb) __attribute__((always_inline)) {
+        if (used + 2 >= held) {
+            while (held - used < 2 && blk < n_blk)
+                scan();
+            if (used >= held)
                 return false;
         }
-        ++r;
+        const u32x2 pair = *reinterpret_cast<const u32x2*>(lst + used);  // (used is even)
+        ja = __builtin_amdgcn_readfirstlane(pair[0]);
+        jb = __builtin_amdgcn_readfirstlane(pair[1]);
+        used += 2;
+        if (used >= held && blk >= n_blk) {
+            const bool odd = used > held;
+            if (odd)
+                jb = ja;  // (any bytes)
+            used = held;
+            if (__builtin_amdgcn_readfirstlane(lcut)) {
+                const uint32_t keys = (1u << (dhi - (odd ? ja : jb) / (2 * kLD))) - 1;
+                last_mask = odd ? keys : keys << 16 | 0xffffu;
+            } else if (odd) {
+                last_mask = 0xffffu;
+            }
+        }
         return true;
     };
 
-    // S^T of the tile whose K image is in buffer buf: register r holds key j0 + 16 (r / 8) + 8 g + r % 8.
+    // S^T of the tile whose K image is in buffer buf: register r holds key 8 g + r % 8 of
+    // the tile's group r / 8.
     auto k_scores = [&](uint32_t buf) __attribute__((always_inline)) {
         f32x16 sc = f32x16{};
         const unsigned char* kr = lds + buf * kLBuf + c32 * kLKRow + 16 * g;
@@ -285,15 +363,16 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             sc = E::mfma32(*reinterpret_cast<const V8*>(kr + 32 * kk), qreg[kk], sc);
         return sc;
     };
-    // bit i: key j0 + i of the tile in buffer buf valid and before the pass's end
-    auto tile_mask = [&](uint32_t j0, uint32_t hi, uint32_t buf) __attribute__((always_inline)) {
+    // bit i: key i % 16 of group i / 16 of the tile in buffer buf is valid (last: and one of the last tile's keys)
+    auto tile_mask = [&](bool last, uint32_t buf) __attribute__((always_inline)) {
         const uint32_t vflag = lds[buf * kLBuf + kLKImg + kLVImg + c32];
-        return (uint32_t)__ballot(vflag != 0 && j0 + c32 < hi);
+        const uint32_t vm = (uint32_t)__ballot(vflag != 0);
+        return last ? vm & last_mask : vm;
     };
-    // -inf for the scores of keys not seen: invalid, past the pass's end or (causal) past the lane's row. Without
+    // -inf for the scores of keys not seen: invalid, past the end of the keys or (causal) past the lane's row. Without
     // the causal limit, register r's key is a wave-uniform bit of vmask for each lane half (8 g + r % 8 + 16 (r / 8)),
     // so its lane mask is two bit tests on the scalar unit and the masking one v_cndmask a register.
-    auto mask_scores = [&](f32x16& sc, uint32_t vmask, uint32_t j0) __attribute__((always_inline)) {
+    auto mask_scores = [&](f32x16& sc, uint32_t vmask, uint32_t ja, uint32_t jb) __attribute__((always_inline)) {
         if (!CAUSAL && vmask != 0xffffffffu) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
@@ -302,14 +381,12 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                                       (((vmask >> (b + 8)) & 1u) ? 0xffffffff00000000ull : 0ull);
                 sc[r] = keep_or_ninf(sc[r], keep);
             }
-        } else if (CAUSAL && (vmask != 0xffffffffu || j0 + kLKeys - 1 > q0)) {
+        } else if (CAUSAL && (vmask != 0xffffffffu || max(ja, jb) / (2 * kLD) + kLGroup - 1 > row_lo)) {
             const uint32_t lm = ((vmask >> (8 * g)) & 0xffu) | (((vmask >> (16 + 8 * g)) & 0xffu) << 8);
-            const int lim = CAUSAL ? (int)row - (int)j0 : 1 << 30;  // keys j0 + kidx <= row
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const int kidx = 16 * (r >> 3) + 8 * (int)g + (r & 7);
-                const bool seen = ((lm >> r) & 1u) && (!CAUSAL || kidx <= lim);
-                sc[r] = seen ? sc[r] : -INFINITY;
+                const uint32_t j = (r < 8 ? ja : jb) / (2 * kLD) + 8 * g + (r & 7);
+                sc[r] = ((lm >> r) & 1u) && j <= row ? sc[r] : -INFINITY;
             }
         }
     };
@@ -324,50 +401,53 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // Two stages: iteration t computes tile t + 1's scores (its K image, DMA'd an iteration ahead of V) beside
     // tile t's exponentials and P V. Buffer t % 2 holds K(t) and V(t); at iteration t, K(t + 2) and its validity
     // bytes go to the slot K(t) left and V(t + 1) to the slot V(t - 1) left.
-    uint32_t r = 0, ja = 0, ha = 0, jb = 0, hb = 0;
-    const bool ta = next_tile(r, ja, ha);
-    bool tb = ta && next_tile(r, jb, hb);
+    uint32_t a0 = 0, a1 = 0, b0 = 0, b1 = 0;  // the groups of tiles t and t + 1
+    const bool ta = next_tile(a0, a1);
+    bool tb = ta && next_tile(b0, b1);
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk)
+        settle(qreg[kk]);
     if (ta) {
-        dma_k(ja, 0);
-        dma_v(ja, 0);
+        dma_k(a0, a1, 0);
+        dma_v(a0, a1, 0);
     }
     if (tb)
-        dma_k(jb, 1);
+        dma_k(b0, b1, 1);
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-    // A wave none of whose 32 rows has an output (the padding rows of a partly filled cube: in H3's layout the
-    // second wave of every cube of the last, one-frame cube layer) computes nothing: it stages its share of each
-    // tile and keeps the barriers of the other wave's loop, then leaves.
-    if (__ballot(live && row < p.n_q && p.map[row] >= 0) == 0) {
+    // A wave with no row to compute (tiles of at most 32 rows with an output) stages its share of each tile and keeps
+    // the barriers of the other wave's loop, then leaves.
+    if (32 * w >= n_rows) {
         uint32_t bl = 0;
         for (bool have_l = ta; have_l;) {
-            uint32_t jc = 0, hc = 0;
-            const bool tc = tb && next_tile(r, jc, hc);
+            uint32_t c0 = 0, c1 = 0;
+            const bool tc = tb && next_tile(c0, c1);
             asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
             if (tc)
-                dma_k(jc, bl);
+                dma_k(c0, c1, bl);
             if (tb)
-                dma_v(jb, bl ^ 1);
+                dma_v(b0, b1, bl ^ 1);
             have_l = tb;
             tb = tc;
-            jb = jc;
+            b0 = c0;
+            b1 = c1;
             bl ^= 1;
         }
         return;
     }
     f32x16 s_cur = k_scores(0);
-    mask_scores(s_cur, tile_mask(ja, ha, 0), ja);
+    mask_scores(s_cur, tile_mask(!tb, 0), a0, a1);
     uint32_t b = 0;
     bool have = ta;
     while (have) {
-        uint32_t jc = 0, hc = 0;
-        const bool tc = tb && next_tile(r, jc, hc);
+        uint32_t c0 = 0, c1 = 0;
+        const bool tc = tb && next_tile(c0, c1);
         // this wave's DMAs of K(t + 1) and V(t) have landed; past the barrier, the other wave's too, and neither
         // reads the slots of K(t) and V(t - 1) any more
         asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
         if (tc)
-            dma_k(jc, b);
+            dma_k(c0, c1, b);
         if (tb)
-            dma_v(jb, b ^ 1);
+            dma_v(b0, b1, b ^ 1);
         // tile t's row maxima and the rescale decision
         const float mx0 = max3(s_cur[0], s_cur[1], s_cur[2]), mx1 = max3(s_cur[3], s_cur[4], s_cur[5]);
         const float mx2 = max3(s_cur[6], s_cur[7], s_cur[8]), mx3 = max3(s_cur[9], s_cur[10], s_cur[11]);
@@ -386,7 +466,7 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 for (int rr = 0; rr < 16; ++rr)
                     oacc[db][rr] *= f;
         // tile t + 1's scores (stale bytes when there is none: never used) beside tile t's exponentials
-        const uint32_t vmask_n = tile_mask(jb, hb, b ^ 1);
+        const uint32_t vmask_n = tile_mask(!tc, b ^ 1);
         f32x16 s_nxt = k_scores(b ^ 1);
         const float mu = m == -INFINITY ? 0.0f : m;
         V8 pb[2];
@@ -414,31 +494,28 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 const V8 a = __builtin_bit_cast(V8, __builtin_shufflevector(lo, hi4, 0, 1, 2, 3, 4, 5, 6, 7));
                 oacc[db] = E::mfma32(a, pb[cc], oacc[db]);
             }
-        mask_scores(s_nxt, vmask_n, jb);
+        mask_scores(s_nxt, vmask_n, b0, b1);
         s_cur = s_nxt;
         have = tb;
         tb = tc;
-        jb = jc;
-        hb = hc;
+        b0 = c0;
+        b1 = c1;
         b ^= 1;
     }
 
     // Normalise and store through the row map; the LSE by tile row.
     const float lt = pair_sum(l);
     const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
-    if (live && row < p.n_q) {
-        const int32_t dst = p.map[row];
-        if (dst >= 0) {
-            TO* orow = static_cast<TO*>(p.o) + (size_t)dst * p.width + (size_t)h * kLD;
+    if (stores) {
+        TO* orow = static_cast<TO*>(p.o) + (size_t)p.map[row] * p.width + (size_t)h * kLD;
 #pragma unroll
-            for (int db = 0; db < 4; ++db)
+        for (int db = 0; db < 4; ++db)
 #pragma unroll
-                for (int r4 = 0; r4 < 4; ++r4)
-                    store4<TO>(orow + 32 * db + 8 * r4 + 4 * g, oacc[db][4 * r4] * inv, oacc[db][4 * r4 + 1] * inv,
-                               oacc[db][4 * r4 + 2] * inv, oacc[db][4 * r4 + 3] * inv);
-            if (p.lse && g == 0)
-                p.lse[(size_t)h * p.q_pad + row] = lt > 0.0f ? (m + __log2f(lt)) * kLn2 : -INFINITY;
-        }
+            for (int r4 = 0; r4 < 4; ++r4)
+                store4<TO>(orow + 32 * db + 8 * r4 + 4 * g, oacc[db][4 * r4] * inv, oacc[db][4 * r4 + 1] * inv,
+                           oacc[db][4 * r4 + 2] * inv, oacc[db][4 * r4 + 3] * inv);
+        if (p.lse && g == 0)
+            p.lse[(size_t)h * p.q_pad + row] = lt > 0.0f ? (m + __log2f(lt)) * kLn2 : -INFINITY;
     }
 }
 

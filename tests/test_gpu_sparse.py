@@ -325,3 +325,46 @@ def test_per_head_lists(heads, kv, causal, dt, cubes, dense, cut, topk):
         assert np.all(o[~written] == SENTINEL), "rows outside the map were written"
         rows = np.nonzero(map_ >= 0)[0]
         G.assert_lse_close(lse[:, rows], want_l[:, rows], "lse")
+
+
+@pytest.mark.parametrize("causal,dense", [(0, 71), (1, 200)])
+def test_per_head_lists_in_groups(causal, dense):
+    """The key sequence of a list per query head, in groups of 16 keys with a valid one: groups missing anywhere (odd
+    counts, cubes and dense rows with none), lists and dense query tiles of more blocks than one scan takes (128), tiles
+    with no row, one, 32 and 33 rows to compute; one row of every query tile and 200 more against the oracle."""
+    heads, cubes, topk, dt = 2, 150, 145, O.F16
+    n = cubes * 64 + dense
+    q_pad, k_pad = (n + 63) // 64 * 64, (n + 127) // 128 * 128
+    rng = np.random.default_rng(7 + causal)
+    group = rng.random(k_pad // 16) < 0.6
+    valid = (np.repeat(group, 16) & (rng.random(k_pad) < 0.9)).astype(np.uint8)
+    valid[3 * 64:4 * 64] = 0
+    valid[n:] = 0
+    map_ = np.where(valid[:q_pad] == 1, 0, -1).astype(np.int32)
+    for tile, rows in ((5, 1), (6, 32), (7, 33), (8, 64)):
+        map_[tile * 64:tile * 64 + 64] = -1
+        map_[tile * 64 + rng.permutation(64)[:rows]] = 0
+    live = np.nonzero(map_ >= 0)[0]
+    map_[live] = rng.permutation(len(live)).astype(np.int32)
+    sel = np.zeros((heads, cubes, topk), np.uint16)
+    nsel = np.zeros((heads, cubes), np.uint16)
+    for h in range(heads):
+        for c in range(cubes):
+            ch = rng.permutation(cubes)[:topk if c % 2 else rng.integers(0, topk + 1)]
+            sel[h, c, :len(ch)] = ch
+            nsel[h, c] = len(ch)
+    qb, kb, vb = (G.randn_bits(rng, (heads, pad, 128), dt) for pad in (q_pad, k_pad, k_pad))
+    args = dict(n_q=n, q_pad=q_pad, n_k=n, k_pad=k_pad, heads=heads, kv_heads=heads, n_cubes=cubes, max_sel=topk,
+                dense0=cubes * 64, dense1=n, causal=causal, sel_heads=heads)
+    print(f"lists in groups, causal {causal}", flush=True)
+    o, lse = run_sparse(G.to_dev(qb, dt), G.to_dev(kb, dt), G.to_dev(vb, dt), dev_u16(sel), dev_u16(nsel), dev(valid),
+                        dev(map_), out=torch.float32, o_rows=len(live), **args)
+    first = [live[live // 64 == t][0] for t in np.unique(live // 64)]
+    rows = np.concatenate([first, rng.choice(live, 200), live[np.isin(live // 64, (5, 6, 7, 8))]])
+    hr = np.stack([rng.integers(0, heads, len(rows)), rows], 1).astype(np.uint32)
+    want_o, want_l = O.attn_sparse_rows(qb, kb, vb, sel, nsel, valid, hr, dtype=dt, **args)
+    got = np.stack([o[map_[r], h * 128:(h + 1) * 128] for h, r in hr])
+    G.assert_attn_close(got, want_o, "output")
+    G.assert_rows_l2(got, want_o, "output", 128)
+    G.assert_lse_close(np.array([lse[h, r] for h, r in hr]), want_l, "lse")
+    assert np.all(o != SENTINEL)
