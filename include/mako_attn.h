@@ -314,7 +314,7 @@ int mako_idx_dots(const mako_idx_dot_args* a, uint32_t tokens, const float* q, c
  * mako_gemm_args is GemmArgs (gemm.metal:18-22, src/mtl/gemm.cpp:13-15) field for field: row_bytes is the weight
  * row's bytes (2 k for BF16), ldy / ldx the row strides of y / x in elements (0: n / k). w bf16 [n][k]; y f32
  * [t][ldy]. x_dtype MAKO_BF16: x is bf16 [t][ldx], e.g. the attention output written in bf16 by mako_attn_fwd (no
- * conversion pass); MAKO_F32: x is f32 [t][ldx] and its rounding to bf16 (to_bf16, gemm.metal:676-681) happens in
+ * conversion pass); MAKO_F32: x is f32 [t][ldx] and is rounded to bf16 (to_bf16, gemm.metal:676-681) first, or in
  * the GEMM's loads. split (f32 x only): Runtime's bf16_split_ (src/gpu/runtime.cpp:184-203; set by the Qwen encoders,
  * src/models/qwen_text.cpp:271): the rounding's remainder bf16(x - bf16(x)) goes through the GEMM too and adds into
  * y. k a multiple of 64 (the reference's "BF16 {k}x{n}: k must be a multiple of 64"); w and x 16-byte aligned, ldx a
@@ -328,6 +328,16 @@ typedef struct mako_gemm_args {
 
 int mako_proj_bf16(const mako_gemm_args* a, int x_dtype, int split, const void* w, const void* x, float* y,
                    void* stream);
+
+/*
+ * mako_proj_bf16 with the caller's workspace. f32 x is rounded to bf16 once, into mako_proj_bf16_workspace(a, x_dtype,
+ * split) bytes (0: nothing to round ahead; at most 256 MiB); mako_proj_bf16 keeps them itself per (device, stream) until
+ * mako_attn_release. With less, none, or under a capture that would have to allocate, the GEMM rounds in its loads
+ * instead (slower, the same rounding).
+ */
+size_t mako_proj_bf16_workspace(const mako_gemm_args* a, int x_dtype, int split);
+int mako_proj_bf16_ws(const mako_gemm_args* a, int x_dtype, int split, const void* w, const void* x, float* y,
+                      void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * The gated delta rule with a decay per channel: kda_scan (src/kernels/ops.metal:459-519), run by the linear-

@@ -5,7 +5,8 @@
 //   y[r][c] = sum_j w[c][j] * bf16(x[r][j])  (+ sum_j w[c][j] * bf16(x[r][j] - bf16(x[r][j])) with split)
 //
 // The design is this one's own. Bound: MFMA (a 4096-token, 4096 x 4096 projection is 137 GFLOP against 67 MB of
-// output and 64 MB of operands). A workgroup of 4 waves computes a BM x 256 tile of y (BM = 256; 128 with split),
+// output and 64 MB of operands); the read of w for a few rows. Routes: proj_few (few rows), proj_dma and proj_ring (bf16
+// rows, and f32 rows after round_rows), proj_tiles (f32 rows without a workspace to round into). In proj_tiles a workgroup of 4 waves computes a BM x 256 tile of y (BM = 256; 128 with split),
 // each wave a (BM / 2) x 128 block as 32 x 32 MFMA blocks (v_mfma_f32_32x32x16_bf16) accumulating in f32.
 // 64-wide K chunks of x rows and w rows go through LDS, two buffers with one barrier a chunk; the next chunk waits in
 // registers while the current one is multiplied, and is stored, and the one after fetched, behind the first MFMAs. Both operands are K-contiguous rows, so every 16-byte run of a row
@@ -13,6 +14,9 @@
 // c ^ ((r / 2) % 8), so the 16 lanes of a ds_read_b128 (16 consecutive rows, one run) and of a ds_write_b128 (two
 // rows, eight runs) hit 64 distinct banks. f32 activations are rounded to bf16 (to nearest even) as they are
 // staged: the reference's separate to_bf16 pass (and its bf16 copy of x in HBM) is gone.
+#include <algorithm>
+#include <type_traits>
+
 #include "device.hpp"
 
 namespace mako {
@@ -26,6 +30,7 @@ struct ProjParams {
     float* y;         // [t][ldy]
     uint32_t t, k, n, ldy, ldx;
     uint32_t tiles_m, tiles_n, tiles, per_xcd;
+    uint32_t planes;  // bf16 x of the DMA kernels: 2 when a row's k values are followed by k remainders (ldx covers both)
 };
 
 // Tile q of the output walks bands of 4 tile rows column by column, and XCD x takes tiles x * per_xcd .. (workgroup
@@ -238,6 +243,19 @@ constexpr int kEK = 64;
 
 __device__ __forceinline__ uint32_t epos(uint32_t row, uint32_t run) { return row * kEK + ((run ^ ((row >> 1) & 7u)) << 3); }
 
+// The DMA is issued as inline asm: the compiler, seeing the builtin, waits for every DMA in flight before any LDS read
+// (it cannot tell the stages apart). Here the only waits are the stage barriers'. M0 (the DMA's LDS base) is listed as
+// clobbered; nothing else in these kernels uses it.
+__device__ __forceinline__ void dma_lds(uint32_t voff, uint32_t soff, u32x4 rs, uint32_t lds)
+{
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rs),
+                 "s"(__builtin_amdgcn_readfirstlane(soff))
+                 : "memory", "m0");
+#pragma clang diagnostic pop
+}
+
 __global__ __launch_bounds__(256, 1) void proj_dma(const ProjParams a)
 {
     __shared__ __attribute__((aligned(16))) __bf16 as[2][kBN * kEK];
@@ -258,26 +276,16 @@ __global__ __launch_bounds__(256, 1) void proj_dma(const ProjParams a)
     const u32x4 xrs = panel_rsrc(x + (size_t)t0 * a.ldx, a.t - t0, a.ldx);
     const u32x4 wrs = panel_rsrc(a.w + (size_t)n0 * a.k, a.n - n0, a.k);
     const uint32_t wl = __builtin_amdgcn_readfirstlane(64 * w * kEK * 2);  // this wave's first row, LDS bytes
-    // The DMA is issued as inline asm: the compiler, seeing the builtin, waits for every DMA in flight before any LDS
-    // read (it cannot tell the stages apart). Here the only waits are the stage barriers'. M0 (the DMA's LDS base) is
-    // listed as clobbered; nothing else in this kernel uses it.
-    auto dma = [&](uint32_t voff, uint32_t soff, u32x4 rs, uint32_t lds) __attribute__((always_inline)) {
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff),
-                     "s"(rs), "s"(soff)
-                     : "memory", "m0");
-#pragma clang diagnostic pop
-    };
+    const uint32_t nk = a.k / kEK, nq = nk * a.planes;  // K stages of w (>= 1), and of x's planes
     const uint32_t abase = (uint32_t)(uintptr_t)&as[0][0] + wl, bbase = (uint32_t)(uintptr_t)&bs[0][0] + wl;
     // DMA instruction i (0 .. 15) of K stage q (values 64 q .. 64 q + 63) into LDS stage q % 2: x piece i / 2 (8 rows)
     // for even i, w piece i / 2 for odd
     auto dma1 = [&](uint32_t q, int i) __attribute__((always_inline)) {
         const uint32_t so = 2 * kEK * q, st = (q & 1) * (kBN * kEK * 2) + 1024 * (i / 2);
         if (i % 2 == 0)
-            dma(xo[i / 2], so, xrs, abase + st);
+            dma_lds(xo[i / 2], so, xrs, abase + st);
         else
-            dma(wo[i / 2], so, wrs, bbase + st);
+            dma_lds(wo[i / 2], q < nk ? so : so - 2 * a.k, wrs, bbase + st);
     };
     f32x16 acc[4][4];
     #pragma unroll
@@ -316,7 +324,6 @@ __global__ __launch_bounds__(256, 1) void proj_dma(const ProjParams a)
     };
     using Y = std::true_type;
     using N = std::false_type;
-    const uint32_t nq = a.k / kEK;  // >= 1
     Frag fa, fb;
     #pragma unroll
     for (int i = 0; i < 16; ++i)
@@ -373,6 +380,142 @@ __global__ __launch_bounds__(256, 1) void proj_dma(const ProjParams a)
     }
 }
 
+// The same in smaller tiles, for calls that make too few 256 x 256 ones for the chip: BM x BN a workgroup, 2 x 2 waves
+// of BM / 2 x BN / 2, and a ring of NST K stages, since a small tile multiplies a stage in less time than its DMA takes
+// to land: after barrier q, stage q + NST - 1 goes out into the slot stage q - 1 left, and the wait before the barrier
+// leaves the NST - 2 stages after q in flight. Past the last stage the DMA reads it again (into slots nothing reads any
+// more), so the waits' counts hold to the end; the last ones land before the wave ends.
+template <int BM, int BN, int NST>
+__global__ __launch_bounds__(256, 1) void proj_ring(const ProjParams a)
+{
+    constexpr int MB = BM / 64, NB = BN / 64, NM = MB * NB, NR = MB + NB, XD = BM / 32, ND = XD + BN / 32;
+    constexpr uint32_t kStage = (BM + BN) * kEK;  // values a stage: BM x rows, then BN w rows
+    __shared__ __attribute__((aligned(16))) __bf16 lds[NST * kStage];
+    uint32_t tm, tn;
+    if (!tile_of(a, tm, tn))
+        return;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 5, c32 = lane & 31;
+    const uint32_t t0 = tm * BM, n0 = tn * BN;
+    // this wave's DMA instructions of a stage: 8 rows each, x's then w's
+    uint32_t off[ND];
+    #pragma unroll
+    for (int i = 0; i < ND; ++i) {
+        const bool x = i < XD;
+        const uint32_t row = 8 * (x ? XD * w + i : (ND - XD) * w + i - XD) + (lane >> 3), run = (lane & 7) ^ ((row >> 1) & 7);
+        off[i] = (x ? (min(t0 + row, a.t - 1) - t0) * a.ldx : (min(n0 + row, a.n - 1) - n0) * a.k) * 2 + 16 * run;
+    }
+    const u32x4 xrs = panel_rsrc(static_cast<const __bf16*>(a.x) + (size_t)t0 * a.ldx, a.t - t0, a.ldx);
+    const u32x4 wrs = panel_rsrc(a.w + (size_t)n0 * a.k, a.n - n0, a.k);
+    const uint32_t base = (uint32_t)(uintptr_t)lds;
+    const uint32_t xl = __builtin_amdgcn_readfirstlane(base + 1024 * XD * w);
+    const uint32_t wl = __builtin_amdgcn_readfirstlane(base + 1024 * (BM / 8 + (ND - XD) * w));
+    const uint32_t nk = a.k / kEK, nq = nk * a.planes;
+    auto dma1 = [&](uint32_t q, uint32_t slot, int i) __attribute__((always_inline)) {
+        const uint32_t st = 2 * kStage * slot;
+        if (i < XD)
+            dma_lds(off[i], 2 * kEK * q, xrs, xl + st + 1024 * i);
+        else
+            dma_lds(off[i], 2 * kEK * (q < nk ? q : q - nk), wrs, wl + st + 1024 * (i - XD));
+    };
+    f32x16 acc[NM];
+    #pragma unroll
+    for (int i = 0; i < NM; ++i)
+        acc[i] = f32x16{};
+    const uint32_t ra = (w >> 1) * (BM / 2), rb = BM + (w & 1) * (BN / 2);
+    struct Frag {
+        bf16x8 f[NR];  // x's MB blocks, then w's NB
+    };
+    auto read1 = [&](Frag& f, uint32_t slot, int kk, int i) __attribute__((always_inline)) {
+        const uint32_t row = (i < MB ? ra + 32 * i : rb + 32 * (i - MB)) + c32;
+        f.f[i] = *reinterpret_cast<const bf16x8*>(lds + slot * kStage + epos(row, 2 * kk + g));
+    };
+    // one K step's MFMAs on `use`, with the reads of `next` (slot, K step kk; kk < 0: none) and, with DMA, stage q's
+    // instructions spread between them
+    auto step = [&](const Frag& use, Frag& next, uint32_t slot, int kk, auto DMA, uint32_t q, uint32_t to)
+        __attribute__((always_inline)) {
+        #pragma unroll
+        for (int i = 0; i < NM; ++i) {
+            acc[i] = Elem<__bf16>::mfma32(use.f[i / NB], use.f[MB + i % NB], acc[i]);
+            __builtin_amdgcn_sched_barrier(0);
+            if (kk >= 0)
+                #pragma unroll
+                for (int r = i * NR / NM; r < (i + 1) * NR / NM; ++r)
+                    read1(next, slot, kk, r);
+            if constexpr (decltype(DMA)::value)
+                #pragma unroll
+                for (int d = i * ND / NM; d < (i + 1) * ND / NM; ++d)
+                    dma1(q, to, d);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    using Y = std::true_type;
+    using N = std::false_type;
+    #pragma unroll
+    for (int q = 0; q < NST - 1; ++q)
+        #pragma unroll
+        for (int i = 0; i < ND; ++i)
+            dma1(min((uint32_t)q, nq - 1), q, i);
+    Frag fa, fb;
+    #pragma unroll
+    for (int i = 0; i < NR; ++i)
+        fb.f[i] = bf16x8{};  // (the first "last K step of the stage before": zeros)
+    uint32_t slot = 0, prev = NST - 1;
+    for (uint32_t q = 0; q < nq; ++q) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NST - 2) * ND) : "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        step(fb, fa, slot, 0, Y{}, min(q + NST - 1, nq - 1), prev);
+        step(fa, fb, slot, 1, N{}, 0, 0);
+        step(fb, fa, slot, 2, N{}, 0, 0);
+        step(fa, fb, slot, 3, N{}, 0, 0);
+        prev = slot;
+        slot = slot + 1 == NST ? 0 : slot + 1;
+    }
+    step(fb, fa, 0, -1, N{}, 0, 0);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    #pragma unroll
+    for (int bj = 0; bj < NB; ++bj) {
+        const uint32_t c = n0 + (w & 1) * (BN / 2) + 32 * bj + c32;
+        if (c >= a.n)
+            continue;
+        #pragma unroll
+        for (int bi = 0; bi < MB; ++bi)
+            #pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const uint32_t row = t0 + ra + 32 * bi + 8 * (r >> 2) + 4 * g + (r & 3);
+                if (row < a.t)
+                    a.y[(size_t)row * a.ldy + c] = acc[bi * NB + bj][r];
+            }
+    }
+}
+
+// f32 rows rounded to bf16 once, for the DMA kernels (with SPLIT a row's remainders follow its k values). Eight values a
+// thread, streamed; bound by HBM (100 MB in 17.6 us at 4096 x 4096, 5.7 TB/s). Rounding in the tiles' staging repeats
+// the work and the 32-bit reads in every column of tiles and goes through registers: 167 us at 4096 x 4096, against 129
+// for this pass and the DMA kernel (with the split 269 and 233; t = 300: 133 and 28).
+template <bool SPLIT>
+__global__ __launch_bounds__(256) void round_rows(const float* __restrict__ x, __bf16* __restrict__ out, uint32_t t,
+                                                  uint32_t k, uint32_t ldx)
+{
+    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    const uint32_t row = (uint32_t)(i / (k / 8)), c = 8 * (uint32_t)(i % (k / 8));
+    if (row >= t)
+        return;
+    const f32x4* p = reinterpret_cast<const f32x4*>(x + (size_t)row * ldx + c);
+    const f32x4 v0 = __builtin_nontemporal_load(p), v1 = __builtin_nontemporal_load(p + 1);
+    const float f[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
+    u32x4 hi, lo;
+    #pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        hi[e] = Elem<__bf16>::pack2(f[2 * e], f[2 * e + 1]);
+        if (SPLIT)
+            lo[e] = Elem<__bf16>::pack2(f[2 * e] - (float)(__bf16)f[2 * e], f[2 * e + 1] - (float)(__bf16)f[2 * e + 1]);
+    }
+    __bf16* o = out + (size_t)row * k * (SPLIT ? 2 : 1) + c;
+    *reinterpret_cast<u32x4*>(o) = hi;
+    if (SPLIT)
+        *reinterpret_cast<u32x4*>(o + k) = lo;
+}
+
 // A few rows of x (decode, short verification steps): t <= 16 TB. Bound: the read of w (33.6 MB at 4096 x 4096). A
 // 256 x 256 tile a workgroup leaves n / 256 workgroups for the whole chip (16 at n = 4096), so here a workgroup of 8
 // waves takes 16 rows of w and all of x, and the waves take every eighth 64-wide K chunk: together they read 1 KiB runs
@@ -380,11 +523,15 @@ __global__ __launch_bounds__(256, 1) void proj_dma(const ProjParams a)
 // v_mfma_f32_16x16x32_bf16 with no LDS: lane (r, g) holds k values 16 g .. 16 g + 15 of a chunk's row r, as two 16-byte
 // runs (both operands permute k alike, so a row's 128-byte line is read whole). The waves' partial tiles meet in LDS.
 // The next U chunks are loaded while the current U are multiplied. w is read once and streams past the caches; x
-// stays in L2 for all workgroups. 4096 x 4096, bf16 x: 77 -> 10.0 us at t = 1 (3.4 TB/s, launch included), 78 -> 21.7
-// at t = 64; f32 x 121 -> 10.7 and 38; 2048 x 1024 at t = 1 43 -> 7.2. Past 64 rows every workgroup's own read of x
+// stays in L2 for all workgroups. 4096 x 4096, bf16 x: 77 -> 10.0 us at t = 1 (3.4 TB/s, launch included), 78 -> 15.6
+// at t = 32; f32 x 121 -> 10.7 and 24; 2048 x 1024 at t = 1 43 -> 7.2. With more rows every workgroup's own read of x
 // from L2 outweighs w's.
 constexpr int kFewWaves = 8;
-constexpr uint32_t kFewRows = 64;
+constexpr uint32_t kFewRows = 64;  // at most
+// Rows up to which proj_few is the faster one, at 4096 x 4096: bf16 15.6 us at 32 rows and 18.9 at 48 (64 x 64 tiles: 18
+// for both); f32 rows 21 at 24 and 24 at 32 (rounded first, then tiles: 20.5); with the split 24 at 32, 32 at 48 and 38
+// at 64 (36 from 28 on).
+constexpr uint32_t kFewBf16 = 32, kFewF32 = 24, kFewSplit = 48;
 
 typedef __attribute__((address_space(1))) const u32x4 global_u32x4;
 
@@ -505,20 +652,87 @@ void launch_few(const ProjParams& p, hipStream_t stream)
     const dim3 grid((p.n + 15) / 16), block(64 * kFewWaves);
     if (p.t <= 16)
         hipLaunchKernelGGL((proj_few<1, XF32, SPLIT>), grid, block, 0, stream, p);
-    else if (p.t <= 32)
+    else if (!XF32 || p.t <= 32)
         hipLaunchKernelGGL((proj_few<2, XF32, SPLIT>), grid, block, 0, stream, p);
-    else
+    else if constexpr (XF32)
         hipLaunchKernelGGL((proj_few<4, XF32, SPLIT>), grid, block, 0, stream, p);
+}
+
+void set_tiles(ProjParams& p, uint32_t bm, uint32_t bn)
+{
+    p.tiles_m = (p.t + bm - 1) / bm;
+    p.tiles_n = (p.n + bn - 1) / bn;
+    p.tiles = p.tiles_m * p.tiles_n;
+    p.per_xcd = (p.tiles + 7) / 8;
 }
 
 template <int BM, bool XF32, bool SPLIT>
 void launch_proj(ProjParams p, hipStream_t stream)
 {
-    p.tiles_m = (p.t + BM - 1) / BM;
-    p.tiles_n = (p.n + kBN - 1) / kBN;
-    p.tiles = p.tiles_m * p.tiles_n;
-    p.per_xcd = (p.tiles + 7) / 8;
+    set_tiles(p, BM, kBN);
     hipLaunchKernelGGL((proj_tiles<BM, XF32, SPLIT>), dim3(8 * p.per_xcd), dim3(256), 0, stream, p);
+}
+
+template <int BM, int BN, int NST>
+void launch_ring(ProjParams p, hipStream_t stream)
+{
+    set_tiles(p, BM, BN);
+    hipLaunchKernelGGL((proj_ring<BM, BN, NST>), dim3(8 * p.per_xcd), dim3(256), 0, stream, p);
+}
+
+// bf16 rows: the tile by an estimate of each one's time, rounds of workgroups times the time of their K stages, which
+// grows with the share of the CUs that work (clock and L2), and kRoundUs a round. One round at 4096 x 4096 weights
+// (64 stages), alone and on every CU: 256 x 256 78 and 109 us, 128 x 256 48 and 64, 128 x 128 28 and 36, 64 x 128 23 and
+// 26, 64 x 64 18 and 19 (two rounds 36). So t = 128 takes 18 us (79 in 256 x 256 tiles), 512 26 (82), 1000 36 (83), 2048
+// 64 (84), 3000 and 4096 the large tiles' 91 and 109.
+void launch_bf16(ProjParams p, uint32_t cus, hipStream_t stream)
+{
+    struct Tile {
+        uint32_t bm, bn;
+        double alone, full;  // us a stage: on an idle chip, and what a full one adds
+    };
+    static constexpr Tile kTiles[] = {
+        {256, 256, 1.14, 0.50}, {128, 256, 0.68, 0.24}, {128, 128, 0.37, 0.12}, {64, 128, 0.28, 0.10}, {64, 64, 0.20, 0.05}};
+    constexpr double kRoundUs = 3;
+    int best = 0;
+    double best_us = 0;
+    for (int i = 0; i < 5; ++i) {
+        const Tile& c = kTiles[i];
+        const uint64_t n = (uint64_t)((p.t + c.bm - 1) / c.bm) * ((p.n + c.bn - 1) / c.bn);
+        const double rounds = (double)((n + cus - 1) / std::max(cus, 1u)), share = (double)n / (rounds * cus);
+        const double us = rounds * (kRoundUs + p.planes * p.k / kEK * (c.alone + c.full * share));
+        if (i == 0 || us < best_us) {
+            best = i;
+            best_us = us;
+        }
+    }
+    switch (best) {
+    case 0:
+        set_tiles(p, kBN, kBN);
+        hipLaunchKernelGGL(proj_dma, dim3(8 * p.per_xcd), dim3(256), 0, stream, p);
+        break;
+    case 1:
+        launch_ring<128, 256, 3>(p, stream);
+        break;
+    case 2:
+        launch_ring<128, 128, 4>(p, stream);
+        break;
+    case 3:
+        launch_ring<64, 128, 6>(p, stream);
+        break;
+    default:
+        launch_ring<64, 64, 8>(p, stream);
+        break;
+    }
+}
+
+// f32 rows are rounded into at most this much workspace.
+constexpr uint64_t kMaxRounded = 256ull << 20;
+
+// Whether a tile's DMA can address its panels by 32-bit offsets (up to 256 rows, a row's values, a margin).
+bool span_fits(uint32_t rows, uint64_t ld, uint64_t k)
+{
+    return (uint64_t)std::min(rows, 256u) * ld * 2 + 2 * k + 128 <= 0xffffffffu;
 }
 
 bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -528,8 +742,19 @@ bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 using namespace mako;
 
-extern "C" int mako_proj_bf16(const mako_gemm_args* a, int x_dtype, int split, const void* w, const void* x, float* y,
-                              void* stream)
+namespace {
+
+// The workspace f32 rows are rounded into (0: the call's kernels round as they load).
+size_t rounded_bytes(const mako_gemm_args* a, int x_dtype, int split)
+{
+    if (x_dtype != MAKO_F32 || a->t <= (split ? kFewSplit : kFewF32))
+        return 0;
+    const uint64_t planes = split ? 2 : 1, bytes = planes * a->t * a->k * 2;
+    return bytes <= kMaxRounded && span_fits(a->t, planes * a->k, planes * a->k) && span_fits(a->n, a->k, a->k) ? bytes : 0;
+}
+
+int proj_core(const mako_gemm_args* a, int x_dtype, int split, const void* w, const void* x, float* y,
+              const Workspace& work, void* stream)
 {
     if (!a || !w || !x || !y)
         return fail(MAKO_EINVAL, "proj: a null argument");
@@ -552,32 +777,62 @@ extern "C" int mako_proj_bf16(const mako_gemm_args* a, int x_dtype, int split, c
                     a->k);
     if (a->t == 0 || a->n == 0)
         return ok();
-    ProjParams p{static_cast<const __bf16*>(w), x, y, a->t, a->k, a->n, ldy, ldx, 0, 0, 0, 0};
+    ProjParams p{static_cast<const __bf16*>(w), x, y, a->t, a->k, a->n, ldy, ldx, 0, 0, 0, 0, 1};
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    const bool few = p.t <= kFewRows;
     if (x_dtype == MAKO_BF16) {
-        // a tile's DMA addresses its panels by 32-bit offsets (up to 256 rows, a row's k values, a margin)
-        const auto span = [&](uint32_t rows, uint32_t ld) {
-            return (uint64_t)std::min(rows, 256u) * ld * 2 + 2ull * a->k + 128;
-        };
-        if (span(a->t, ldx) > 0xffffffffu || span(a->n, a->k) > 0xffffffffu)
+        if (!span_fits(a->t, ldx, a->k) || !span_fits(a->n, a->k, a->k))
             return fail(MAKO_EINVAL, "proj: rows of %u (x) and %u (w) values are too long for 32-bit tile offsets", ldx,
                         a->k);
-        if (few) {
+        if (p.t <= kFewBf16)
             launch_few<false, false>(p, s);
+        else
+            launch_bf16(p, device_cus(), s);
+        return check_launch("proj");
+    }
+    // f32 rows: rounded once into the workspace and then as bf16 rows; where it cannot be had (a capture, no memory, a
+    // caller's shorter one, more than kMaxRounded bytes) the kernels round as they load.
+    const uint64_t planes = split ? 2 : 1;
+    const size_t bytes = rounded_bytes(a, x_dtype, split);
+    if (bytes && !(work.given && (work.bytes < bytes || !al16(work.ptr)))) {
+        if (void* ws = work.get(bytes, s)) {
+            const dim3 grid((uint32_t)(((uint64_t)a->t * (a->k / 8) + 255) / 256));
+            if (split)
+                hipLaunchKernelGGL(round_rows<true>, grid, dim3(256), 0, s, static_cast<const float*>(x),
+                                   static_cast<__bf16*>(ws), a->t, a->k, ldx);
+            else
+                hipLaunchKernelGGL(round_rows<false>, grid, dim3(256), 0, s, static_cast<const float*>(x),
+                                   static_cast<__bf16*>(ws), a->t, a->k, ldx);
+            p.x = ws;
+            p.ldx = (uint32_t)planes * a->k;
+            p.planes = (uint32_t)planes;
+            launch_bf16(p, device_cus(), s);
             return check_launch("proj");
         }
-        p.tiles_m = (p.t + kBN - 1) / kBN;
-        p.tiles_n = (p.n + kBN - 1) / kBN;
-        p.tiles = p.tiles_m * p.tiles_n;
-        p.per_xcd = (p.tiles + 7) / 8;
-        hipLaunchKernelGGL(proj_dma, dim3(8 * p.per_xcd), dim3(256), 0, s, p);
     }
-    else if (few)
+    if (p.t <= kFewRows)
         split ? launch_few<true, true>(p, s) : launch_few<true, false>(p, s);
-    else if (!split)
-        launch_proj<256, true, false>(p, s);
-    else
+    else if (split)
         launch_proj<128, true, true>(p, s);
+    else
+        launch_proj<256, true, false>(p, s);
     return check_launch("proj");
+}
+
+}  // namespace
+
+extern "C" size_t mako_proj_bf16_workspace(const mako_gemm_args* a, int x_dtype, int split)
+{
+    return a ? rounded_bytes(a, x_dtype, split) : 0;
+}
+
+extern "C" int mako_proj_bf16(const mako_gemm_args* a, int x_dtype, int split, const void* w, const void* x, float* y,
+                              void* stream)
+{
+    return proj_core(a, x_dtype, split, w, x, y, library_workspace(kWsRounded, "proj"), stream);
+}
+
+extern "C" int mako_proj_bf16_ws(const mako_gemm_args* a, int x_dtype, int split, const void* w, const void* x,
+                                 float* y, void* workspace, size_t workspace_bytes, void* stream)
+{
+    return proj_core(a, x_dtype, split, w, x, y, caller_workspace(workspace, workspace_bytes, "proj"), stream);
 }

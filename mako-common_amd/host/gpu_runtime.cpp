@@ -375,11 +375,15 @@ void Runtime::proj(Encoder*& enc, const Weight& w, Buffer* x, uint64_t x_off, Bu
     }
     const mako_gemm_args a{T, w.k, w.n, 2 * w.k, ldy, 0};
     const char* label = bf16_split_ && !x_bf16 ? "proj BF16 split" : "proj BF16";
+    const int dtype = x_bf16 ? MAKO_BF16 : MAKO_F32, split = bf16_split_ && !x_bf16 ? 1 : 0;
+    const size_t need = mako_proj_bf16_workspace(&a, dtype, split);  // f32 rows rounded to bf16
+    Buffer* ws = need ? scratch("proj_rounded", need) : nullptr;
     before(enc);
     for (int r = repeats(label); r > 0; --r)
-        check(mako_proj_bf16(&a, x_bf16 ? MAKO_BF16 : MAKO_F32, bf16_split_ && !x_bf16 ? 1 : 0,
-                             static_cast<const char*>(w.buf->ptr) + w.off, static_cast<const char*>(x->ptr) + x_off,
-                             reinterpret_cast<float*>(static_cast<char*>(y->ptr) + y_off), enc->stream));
+        check(mako_proj_bf16_ws(&a, dtype, split, static_cast<const char*>(w.buf->ptr) + w.off,
+                                static_cast<const char*>(x->ptr) + x_off,
+                                reinterpret_cast<float*>(static_cast<char*>(y->ptr) + y_off), ws ? ws->ptr : nullptr,
+                                ws ? ws->bytes : 0, enc->stream));
     after(enc, label);
 }
 

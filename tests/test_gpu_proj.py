@@ -129,3 +129,56 @@ def test_few_rows(t, k, n, ldx, ldy, xd, split):
     got, want, mag = run_proj(np.random.default_rng(t + k), t, k, n, xd, split, ldx, ldy)
     assert_sum_close(got[:, :n], want[:, :n], (4 if split else 2) * k * U * mag[:, :n], "proj")
     assert (got[:, n:] == SENTINEL).all(), "a column past n was written"
+
+
+@pytest.mark.parametrize("t,k,n,ldx,ldy", [
+    (100, 64, 130, 0, 0), (65, 576, 257, 584, 260),   # 64 x 64 tiles: fewer K stages than the ring, and more
+    (300, 192, 4100, 0, 0), (290, 448, 4090, 456, 0),  # 64 x 128
+    (900, 128, 4100, 0, 0), (1000, 320, 4090, 328, 4092),  # 128 x 128
+    (2000, 64, 4090, 0, 0), (1990, 256, 4100, 0, 0),   # 128 x 256
+])
+@pytest.mark.parametrize("xd,split", [(O.BF16, 0), (O.F32, 0), (O.F32, 1)], ids=["bf16", "f32", "split"])
+def test_ring_tiles(t, k, n, ldx, ldy, xd, split):
+    """proj_ring's tiles with part tiles in both dimensions, and the rounding pass before them for f32 rows; 40 rows
+    (the last one among them) against the oracle."""
+    rng = np.random.default_rng(t + k)
+    ld = ldx or k
+    w = O.to_bf16_bits(rng.standard_normal((n, k)) * 0.05)
+    xf = rng.standard_normal((t, ld)).astype(np.float32)
+    x = xf if xd == O.F32 else O.to_bf16_bits(xf)
+    y = torch.full((t, ldy or n), SENTINEL, dtype=torch.float32, device="cuda")
+    print(f"proj ring t={t} k={k} n={n} xd={xd} split={split}", flush=True)
+    M.proj_bf16(G.to_dev(w, O.BF16), torch.from_numpy(x).to("cuda") if xd == O.F32 else G.to_dev(x, O.BF16), y, t=t, k=k,
+                n=n, ldx=ldx, ldy=ldy, split=split)
+    torch.cuda.synchronize()
+    rows = np.sort(np.append(rng.choice(t - 1, 39, replace=False), t - 1))
+    got = y.cpu().numpy()
+    assert (got[:, n:] == SENTINEL).all(), "a column past n was written"
+    xr = np.ascontiguousarray(x[rows])
+    want = O.proj_bf16(xr, w, t=40, k=k, n=n, ldx=ldx, x_dtype=xd, split=split)
+    mag = O.proj_bf16(np.abs(xr) if xd == O.F32 else abs_bits(xr), abs_bits(w), t=40, k=k, n=n, ldx=ldx, x_dtype=xd,
+                      split=split)
+    assert_sum_close(got[rows][:, :n], want[:, :n], (4 if split else 2) * k * U * mag[:, :n], "proj")
+
+
+@pytest.mark.parametrize("t,split", [(60, 1), (300, 0)])
+def test_f32_rows_under_capture(t, split):
+    """A captured call on a stream the library holds no workspace for rounds in the tiles: each replay gives the bound."""
+    k, n = 256, 320
+    rng = np.random.default_rng(t)
+    w = O.to_bf16_bits(rng.standard_normal((n, k)) * 0.05)
+    x = rng.standard_normal((t, k)).astype(np.float32)
+    wd, xd = G.to_dev(w, O.BF16), torch.from_numpy(x).to("cuda")
+    y = torch.empty((t, n), dtype=torch.float32, device="cuda")
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        M.proj_bf16(wd, xd, y, t=t, k=k, n=n, split=split, stream=s.cuda_stream)
+    want = O.proj_bf16(x, w, t=t, k=k, n=n, x_dtype=O.F32, split=split)
+    mag = O.proj_bf16(np.abs(x), abs_bits(w), t=t, k=k, n=n, x_dtype=O.F32, split=split)
+    for _ in range(3):
+        y.fill_(SENTINEL)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert_sum_close(y.cpu().numpy(), want, (4 if split else 2) * k * U * mag, "proj")
