@@ -358,6 +358,17 @@ typedef struct mako_scan_args {
 int mako_kda_scan(const mako_scan_args* a, const float* q, const float* k, const float* v, const float* g,
                   const float* beta, float* state, float* o, float* snap_state, void* stream);
 
+/*
+ * mako_kda_scan with the caller's workspace. Long runs are computed in chunks of 16 tokens whose operands take
+ * mako_kda_scan_workspace(a) bytes (0: token by token; at most 64 MiB, or one chunk's); mako_kda_scan keeps them itself
+ * per (device, stream) until mako_attn_release. With less, none, or under a capture that would have to allocate, the
+ * tokens run one by one.
+ */
+size_t mako_kda_scan_workspace(const mako_scan_args* a);
+int mako_kda_scan_ws(const mako_scan_args* a, const float* q, const float* k, const float* v, const float* g,
+                     const float* beta, float* state, float* o, float* snap_state, void* workspace,
+                     size_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

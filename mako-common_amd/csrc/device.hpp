@@ -194,7 +194,7 @@ uint32_t device_cus();
 // handle). Returns null, with nothing allocated and the error recorded, when the allocation fails (MAKO_EHIP) or
 // when the stream is capturing a graph and the buffer would have to grow (MAKO_EWORKSPACE: an allocation in a
 // capture would belong to the graph).
-enum WorkspacePurpose { kWsVtImages = 0, kWsSplitK = 1, kWsRowTiles = 2, kWsPassTable = 3, kWsRounded = 4, kWsPurposes = 5 };
+enum WorkspacePurpose { kWsVtImages = 0, kWsSplitK = 1, kWsRowTiles = 2, kWsPassTable = 3, kWsRounded = 4, kWsScan = 5, kWsPurposes = 6 };
 void* stream_workspace(WorkspacePurpose purpose, size_t bytes, hipStream_t s, const char* what);
 
 // A call's workspace: the caller's buffer (given, from an entry point that takes one: never allocates) or the

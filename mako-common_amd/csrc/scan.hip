@@ -19,10 +19,12 @@
 // state update (it is off the state's chain), the rollback snapshot has a loop of its own for the one batch that
 // holds it, and nothing in the loop is conditional.
 // Bound: the token recurrence (a dependent chain of decay, dot product, lane reduction and update per token) and
-// the VALU (no packed FP32 here): 7 flops a channel a row a token.
-#include "device.hpp"
-
+// the VALU (no packed FP32 here): 7 flops a channel a row a token. This is the kernel of short runs, and of calls with no
+// workspace; long runs go by chunks of 16 tokens (below).
+#include <algorithm>
 #include <type_traits>
+
+#include "device.hpp"
 
 namespace mako {
 namespace {
@@ -236,6 +238,325 @@ __global__ __launch_bounds__(256) void kda_scan_rows(const ScanParams a)
         *reinterpret_cast<f32x4*>(mg + ch[r]) = f32x4{m[4 * r], m[4 * r + 1], m[4 * r + 2], m[4 * r + 3]};
 }
 
+// ---- long runs: chunks of 16 tokens ------------------------------------------------------------------------------
+//
+// Token by token the recurrence is a serial chain of ~400 cycles a token on a quarter of the issue slots (4096 tokens of
+// 32 heads: 717 us). Over a chunk of 16 tokens with S its first state, E(t, s) the product of the decays of tokens
+// s + 1 .. t and Gamma_t that of all up to t (per channel),
+//   d = W (v - (Gamma k) S),  o = ((Gamma q) S + B d) / sqrt(128),  S' = Gamma_last S + (E(last, .) k)^T d
+//   A[t][s] = k_t . E(t, s) k_s (s < t),  B[t][s] = q_t . E(t, s) k_s (s <= t),  W = (1 + diag(beta) A)^-1 diag(beta)
+// (the delta rule's 16 rank-one updates solved at once), which is seven small matrix products. Products of decays are
+// formed one factor at a time as the recurrence forms them, never as exponentials of summed logarithms or as ratios:
+// no cancellation, no overflow where the recurrence has none. Everything is f32, on v_mfma_f32_16x16x4_f32; against 64
+// bits the outputs are within 1 % of the recurrence's error (1.65e-7 against 1.67e-7 over 97 to 3000 tokens), the state
+// closer (1.37e-7 and 1.53e-7: one rounding at its size a chunk).
+//
+// kda_chunk: a workgroup a (chunk, head) makes everything of a chunk that needs no state, as the LDS image of the next
+// kernel's stage (28 KiB in the workspace): Gamma k, Gamma q, E(last, .) k, Gamma_last, W and B.
+// kda_scan_chunks: a workgroup a (head, 16 columns of S), the chunks in order. Waves 0 - 3 hold S, 32 channels each, as
+// the accumulators of 16 x 16 blocks: register r of lane (g, c) is channel 16 b + 4 g + r of column c, which is also the
+// B operand of the products with S when MFMA r takes channels 4 g + r as its k, and likewise d's and v's tokens, so
+// nothing moves between lanes. The waves' shares of (Gamma k) S meet in LDS; d is computed by each. Waves 4 and 5 bring
+// the images and v in by LDS DMA, three chunks ahead. (A first form made the images in the workgroup, from rows loaded a
+// chunk ahead: 2.1 us a chunk, waiting for the loads.)
+// A snapshot's token ends a chunk: the chunks of tokens [0, snap) are followed by those of [snap, tokens).
+constexpr uint32_t kChunk = 16, kCRow = kD + 4;  // floats a staged row (the pad spreads 16 rows over the banks)
+
+struct ChunkImage {
+    float kg[kChunk][kCRow], qg[kChunk][kCRow], ke[kChunk][kCRow];
+    float last[kD];
+    float w[kChunk][kChunk], b[kChunk][kChunk];
+    float pad[192];
+};
+static_assert(sizeof(ChunkImage) == 28 * 1024, "whole DMA pieces");
+
+struct ChunkParams {
+    ScanParams s;
+    ChunkImage* image;    // [chunk of the launch][head]
+    uint32_t c0, n;       // the launch's chunks, of all
+    uint32_t before;      // chunks of [0, snap)
+};
+
+// Chunk c's first token and count.
+__device__ __forceinline__ void chunk_of(const ChunkParams& a, uint32_t c, uint32_t& t0, uint32_t& np)
+{
+    t0 = c < a.before ? c * kChunk : a.s.snap + (c - a.before) * kChunk;
+    np = min(kChunk, (c < a.before ? a.s.snap : a.s.tokens) - t0);
+}
+
+__global__ __launch_bounds__(256) void kda_chunk(const ChunkParams a)
+{
+    __shared__ __attribute__((aligned(16))) float ks[kChunk][kD], qs[kChunk][kD], es[kChunk][kD];
+    __shared__ float as[kChunk][kChunk + 1], bs[kChunk][kChunk + 1], beta[kChunk];
+    const uint32_t tid = threadIdx.x, h = blockIdx.x, c = a.c0 + blockIdx.y;
+    uint32_t t0, np;
+    chunk_of(a, c, t0, np);
+    const size_t hq = (size_t)h * kD;
+    #pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t e = tid + 256 * i, t = e >> 5, ch = 4 * (e & 31);
+        f32x4 k{}, q{}, d{1.0f, 1.0f, 1.0f, 1.0f};
+        if (t < np) {
+            const size_t qo = (size_t)(t0 + t) * a.s.qkv_stride + hq + ch;
+            k = *reinterpret_cast<const f32x4*>(a.s.k + qo);
+            q = *reinterpret_cast<const f32x4*>(a.s.q + qo);
+            const f32x4 g = *reinterpret_cast<const f32x4*>(a.s.g + (size_t)(t0 + t) * a.s.inner + hq + ch);
+            d = f32x4{__expf(g[0]), __expf(g[1]), __expf(g[2]), __expf(g[3])};
+        }
+        *reinterpret_cast<f32x4*>(&ks[t][ch]) = k;
+        *reinterpret_cast<f32x4*>(&qs[t][ch]) = q;
+        *reinterpret_cast<f32x4*>(&es[t][ch]) = d;
+    }
+    if (tid < kChunk)
+        beta[tid] = tid < np ? a.s.beta[(size_t)(t0 + tid) * a.s.heads + h] : 0.0f;
+    __syncthreads();
+    // Row s of 16 lanes, 8 channels a lane: p = E(t, s) k_s, one more factor a step.
+    const uint32_t s = tid >> 4, l = tid & 15, first = __builtin_amdgcn_readfirstlane(s);
+    const f32x4 one{1.0f, 1.0f, 1.0f, 1.0f};
+    f32x4 p0 = *reinterpret_cast<const f32x4*>(&ks[s][4 * l]), p1 = *reinterpret_cast<const f32x4*>(&ks[s][64 + 4 * l]);
+    for (uint32_t t = first; t < kChunk; ++t) {
+        const f32x4 e0 = *reinterpret_cast<const f32x4*>(&es[t][4 * l]), e1 = *reinterpret_cast<const f32x4*>(&es[t][64 + 4 * l]);
+        const f32x4 k0 = *reinterpret_cast<const f32x4*>(&ks[t][4 * l]), k1 = *reinterpret_cast<const f32x4*>(&ks[t][64 + 4 * l]);
+        const f32x4 q0 = *reinterpret_cast<const f32x4*>(&qs[t][4 * l]), q1 = *reinterpret_cast<const f32x4*>(&qs[t][64 + 4 * l]);
+        p0 *= t > s ? e0 : one;
+        p1 *= t > s ? e1 : one;
+        float x = 0.0f, y = 0.0f;
+        #pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            x = fmaf(k0[n], p0[n], x);
+            y = fmaf(q0[n], p0[n], y);
+        }
+        #pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            x = fmaf(k1[n], p1[n], x);
+            y = fmaf(q1[n], p1[n], y);
+        }
+        x = row_sum<16>(x);
+        y = row_sum<16>(y);
+        as[t][s] = x;             // (used for s < t only)
+        bs[t][s] = t >= s ? y : 0.0f;
+    }
+    for (uint32_t t = 0; t < first; ++t)
+        bs[t][s] = 0.0f;
+    __syncthreads();
+    ChunkImage& out = a.image[(size_t)blockIdx.y * a.s.heads + h];
+    {
+        // the running products: 128 threads forward, 128 backward, a channel each
+        const uint32_t i = tid & 127;
+        float p = 1.0f;
+        if (tid < 128) {
+            #pragma unroll
+            for (uint32_t t = 0; t < kChunk; ++t) {
+                p *= es[t][i];
+                out.kg[t][i] = p * ks[t][i];
+                out.qg[t][i] = p * qs[t][i];
+            }
+            out.last[i] = p;
+        } else {
+            #pragma unroll
+            for (uint32_t n = 0; n < kChunk; ++n) {
+                const uint32_t t = kChunk - 1 - n;
+                out.ke[t][i] = p * ks[t][i];
+                p *= es[t][i];
+            }
+        }
+    }
+    if (tid < kChunk) {  // column tid of W by forward substitution
+        float w[kChunk];
+        #pragma unroll
+        for (uint32_t t = 0; t < kChunk; ++t) {
+            float x = t == tid ? 1.0f : 0.0f;
+            #pragma unroll
+            for (uint32_t r = 0; r < t; ++r)
+                x = fmaf(-as[t][r], w[r], x);
+            w[t] = x * beta[t];
+            out.w[t][tid] = w[t];
+        }
+    }
+    out.b[tid >> 4][tid & 15] = bs[tid >> 4][tid & 15];
+}
+
+__device__ __forceinline__ f32x4 mfma4(float x, float y, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, c, 0, 0, 0); }
+
+// 16 bytes a lane from base + off to LDS m0 + 16 lane.
+__device__ __forceinline__ void dma16(uint32_t m0, const void* base, uint32_t off)
+{
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(m0), "v"(off), "s"(base)
+                 : "memory", "m0");
+#pragma clang diagnostic pop
+}
+
+__global__ __launch_bounds__(448) void kda_scan_chunks(const ChunkParams a)
+{
+    constexpr uint32_t kSlots = 4, kPieces = sizeof(ChunkImage) / 1024;  // a wave DMAs half the pieces, and v
+    struct Stage {
+        ChunkImage x;
+        float v[kChunk][kChunk];
+    };
+    __shared__ __attribute__((aligned(1024))) Stage st[kSlots];
+    __shared__ f32x4 pu[4][64], pq[2][4][64];  // the waves' shares of (Gamma k) S and (Gamma q) S
+    __shared__ f32x4 pd[2][64];                // d
+    const uint32_t tid = threadIdx.x, lane = tid & 63, h = blockIdx.x, j0 = blockIdx.y * 16;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, c16 = lane & 15;
+    const size_t hq = (size_t)h * kD;
+    const float scale = 0.08838834764831845f;  // 1 / sqrt(128)
+    if (w == 4 || w == 5) {
+        // Chunk c into slot c % kSlots: pieces w - 4, w - 2, .. of the image, and v (both waves, the same bytes: lane 4 t
+        // + n takes columns 4 n .. of token t; past a part chunk's end the last token's, whose products are zeros'), so
+        // each wave has the same number in flight. Past the last chunk the DMA reads it again (into slots not read).
+        const auto issue = [&](uint32_t c) __attribute__((always_inline)) {
+            const uint32_t slot = c % kSlots, cc = min(c, a.n - 1);
+            uint32_t t0, np;
+            chunk_of(a, a.c0 + cc, t0, np);
+            const uint32_t lds = __builtin_amdgcn_readfirstlane((uint32_t)reinterpret_cast<uintptr_t>(&st[slot]));
+            const ChunkImage* im = a.image + ((size_t)cc * a.s.heads + h);
+            #pragma unroll
+            for (uint32_t i = 0; i < kPieces / 2; ++i) {
+                const uint32_t piece = 2 * i + w - 4;
+                dma16(__builtin_amdgcn_readfirstlane(lds + 1024 * piece), im, 1024 * piece + 16 * lane);
+            }
+            const float* v = a.s.v + (size_t)t0 * a.s.qkv_stride + hq + j0;
+            dma16(__builtin_amdgcn_readfirstlane(lds + (uint32_t)sizeof(ChunkImage)), v,
+                  min(lane >> 2, np - 1) * a.s.qkv_stride * 4 + 16 * (lane & 3));
+        };
+        for (uint32_t c = 0; c < kSlots - 1; ++c)
+            issue(c);
+        // the oldest chunk in flight has landed: all but the kSlots - 2 after it
+        const auto landed = [] { asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kSlots - 2) * (kPieces / 2 + 1)) : "memory"); };
+        landed();
+        __syncthreads();
+        for (uint32_t c = 0; c < a.n; ++c) {
+            issue(c + kSlots - 1);  // (its slot: chunk c - 1's, read last before the barrier that ended it)
+            __syncthreads();        // the shares of chunk c
+            landed();
+            __syncthreads();        // the end of chunk c
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        return;
+    }
+    if (w == 6) {
+        // The outputs, a chunk behind the state, so that they are not on its chain (taken by waves 0 - 3 in turn, they
+        // were a quarter of a chunk's time).
+        __syncthreads();
+        for (uint32_t c = 0; c < a.n; ++c) {
+            uint32_t t0, np;
+            chunk_of(a, a.c0 + c, t0, np);
+            const f32x4 br = *reinterpret_cast<const f32x4*>(&st[c % kSlots].x.b[c16][4 * g]);
+            __syncthreads();
+            __syncthreads();  // the end of chunk c (pq and pd are rewritten two chunks on)
+            const f32x4 d = pd[c & 1][lane];
+            f32x4 o{};
+            #pragma unroll
+            for (int r = 0; r < 4; ++r)
+                o = mfma4(br[r], d[r], o);
+            o += (pq[c & 1][0][lane] + pq[c & 1][1][lane]) + (pq[c & 1][2][lane] + pq[c & 1][3][lane]);
+            float* at = a.s.o + (size_t)t0 * a.s.inner + hq + j0 + c16;
+            #pragma unroll
+            for (uint32_t r = 0; r < 4; ++r)
+                if (4 * g + r < np)
+                    at[(size_t)(4 * g + r) * a.s.inner] = o[r] * scale;
+        }
+        return;
+    }
+    // Channel 32 w + 16 b + 4 g + r of column j0 + c16: state[h][j][i].
+    float* mg = a.s.state + ((size_t)h * kD + j0 + c16) * kD + 32 * w + 4 * g;
+    f32x4 m[2];
+    #pragma unroll
+    for (int b = 0; b < 2; ++b)
+        m[b] = *reinterpret_cast<const f32x4*>(mg + 16 * b);
+    __syncthreads();  // chunk 0 is staged
+    for (uint32_t c = 0; c < a.n; ++c) {
+        const Stage& s = st[c % kSlots];
+        uint32_t t0, np;
+        chunk_of(a, a.c0 + c, t0, np);
+        // this wave's shares of (Gamma k) S and (Gamma q) S, tokens 4 g + r of column c16: the second while the first
+        // goes through LDS
+        f32x4 u[2]{}, y[2]{}, kg[2], qg[2], last[2], v;
+        float ke[2][4];
+        #pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            kg[b] = *reinterpret_cast<const f32x4*>(&s.x.kg[c16][32 * w + 16 * b + 4 * g]);
+            qg[b] = *reinterpret_cast<const f32x4*>(&s.x.qg[c16][32 * w + 16 * b + 4 * g]);
+        }
+        const f32x4 wr = *reinterpret_cast<const f32x4*>(&s.x.w[c16][4 * g]);
+        #pragma unroll
+        for (int r = 0; r < 4; ++r)
+            v[r] = s.v[4 * g + r][c16];
+        #pragma unroll
+        for (int r = 0; r < 4; ++r)
+            #pragma unroll
+            for (int b = 0; b < 2; ++b)
+                u[b] = mfma4(kg[b][r], m[b][r], u[b]);
+        #pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            last[b] = *reinterpret_cast<const f32x4*>(&s.x.last[32 * w + 16 * b + 4 * g]);
+            #pragma unroll
+            for (int r = 0; r < 4; ++r)
+                ke[b][r] = s.x.ke[4 * g + r][32 * w + 16 * b + c16];
+        }
+        pu[w][lane] = u[0] + u[1];
+        __builtin_amdgcn_sched_barrier(0);
+        #pragma unroll
+        for (int r = 0; r < 4; ++r)
+            #pragma unroll
+            for (int b = 0; b < 2; ++b)
+                y[b] = mfma4(qg[b][r], m[b][r], y[b]);
+        __syncthreads();
+        const f32x4 e = v - ((pu[0][lane] + pu[1][lane]) + (pu[2][lane] + pu[3][lane]));
+        pq[c & 1][w][lane] = y[0] + y[1];
+        f32x4 d{};
+        #pragma unroll
+        for (int r = 0; r < 4; ++r)
+            d = mfma4(wr[r], e[r], d);
+        // the update summed by itself: one rounding at the state's size a chunk
+        f32x4 n[2]{};
+        #pragma unroll
+        for (int r = 0; r < 4; ++r)
+            #pragma unroll
+            for (int b = 0; b < 2; ++b)
+                n[b] = mfma4(ke[b][r], d[r], n[b]);
+        if (w == 0)
+            pd[c & 1][lane] = d;
+        #pragma unroll
+        for (int b = 0; b < 2; ++b)
+            #pragma unroll
+            for (int r = 0; r < 4; ++r)
+                m[b][r] = fmaf(m[b][r], last[b][r], n[b][r]);
+        if (a.s.snap && t0 + np == a.s.snap) {
+            float* sg = a.s.snap_state + ((size_t)h * kD + j0 + c16) * kD + 32 * w + 4 * g;
+            #pragma unroll
+            for (int b = 0; b < 2; ++b)
+                *reinterpret_cast<f32x4*>(sg + 16 * b) = m[b];
+        }
+        __syncthreads();
+    }
+    #pragma unroll
+    for (int b = 0; b < 2; ++b)
+        *reinterpret_cast<f32x4*>(mg + 16 * b) = m[b];
+}
+
+// Token counts from which the chunks are the faster kernels (32 heads: 96 tokens 21.7 us token by token, 18.2 by chunks;
+// 200 40 and 27; 512 93 and 49; 4096 716 and 367), and the workspace a launch's images take at most: longer runs go in
+// several launches, whose images stay in the last-level cache (73 chunks of 32 heads: 29 us to make, bound by their
+// traffic, and 83 us to run, 1.1 us a chunk of LDS and barrier latencies around 28 MFMAs a wave).
+constexpr uint32_t kChunkTokens = 96;
+constexpr size_t kChunkBytes = 64u << 20;
+
+uint32_t chunks_of(const mako_scan_args* a)
+{
+    return (a->snap + kChunk - 1) / kChunk + (a->tokens - a->snap + kChunk - 1) / kChunk;
+}
+
+size_t chunk_bytes(const mako_scan_args* a) { return (size_t)a->heads * sizeof(ChunkImage); }
+
+// The chunks of one launch.
+uint32_t chunks_a_launch(const mako_scan_args* a)
+{
+    return (uint32_t)std::min<size_t>({chunks_of(a), std::max<size_t>(1, kChunkBytes / chunk_bytes(a)), 65535});
+}
+
 constexpr int kScanLanes = 16;  // lanes a state row: 8 values a lane, one wave a SIMD at 32 heads
 
 bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -245,8 +566,15 @@ bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 using namespace mako;
 
-extern "C" int mako_kda_scan(const mako_scan_args* a, const float* q, const float* k, const float* v, const float* g,
-                             const float* beta, float* state, float* o, float* snap_state, void* stream)
+namespace {
+
+size_t scan_bytes(const mako_scan_args* a)
+{
+    return a->heads && a->tokens >= kChunkTokens && a->snap <= a->tokens ? chunks_a_launch(a) * chunk_bytes(a) : 0;
+}
+
+int scan_core(const mako_scan_args* a, const float* q, const float* k, const float* v, const float* g,
+              const float* beta, float* state, float* o, float* snap_state, const Workspace& work, void* stream)
 {
     if (!a || !q || !k || !v || !g || !beta || !state || !o || (a->snap && !snap_state))
         return fail(MAKO_EINVAL, "kda_scan: a null argument");
@@ -263,7 +591,39 @@ extern "C" int mako_kda_scan(const mako_scan_args* a, const float* q, const floa
     if (a->heads > 65535u)
         return fail(MAKO_EINVAL, "kda_scan: %u heads exceed the grid", a->heads);
     ScanParams p{q, k, v, g, beta, state, o, snap_state, a->tokens, a->qkv_stride, a->inner, a->heads, a->snap};
-    hipLaunchKernelGGL(kda_scan_rows<kScanLanes>, dim3(a->heads, kD / (256 / kScanLanes)), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), p);
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    // chunks, where there is a workspace to be had (a capture, no memory or a caller's shorter one: token by token) and
+    // v's rows suit 16-byte DMA from 32-bit offsets
+    const size_t bytes = scan_bytes(a);
+    if (bytes && al16(v) && a->qkv_stride < (1u << 25) && !(work.given && (work.bytes < bytes || !al16(work.ptr)))) {
+        if (ChunkImage* ws = static_cast<ChunkImage*>(work.get(bytes, s))) {
+            const uint32_t n = chunks_of(a), per = chunks_a_launch(a);
+            for (uint32_t c = 0; c < n; c += per) {
+                const ChunkParams cp{p, ws, c, std::min(per, n - c), (a->snap + kChunk - 1) / kChunk};
+                hipLaunchKernelGGL(kda_chunk, dim3(a->heads, cp.n), dim3(256), 0, s, cp);
+                hipLaunchKernelGGL(kda_scan_chunks, dim3(a->heads, kD / 16), dim3(448), 0, s, cp);
+            }
+            return check_launch("kda_scan");
+        }
+    }
+    hipLaunchKernelGGL(kda_scan_rows<kScanLanes>, dim3(a->heads, kD / (256 / kScanLanes)), dim3(256), 0, s, p);
     return check_launch("kda_scan");
+}
+
+}  // namespace
+
+extern "C" size_t mako_kda_scan_workspace(const mako_scan_args* a) { return a ? scan_bytes(a) : 0; }
+
+extern "C" int mako_kda_scan(const mako_scan_args* a, const float* q, const float* k, const float* v, const float* g,
+                             const float* beta, float* state, float* o, float* snap_state, void* stream)
+{
+    return scan_core(a, q, k, v, g, beta, state, o, snap_state, library_workspace(kWsScan, "kda_scan"), stream);
+}
+
+extern "C" int mako_kda_scan_ws(const mako_scan_args* a, const float* q, const float* k, const float* v, const float* g,
+                                const float* beta, float* state, float* o, float* snap_state, void* workspace,
+                                size_t workspace_bytes, void* stream)
+{
+    return scan_core(a, q, k, v, g, beta, state, o, snap_state,
+                     caller_workspace(workspace, workspace_bytes, "kda_scan"), stream);
 }

@@ -70,9 +70,12 @@ void TransformerRuntime::kda_scan(gpu::Encoder*& enc, gpu::Buffer* q, gpu::Buffe
 {
     const mako_scan_args a{kHeadDim, T, qkv_stride, inner, n_heads, snap};
     auto f = [](gpu::Buffer* b) { return b ? static_cast<float*>(b->ptr) : nullptr; };
+    const size_t need = mako_kda_scan_workspace(&a);  // the chunks' matrices
+    gpu::Buffer* ws = need ? scratch("kda_scan", need) : nullptr;
     before(enc);
     for (int r = repeats("kda_scan"); r > 0; --r)
-        check(mako_kda_scan(&a, f(q), f(k), f(v), f(g), f(beta), f(state), f(o), f(snap_state), enc->stream));
+        check(mako_kda_scan_ws(&a, f(q), f(k), f(v), f(g), f(beta), f(state), f(o), f(snap_state), ws ? ws->ptr : nullptr,
+                               ws ? ws->bytes : 0, enc->stream));
     after(enc, "kda_scan");
 }
 

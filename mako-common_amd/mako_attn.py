@@ -18,7 +18,8 @@ EXPORTS = ("mako_attn_abi_version", "mako_last_error", "mako_attn_fwd", "mako_cu
            "mako_cube_select", "mako_attn_sparse", "mako_attn_decode_workspace", "mako_attn_decode",
            "mako_attn_decode_noalloc", "mako_heads", "mako_attn_fwd_rows",
            "mako_attn_pv", "mako_attn_gather_scores", "mako_attn_gather_pv", "mako_idx_dots", "mako_proj_bf16",
-           "mako_proj_bf16_workspace", "mako_proj_bf16_ws", "mako_kda_scan", "mako_attn_fwd_workspace", "mako_attn_fwd_ws", "mako_attn_sparse_workspace",
+           "mako_proj_bf16_workspace", "mako_proj_bf16_ws", "mako_kda_scan", "mako_kda_scan_workspace",
+           "mako_kda_scan_ws", "mako_attn_fwd_workspace", "mako_attn_fwd_ws", "mako_attn_sparse_workspace",
            "mako_attn_sparse_ws", "mako_attn_fwd_rows_workspace", "mako_attn_fwd_rows_ws", "mako_attn_release",
            "mako_attn_held_bytes")
 
@@ -104,6 +105,9 @@ def lib():
         L.mako_proj_bf16_workspace.restype = SZ
         L.mako_proj_bf16_ws.argtypes = [ctypes.POINTER(GemmArgs), I, I, P, P, P, P, SZ, P]
         L.mako_kda_scan.argtypes = [ctypes.POINTER(ScanArgs)] + [P] * 9
+        L.mako_kda_scan_workspace.argtypes = [ctypes.POINTER(ScanArgs)]
+        L.mako_kda_scan_workspace.restype = SZ
+        L.mako_kda_scan_ws.argtypes = [ctypes.POINTER(ScanArgs)] + [P] * 9 + [SZ, P]
         L.mako_attn_fwd_workspace.argtypes = [ctypes.POINTER(AttnArgs), U32]
         L.mako_attn_fwd_workspace.restype = SZ
         L.mako_attn_fwd_ws.argtypes = [ctypes.POINTER(AttnArgs), U32, I, I, P, P, P, P, P, P, SZ, P]
@@ -121,7 +125,8 @@ def lib():
                      "mako_attn_decode_noalloc", "mako_heads", "mako_attn_fwd_rows", "mako_attn_fwd_ws",
                      "mako_attn_sparse_ws", "mako_attn_fwd_rows_ws", "mako_attn_release",
                      "mako_attn_pv", "mako_attn_gather_scores", "mako_attn_gather_pv", "mako_idx_dots",
-                     "mako_proj_bf16", "mako_proj_bf16_ws", "mako_kda_scan"):
+                     "mako_proj_bf16", "mako_proj_bf16_ws", "mako_kda_scan",
+                     "mako_kda_scan_ws"):
             getattr(L, name).restype = I
         _lib = L
     return _lib

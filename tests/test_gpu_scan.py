@@ -116,3 +116,69 @@ def test_qwen35_linear_attention_shape():
         want_o, want_st, _ = O.kda_scan(q[:, sl], k[:, sl], v[:, sl], g[:, sl], beta[:, h:h + 1], tokens=T, heads=1)
         assert_close(o[:, sl], want_o, f"o head {h}")
         assert_close(st[h], want_st[0], f"state head {h}")
+
+
+@pytest.mark.parametrize("T,H,ld,snap", [(96, 2, 0, 0), (97, 1, 0, 97), (111, 2, 320, 1), (128, 3, 0, 16),
+                                         (150, 2, 0, 33), (300, 1, 0, 299), (1000, 2, 400, 512)])
+def test_chunks(T, H, ld, snap):
+    """Runs long enough for the chunks of 16 tokens: whole and part last chunks, a snapshot that ends a chunk after the
+    first token, at a chunk's edge, inside one and before the last token."""
+    rng = np.random.default_rng(T * 3 + snap)
+    q, k, v, g, beta, state = inputs(rng, T, H, ld or None, scale_state=0.3)
+    o, st, sn = run(q, k, v, g, beta, state, T=T, H=H, ld=ld or None, snap=snap)
+    ldx = ld or H * D
+    want_o, want_st, want_sn = O.kda_scan(q, k, v, g, beta, state.astype(np.float64), tokens=T, heads=H,
+                                          qkv_stride=ldx, inner=ldx, snap=snap, o=np.full((T, ldx), 7.0))
+    assert_close(o[:T], want_o, "o")
+    assert_close(st, want_st, "state")
+    if snap:
+        assert_close(sn, want_sn, "snapshot")
+
+
+def test_chunks_strong_decays_and_growth():
+    """test_strong_decays_and_growth's decays in a run that goes by chunks: factors of e^-64 and e^48 over a chunk, a
+    channel and a head cleared by one token, a channel that grows and is cut back inside a chunk. An output is a sum of 128 terms of the state's size, each rounded
+    by up to 2^-24 an operation, and the growth leaves states of 1e18 whose terms cancel in some outputs (the recurrence
+    itself, token by token in f32, is off by 1e-3 of such an output): 128 2^-24 of the largest output of the head so
+    far, which stands for the state's size, is added to the tolerance."""
+    rng = np.random.default_rng(78)
+    T, H = 187, 2
+    q, k, v, g, beta, state = inputs(rng, T, H, scale_state=0.3)
+    g[16:32, 5] = -4.0
+    g[40, D + 7] = -50.0
+    g[70, :D] = -50.0
+    g[48:64, D + 9] = 3.0
+    g[100:104, 11] = 6.0
+    g[104:108, 11] = -6.0
+    o, st, _ = run(q, k, v, g, beta, state, T=T, H=H)
+    want_o, want_st, _ = O.kda_scan(q, k, v, g, beta, state.astype(np.float64), tokens=T, heads=H)
+    for h in range(H):
+        got, want = o[:T, h * D:(h + 1) * D], want_o[:, h * D:(h + 1) * D]
+        size = np.maximum.accumulate(np.abs(want).max(1))[:, None]
+        err = np.abs(got - want)
+        assert np.all(err <= ATOL + RTOL * np.abs(want) + 128 * 2.0 ** -24 * size), f"head {h}: worst {err.max():.3e}"
+    size = np.abs(want_st).max((1, 2), keepdims=True)
+    assert np.all(np.abs(st - want_st) <= ATOL + RTOL * np.abs(want_st) + 128 * 2.0 ** -24 * size), "state"
+
+
+def test_chunks_under_capture():
+    """A captured call on a stream the library holds no workspace for runs token by token; each replay continues the
+    state as the eager call does."""
+    rng = np.random.default_rng(79)
+    T, H = 130, 2
+    host = inputs(rng, T, H, scale_state=0.3)
+    q, k, v, g, beta, st = (dev(x) for x in host)
+    state0, o = st.clone(), torch.empty_like(v)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        M.kda_scan(q, k, v, g, beta, st, o, tokens=T, heads=H, stream=s.cuda_stream)
+    want_o, want_st, _ = O.kda_scan(*host[:5], host[5].astype(np.float64), tokens=T, heads=H)
+    for _ in range(3):
+        st.copy_(state0)
+        o.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert_close(o.cpu().numpy(), want_o, "o")
+        assert_close(st.cpu().numpy(), want_st, "state")
