@@ -176,6 +176,7 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // The rows: those of the tile's 64 that have an output (the others, a partly filled cube's padding, are not
     // computed), packed in order, 32 a wave; a lane past the last one computes a row of zeros and stores nothing.
     uint32_t row, n_rows;
+    int32_t dst;  // the row's output row
     {
         const bool has = map_l >= 0;
         const uint64_t bal = __ballot(has);
@@ -184,7 +185,9 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         // lane rank of `packed` gets the lane of the rank-th such row (the others are pushed behind, in any order)
         const uint32_t at = has ? rank : n_rows + lane - rank;
         const int packed = __builtin_amdgcn_ds_permute((int)(4 * at), (int)lane);
-        row = qt * 64 + (uint32_t)__builtin_amdgcn_ds_bpermute((int)(4 * (32 * w + c32)), packed);
+        const int from = __builtin_amdgcn_ds_bpermute((int)(4 * (32 * w + c32)), packed);
+        row = qt * 64 + (uint32_t)from;
+        dst = __builtin_amdgcn_ds_bpermute(4 * from, map_l);
     }
     const bool stores = 32 * w + c32 < n_rows;
     const uint32_t row_lo = __builtin_amdgcn_readfirstlane(row);  // this wave's first row
@@ -273,7 +276,8 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const uint32_t n_blk = ns + nd;
     uint32_t blk = 0, used = 0, held = 0;  // the next block to scan; groups of lst taken, and held
     auto scan = [&]() __attribute__((always_inline)) {
-        __syncthreads();  // both waves are done with lst
+        if (blk)
+            __syncthreads();  // both waves are done with lst
         uint32_t n = 0;
         if (used < held) {
             const uint32_t carry = lst[used];
@@ -507,7 +511,7 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const float lt = pair_sum(l);
     const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
     if (stores) {
-        TO* orow = static_cast<TO*>(p.o) + (size_t)p.map[row] * p.width + (size_t)h * kLD;
+        TO* orow = static_cast<TO*>(p.o) + (size_t)dst * p.width + (size_t)h * kLD;
 #pragma unroll
         for (int db = 0; db < 4; ++db)
 #pragma unroll

@@ -368,3 +368,35 @@ def test_per_head_lists_in_groups(causal, dense):
     G.assert_rows_l2(got, want_o, "output", 128)
     G.assert_lse_close(np.array([lse[h, r] for h, r in hr]), want_l, "lse")
     assert np.all(o != SENTINEL)
+
+
+@pytest.mark.parametrize("n_cubes,topk,local,stride,dup", [(64, 64, 0, 0, 0), (65, 33, 3, 7, 0), (405, 51, 3, 135, 0),
+                                                           (405, 51, 0, 0, 1), (100, 64, 1, 0, 2), (600, 67, 3, 11, 0)])
+def test_cube_select_many_picks(n_cubes, topk, local, stride, dup):
+    """Picks found together (up to 64 beyond the local ones) or, past 64 or where equal scores meet at the last pick, one
+    at a time: dup 1: every cube's keys twice, so that scores come in equal pairs (an odd count of picks cuts one); dup 2:
+    zero queries, all scores equal. q and k one element off 16-byte alignment. Exact against the oracle."""
+    heads, pad = 2, n_cubes * 64
+    rng = np.random.default_rng(n_cubes + topk + dup)
+    qb = G.randn_bits(rng, (heads, pad, 128), O.F16)
+    kb = G.randn_bits(rng, (heads, pad, 128), O.F16)
+    if dup == 1:
+        kc = kb.reshape(heads, n_cubes, 64 * 128)
+        kc[:, 1::2] = kc[:, 0:2 * (n_cubes // 2):2]
+    if dup == 2:
+        qb[:] = 0
+    cnt = np.full(n_cubes, 64, np.uint32)
+    want, want_n = O.cube_select(qb, kb, cnt, heads=heads, dim=128, q_pad=pad, k_pad=pad, n_cubes=n_cubes, topk=topk,
+                                 local=local, stride=stride, dtype=O.F16)[:2]
+    off = lambda b: torch.cat([torch.zeros(1, dtype=torch.float16, device="cuda"),  # noqa: E731
+                               G.to_dev(b, O.F16).reshape(-1)])[1:].reshape(b.shape)
+    kk = min(topk, n_cubes)
+    sel = torch.zeros((heads, n_cubes, kk), dtype=torch.int16, device="cuda")
+    nsel = torch.zeros((heads, n_cubes), dtype=torch.int16, device="cuda")
+    ws = torch.empty(M.cube_select_workspace(heads, n_cubes), dtype=torch.uint8, device="cuda")
+    print(f"cube select {n_cubes} top {topk} local {local} dup {dup}", flush=True)
+    M.cube_select(off(qb), off(kb), torch.from_numpy(cnt.astype(np.int32)).to("cuda"), sel, nsel, ws, heads=heads,
+                  q_pad=pad, k_pad=pad, n_cubes=n_cubes, topk=topk, local=local, stride=stride)
+    torch.cuda.synchronize()
+    assert np.array_equal(sel.cpu().numpy().view(np.uint16), want)
+    assert np.array_equal(nsel.cpu().numpy().view(np.uint16), want_n)
