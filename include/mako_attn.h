@@ -100,8 +100,8 @@ const char* mako_last_error(void);
  * offsets first write V as f16 V^T tiles into a workspace. mako_attn_fwd keeps that workspace itself, per (device, stream),
  * allocated stream-ordered the first time a call needs it (or more of it) and held until mako_attn_release(stream);
  * under graph capture a call that would grow it fails with MAKO_EWORKSPACE. Prefill calls of heads of 64 and 128 whose
- * query rows leave compute units idle split their keys in up to 128 MiB of that workspace; where it cannot be had
- * (a capture, no memory) they run unsplit.
+ * query rows leave compute units idle split their keys in up to 128 MiB of that workspace; under capture, and where it
+ * cannot be had, they run unsplit (mako_attn_fwd_ws splits them in the caller's under capture too).
  */
 int mako_attn_fwd(const mako_attn_args* a, uint32_t dim, mako_dtype in, mako_dtype out, const void* q,
                   const void* k, const void* v, void* o, float* lse, void* stream);
@@ -332,8 +332,8 @@ int mako_proj_bf16(const mako_gemm_args* a, int x_dtype, int split, const void* 
 /*
  * mako_proj_bf16 with the caller's workspace. f32 x is rounded to bf16 once, into mako_proj_bf16_workspace(a, x_dtype,
  * split) bytes (0: nothing to round ahead; at most 256 MiB); mako_proj_bf16 keeps them itself per (device, stream) until
- * mako_attn_release. With less, none, or under a capture that would have to allocate, the GEMM rounds in its loads
- * instead (slower, the same rounding).
+ * mako_attn_release. With less or none, and in mako_proj_bf16 under capture, the GEMM rounds in its loads instead (slower,
+ * the same rounding).
  */
 size_t mako_proj_bf16_workspace(const mako_gemm_args* a, int x_dtype, int split);
 int mako_proj_bf16_ws(const mako_gemm_args* a, int x_dtype, int split, const void* w, const void* x, float* y,
@@ -361,8 +361,8 @@ int mako_kda_scan(const mako_scan_args* a, const float* q, const float* k, const
 /*
  * mako_kda_scan with the caller's workspace. Long runs are computed in chunks of 16 tokens whose operands take
  * mako_kda_scan_workspace(a) bytes (0: token by token; at most 64 MiB, or one chunk's); mako_kda_scan keeps them itself
- * per (device, stream) until mako_attn_release. With less, none, or under a capture that would have to allocate, the
- * tokens run one by one.
+ * per (device, stream) until mako_attn_release. With less or none, and in mako_kda_scan under capture, the tokens run one
+ * by one.
  */
 size_t mako_kda_scan_workspace(const mako_scan_args* a);
 int mako_kda_scan_ws(const mako_scan_args* a, const float* q, const float* k, const float* v, const float* g,

@@ -109,28 +109,28 @@ __global__ __launch_bounds__(256, 1) void flash_fwd_r64(const R64Params<SPLIT> p
     const bool by_xcd = G % 8 == 0;
     const uint32_t g8 = G / 8, bx = b % 8, bk = b / 8;
     for (uint32_t round = 0;; ++round) {
-    // Item -> (head group, query block); with SPLIT the piece too.
+    const uint32_t item = by_xcd ? bx + 8 * (round * g8 + (round % 2 == 0 ? bk : g8 - 1 - bk)) : b + round * G;
+    if (!SPLIT && item >= p.n_items)
+        break;
+
+    // Item -> (head group, query block); with SPLIT the piece too. (Braces around the unsplit form cost it 14 more spilled
+    // scalar registers.)
     uint32_t hg, qb, piece = 0;
+    const uint32_t id = item;
     if constexpr (SPLIT) {
         // the list of a set of `per` head groups (an XCD's, or all): blocks of rows heaviest first, for each of them
         // its pieces, for each piece the head groups
         const bool xcd_list = by_xcd && p.n_hg % 8 == 0;
-        const uint32_t j = xcd_list ? round * g8 + (round % 2 == 0 ? bk : g8 - 1 - bk) : b + round * G;
-        const uint32_t per = xcd_list ? p.n_hg / 8 : p.n_hg;
+        const uint32_t j = xcd_list ? item / 8 : b + round * G, per = xcd_list ? p.n_hg / 8 : p.n_hg;
         const uint16_t e0 = p.ends[lane], e1 = p.ends[lane + 64];
         const uint32_t qi = __popcll(__ballot(e0 * per <= j)) + __popcll(__ballot(e1 * per <= j));
         if (qi >= p.n_qblk)
             break;
         const uint32_t r = j - (qi ? p.ends[qi - 1] * per : 0u);
         qb = p.n_qblk - 1 - qi;
-        hg = (xcd_list ? bx + 8 * (r % per) : r % per);
+        hg = xcd_list ? bx + 8 * (r % per) : r % per;
         piece = r / per;
-    } else {
-    const uint32_t item = by_xcd ? bx + 8 * (round * g8 + (round % 2 == 0 ? bk : g8 - 1 - bk)) : b + round * G;
-    if (item >= p.n_items)
-        break;
-    const uint32_t id = item;
-    if (p.n_hg % 8 == 0) {
+    } else if (p.n_hg % 8 == 0) {
         const uint32_t x = id % 8, kx = id / 8, per = p.n_hg / 8;
         if (p.block == 0) {  // bidirectional: equal work, one head group of the XCD at a time
             hg = x + 8 * (kx / p.n_qblk);
@@ -142,7 +142,6 @@ __global__ __launch_bounds__(256, 1) void flash_fwd_r64(const R64Params<SPLIT> p
     } else {
         hg = id % p.n_hg;
         qb = p.n_qblk - 1 - id / p.n_hg;
-    }
     }
     const uint32_t h = hg * p.hq + w % p.hq;
     const uint32_t kvh = hg * p.hq / p.group;
@@ -677,6 +676,7 @@ SplitPlan split_plan(const mako_attn_args* a, uint32_t cus)
 {
     constexpr double kTileUs = D == 128 ? 1.25 : 0.8, kFullUs = D == 128 ? 0.5 : 0.2, kWgUs = 8, kTurnUs = 3;
     constexpr double kMergeUs = 5;
+    constexpr uint32_t kMinTiles = 6;  // a piece
     constexpr size_t kMaxBytes = 128u << 20;
     SplitPlan best;
     const uint32_t group = a->heads / a->kv_heads;
@@ -688,6 +688,8 @@ SplitPlan split_plan(const mako_attn_args* a, uint32_t cus)
         return best;
     const auto tiles = [&](uint32_t qb) { return item_tiles(a, rows_wg, qb); };
     const uint32_t nt = tiles(n_qblk - 1);
+    if (nt < 2 * kMinTiles)
+        return best;
     const bool even = 2 * tiles(0) > nt;
     uint64_t total = 0;
     for (uint32_t qb = 0; qb < n_qblk; ++qb)
@@ -698,7 +700,9 @@ SplitPlan split_plan(const mako_attn_args* a, uint32_t cus)
     };
     const double full_us = kFullUs * total / cus;
     double best_us = 0.85 * (kTileUs * path(n_items, nt) + full_us + kWgUs);
-    for (uint32_t np = 2; np <= 16 && nt / np >= 6; ++np) {
+    if (kTileUs * total / cus + full_us + kWgUs + kMergeUs >= best_us)
+        return best;  // an even share and a merge are no shorter
+    for (uint32_t np = 2; np <= 16 && nt / np >= kMinTiles; ++np) {
         SplitPlan s;
         s.piece_tiles = (nt + np - 1) / np;
         s.pieces = np;
@@ -759,10 +763,7 @@ int launch_fwd64(const mako_attn_args* a, float scale_log2, const void* q, const
     const uint32_t n_vt = (a->n_k + 63) / 64, n_hg = a->heads / hq, n_items = n_hg * n_qblk;
     const uint32_t cus = device_cus();
     const SplitPlan sp = split_plan<D>(a, cus);
-    char* ws = nullptr;
-    // (a caller's workspace for another route of the call may be short or unaligned: no error here)
-    if (sp.pieces > 1 && !(work.given && (work.bytes < sp.bytes || reinterpret_cast<uintptr_t>(work.ptr) % 16)))
-        ws = static_cast<char*>(work.get(sp.bytes, s));
+    char* const ws = sp.pieces > 1 ? static_cast<char*>(work.try_get(sp.bytes, s)) : nullptr;
     const Fwd64Params p{q, k, v, o, lse, a->n_q, a->q_pad, a->n_k, a->k_pad, a->heads, a->kv_heads, a->q_pos0,
                         a->block, a->width, scale_log2, group, hq, rows_wg, n_qblk, n_hg, n_vt, n_items};
     if (ws) {

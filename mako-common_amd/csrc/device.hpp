@@ -208,6 +208,10 @@ struct Workspace {
     WorkspacePurpose purpose = kWsVtImages;
     const char* what = "";
     void* get(size_t need, hipStream_t s) const;
+    // For calls that run without it too: null where the caller's is short or unaligned, where the library's could not be
+    // had, and, for the library's, whenever the stream is capturing (the graph would keep the address of a buffer that a
+    // later call may replace).
+    void* try_get(size_t need, hipStream_t s) const;
     Workspace at(size_t offset) const;
 };
 inline Workspace caller_workspace(void* p, size_t bytes, const char* what)

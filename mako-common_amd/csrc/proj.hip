@@ -30,7 +30,7 @@ struct ProjParams {
     float* y;         // [t][ldy]
     uint32_t t, k, n, ldy, ldx;
     uint32_t tiles_m, tiles_n, tiles, per_xcd;
-    uint32_t planes;  // bf16 x of the DMA kernels: 2 when a row's k values are followed by k remainders (ldx covers both)
+    uint32_t planes;  // bf16 x of the DMA kernels: 2 when a row's k values come after its k remainders (ldx covers both)
 };
 
 // Tile q of the output walks bands of 4 tile rows column by column, and XCD x takes tiles x * per_xcd .. (workgroup
@@ -488,8 +488,9 @@ __global__ __launch_bounds__(256, 1) void proj_ring(const ProjParams a)
     }
 }
 
-// f32 rows rounded to bf16 once, for the DMA kernels (with SPLIT a row's remainders follow its k values). Eight values a
-// thread, streamed; bound by HBM (100 MB in 17.6 us at 4096 x 4096, 5.7 TB/s). Rounding in the tiles' staging repeats
+// f32 rows rounded to bf16 once, for the DMA kernels (with SPLIT a row's remainders precede its k values: added
+// first, they meet small sums; after them, the error against 64 bits was 7.0e-7 at k = 4096 where the two products
+// interleaved gave 5.7e-7). Eight values a thread, streamed; bound by HBM (100 MB in 17.6 us at 4096 x 4096, 5.7 TB/s). Rounding in the tiles' staging repeats
 // the work and the 32-bit reads in every column of tiles and goes through registers: 167 us at 4096 x 4096, against 129
 // for this pass and the DMA kernel (with the split 269 and 233; t = 300: 133 and 28).
 template <bool SPLIT>
@@ -511,9 +512,9 @@ __global__ __launch_bounds__(256) void round_rows(const float* __restrict__ x, _
             lo[e] = Elem<__bf16>::pack2(f[2 * e] - (float)(__bf16)f[2 * e], f[2 * e + 1] - (float)(__bf16)f[2 * e + 1]);
     }
     __bf16* o = out + (size_t)row * k * (SPLIT ? 2 : 1) + c;
-    *reinterpret_cast<u32x4*>(o) = hi;
+    *reinterpret_cast<u32x4*>(o + (SPLIT ? k : 0)) = hi;
     if (SPLIT)
-        *reinterpret_cast<u32x4*>(o + k) = lo;
+        *reinterpret_cast<u32x4*>(o) = lo;
 }
 
 // A few rows of x (decode, short verification steps): t <= 16 TB. Bound: the read of w (33.6 MB at 4096 x 4096). A
@@ -793,8 +794,8 @@ int proj_core(const mako_gemm_args* a, int x_dtype, int split, const void* w, co
     // caller's shorter one, more than kMaxRounded bytes) the kernels round as they load.
     const uint64_t planes = split ? 2 : 1;
     const size_t bytes = rounded_bytes(a, x_dtype, split);
-    if (bytes && !(work.given && (work.bytes < bytes || !al16(work.ptr)))) {
-        if (void* ws = work.get(bytes, s)) {
+    if (bytes) {
+        if (void* ws = work.try_get(bytes, s)) {
             const dim3 grid((uint32_t)(((uint64_t)a->t * (a->k / 8) + 255) / 256));
             if (split)
                 hipLaunchKernelGGL(round_rows<true>, grid, dim3(256), 0, s, static_cast<const float*>(x),
