@@ -1,7 +1,7 @@
 """Prefill calls whose keys are split over workgroups (flash_fwd_r64's split grid and merge_pieces): a few blocks of
 query rows over a long cache, causal rows whose last block runs longest, bidirectional rows, prefix-causal rows, at
 heads of 128 and 64. Each is checked against the CPU oracle, and against the same call with no workspace, which runs
-unsplit; under stream capture, where nothing can be allocated, the call runs unsplit too."""
+unsplit; under stream capture the call runs unsplit too, whether or not the library holds a workspace for the stream."""
 import numpy as np
 import pytest
 
@@ -67,6 +67,8 @@ def test_split_prefill_under_capture():
     M.attn_fwd(q, k, v, want, workspace=None, **args)
     s = torch.cuda.Stream()
     s.wait_stream(torch.cuda.current_stream())
+    M.attn_fwd(q, k, v, o, stream=s.cuda_stream, **args)  # the library holds the workspace; the graph must not keep it
+    s.synchronize()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph, stream=s):
         M.attn_fwd(q, k, v, o, lse=lse, stream=s.cuda_stream, **args)
