@@ -100,8 +100,8 @@ const char* mako_last_error(void);
  * offsets first write V as f16 V^T tiles into a workspace. mako_attn_fwd keeps that workspace itself, per (device, stream),
  * allocated stream-ordered the first time a call needs it (or more of it) and held until mako_attn_release(stream);
  * under graph capture a call that would grow it fails with MAKO_EWORKSPACE. Prefill calls of heads of 64 and 128 whose
- * query rows leave compute units idle split their keys in up to 128 MiB of that workspace; under capture, and where it
- * cannot be had, they run unsplit (mako_attn_fwd_ws splits them in the caller's under capture too).
+ * query rows leave compute units idle split their keys in up to 128 MiB of a second one, kept the same way; under capture,
+ * and where it cannot be had, they run unsplit (mako_attn_fwd_ws splits them in the caller's under capture too).
  */
 int mako_attn_fwd(const mako_attn_args* a, uint32_t dim, mako_dtype in, mako_dtype out, const void* q,
                   const void* k, const void* v, void* o, float* lse, void* stream);

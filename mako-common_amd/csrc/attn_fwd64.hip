@@ -763,7 +763,7 @@ int launch_fwd64(const mako_attn_args* a, float scale_log2, const void* q, const
     const uint32_t n_vt = (a->n_k + 63) / 64, n_hg = a->heads / hq, n_items = n_hg * n_qblk;
     const uint32_t cus = device_cus();
     const SplitPlan sp = split_plan<D>(a, cus);
-    char* const ws = sp.pieces > 1 ? static_cast<char*>(work.try_get(sp.bytes, s)) : nullptr;
+    char* const ws = sp.pieces > 1 ? static_cast<char*>(work.try_get(kWsPieces, sp.bytes, s)) : nullptr;
     const Fwd64Params p{q, k, v, o, lse, a->n_q, a->q_pad, a->n_k, a->k_pad, a->heads, a->kv_heads, a->q_pos0,
                         a->block, a->width, scale_log2, group, hq, rows_wg, n_qblk, n_hg, n_vt, n_items};
     if (ws) {

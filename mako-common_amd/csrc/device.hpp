@@ -194,7 +194,13 @@ uint32_t device_cus();
 // handle). Returns null, with nothing allocated and the error recorded, when the allocation fails (MAKO_EHIP) or
 // when the stream is capturing a graph and the buffer would have to grow (MAKO_EWORKSPACE: an allocation in a
 // capture would belong to the graph).
-enum WorkspacePurpose { kWsVtImages = 0, kWsSplitK = 1, kWsRowTiles = 2, kWsPassTable = 3, kWsRounded = 4, kWsScan = 5, kWsPurposes = 6 };
+enum WorkspacePurpose {
+    kWsVtImages = 0, kWsSplitK = 1, kWsRowTiles = 2, kWsPassTable = 3,
+    // of calls that run without it too (Workspace::try_get): never those of get, so that a call that can do without
+    // does not grow, and so replace, a buffer whose address a captured graph holds
+    kWsRounded = 4, kWsScan = 5, kWsPieces = 6,
+    kWsPurposes = 7
+};
 void* stream_workspace(WorkspacePurpose purpose, size_t bytes, hipStream_t s, const char* what);
 
 // A call's workspace: the caller's buffer (given, from an entry point that takes one: never allocates) or the
@@ -208,10 +214,10 @@ struct Workspace {
     WorkspacePurpose purpose = kWsVtImages;
     const char* what = "";
     void* get(size_t need, hipStream_t s) const;
-    // For calls that run without it too: null where the caller's is short or unaligned, where the library's could not be
-    // had, and, for the library's, whenever the stream is capturing (the graph would keep the address of a buffer that a
-    // later call may replace).
-    void* try_get(size_t need, hipStream_t s) const;
+    // For calls that run without it too: null where the caller's is short or unaligned, where the library's (the buffer
+    // of `optional`, not of purpose) could not be had, and, for the library's, whenever the stream is capturing (the
+    // graph would keep the address of a buffer that a later call may replace).
+    void* try_get(WorkspacePurpose optional, size_t need, hipStream_t s) const;
     Workspace at(size_t offset) const;
 };
 inline Workspace caller_workspace(void* p, size_t bytes, const char* what)

@@ -795,7 +795,7 @@ int proj_core(const mako_gemm_args* a, int x_dtype, int split, const void* w, co
     const uint64_t planes = split ? 2 : 1;
     const size_t bytes = rounded_bytes(a, x_dtype, split);
     if (bytes) {
-        if (void* ws = work.try_get(bytes, s)) {
+        if (void* ws = work.try_get(kWsRounded, bytes, s)) {
             const dim3 grid((uint32_t)(((uint64_t)a->t * (a->k / 8) + 255) / 256));
             if (split)
                 hipLaunchKernelGGL(round_rows<true>, grid, dim3(256), 0, s, static_cast<const float*>(x),

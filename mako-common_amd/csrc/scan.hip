@@ -596,7 +596,7 @@ int scan_core(const mako_scan_args* a, const float* q, const float* k, const flo
     // v's rows suit 16-byte DMA from 32-bit offsets
     const size_t bytes = scan_bytes(a);
     if (bytes && al16(v) && a->qkv_stride < (1u << 25)) {
-        if (ChunkImage* ws = static_cast<ChunkImage*>(work.try_get(bytes, s))) {
+        if (ChunkImage* ws = static_cast<ChunkImage*>(work.try_get(kWsScan, bytes, s))) {
             const uint32_t n = chunks_of(a), per = chunks_a_launch(a);
             for (uint32_t c = 0; c < n; c += per) {
                 const ChunkParams cp{p, ws, c, std::min(per, n - c), (a->snap + kChunk - 1) / kChunk};

@@ -112,14 +112,14 @@ void* Workspace::get(size_t need, hipStream_t s) const
     return ptr;
 }
 
-void* Workspace::try_get(size_t need, hipStream_t s) const
+void* Workspace::try_get(WorkspacePurpose optional, size_t need, hipStream_t s) const
 {
     if (given)
         return bytes >= need && reinterpret_cast<uintptr_t>(ptr) % 16 == 0 ? ptr : nullptr;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cap) != hipSuccess)
         (void)hipGetLastError();
-    return cap == hipStreamCaptureStatusNone ? stream_workspace(purpose, need, s, what) : nullptr;
+    return cap == hipStreamCaptureStatusNone ? stream_workspace(optional, need, s, what) : nullptr;
 }
 
 Workspace Workspace::at(size_t offset) const
