@@ -122,6 +122,9 @@ int mako_attn_fwd_ws(const mako_attn_args* a, uint32_t dim, mako_dtype in, mako_
 /*
  * The workspaces the entry points without a workspace argument keep for a stream (on the current device): waits for
  * the stream, then frees them. No counterpart in the reference (its Runtime frees its scratch at destruction).
+ * Threads may call on one stream at the same time: a call has the stream's workspaces to itself from the first use until
+ * its last launch. On hipStreamPerThread they are the calling thread's, which releases them, and calls that can run
+ * without one (split prefill, f32 rows of mako_proj_bf16, chunks of mako_kda_scan) do.
  * mako_attn_held_bytes: the bytes held on the current device, over all streams.
  */
 int mako_attn_release(void* stream);

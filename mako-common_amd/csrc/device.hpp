@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <mutex>
+
 #include "mako_attn.h"
 
 namespace mako {
@@ -189,11 +191,11 @@ uint32_t device_cus();
 
 // Workspaces the library keeps for callers that pass none: one buffer per (purpose, device, stream), grown (stream-
 // ordered) when a call needs more. Calls on one stream are ordered by the stream and calls on different streams use
-// different buffers, so no call waits on the host or inserts a GPU-side wait. A stream's buffers stay until
-// mako_attn_release(stream) frees them (a stream destroyed without it leaves them to a later stream with its
-// handle). Returns null, with nothing allocated and the error recorded, when the allocation fails (MAKO_EHIP) or
-// when the stream is capturing a graph and the buffer would have to grow (MAKO_EWORKSPACE: an allocation in a
-// capture would belong to the graph).
+// different buffers, so no call inserts a GPU-side wait. A call has the stream's buffers to itself from its first
+// lookup until it has enqueued its last launch (StreamHeld::turn), so that another thread's call on the stream neither
+// writes between its launches nor frees what it is about to launch with; threads wait for that time only. A stream's
+// buffers stay until mako_attn_release(stream) frees them (a stream destroyed without it leaves them to a later stream
+// with its handle). hipStreamPerThread is another stream in each thread: its buffers are the thread's.
 enum WorkspacePurpose {
     kWsVtImages = 0, kWsSplitK = 1, kWsRowTiles = 2, kWsPassTable = 3,
     // of calls that run without it too (Workspace::try_get): never those of get, so that a call that can do without
@@ -201,12 +203,13 @@ enum WorkspacePurpose {
     kWsRounded = 4, kWsScan = 5, kWsPieces = 6,
     kWsPurposes = 7
 };
-void* stream_workspace(WorkspacePurpose purpose, size_t bytes, hipStream_t s, const char* what);
 
 // A call's workspace: the caller's buffer (given, from an entry point that takes one: never allocates) or the
-// library's buffer for (purpose, device, stream). get(need) returns memory of at least need bytes, or null with the
-// error recorded (MAKO_EWORKSPACE when the caller's buffer is smaller, else as stream_workspace). Slices of a given
-// workspace are taken with at(offset).
+// library's buffer for (purpose, device, stream), which it keeps from other threads until it is destroyed, at the end
+// of the call. get(need) returns memory of at least need bytes, or null, with nothing allocated and the error recorded,
+// when the caller's buffer is smaller (MAKO_EWORKSPACE), when the allocation fails (MAKO_EHIP) or when the stream is
+// capturing a graph and the buffer would have to grow (MAKO_EWORKSPACE: an allocation in a capture would belong to the
+// graph). Slices of a given workspace are taken with at(offset).
 struct Workspace {
     void* ptr = nullptr;
     size_t bytes = 0;
@@ -216,9 +219,14 @@ struct Workspace {
     void* get(size_t need, hipStream_t s) const;
     // For calls that run without it too: null where the caller's is short or unaligned, where the library's (the buffer
     // of `optional`, not of purpose) could not be had, and, for the library's, whenever the stream is capturing (the
-    // graph would keep the address of a buffer that a later call may replace).
+    // graph would keep the address of a buffer that a later call may replace) or is hipStreamPerThread (each thread
+    // that ends would leave one behind).
     void* try_get(WorkspacePurpose optional, size_t need, hipStream_t s) const;
     Workspace at(size_t offset) const;
+
+private:
+    void* held(WorkspacePurpose which, size_t need, hipStream_t s) const;
+    mutable std::unique_lock<std::recursive_mutex> turn_;  // (a call may hold two workspaces of its stream)
 };
 inline Workspace caller_workspace(void* p, size_t bytes, const char* what)
 {

@@ -1,11 +1,13 @@
 // The C ABI's error plumbing: a per-thread message for mako_last_error().
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdarg>
 #include <cstdio>
 #include <map>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <tuple>
 
 #include "device.hpp"
@@ -65,22 +67,38 @@ uint32_t device_cus()
 }
 
 namespace {
-struct Held {
-    void* ptr = nullptr;
-    size_t bytes = 0;
+// A stream's buffers, one a purpose. Entries stay (without memory) once made, so a reference outlives ws_mu.
+struct StreamHeld {
+    std::recursive_mutex turn;  // held by the call that uses the buffers
+    struct {
+        void* ptr = nullptr;
+        std::atomic<size_t> bytes{0};  // (mako_attn_held_bytes reads it without the turn)
+    } buf[kWsPurposes];
 };
-std::mutex ws_mu;
-std::map<std::tuple<int, int, hipStream_t>, Held> ws_all;  // (purpose, device, stream)
+using StreamKey = std::tuple<int, hipStream_t, std::thread::id>;
+std::mutex ws_mu;  // ws_all, not what its entries hold
+std::map<StreamKey, StreamHeld> ws_all;
+
+StreamKey stream_key(int dev, hipStream_t s)
+{
+    return {dev, s, s == hipStreamPerThread ? std::this_thread::get_id() : std::thread::id()};
+}
 }  // namespace
 
-void* stream_workspace(WorkspacePurpose purpose, size_t bytes, hipStream_t s, const char* what)
+void* Workspace::held(WorkspacePurpose which, size_t need, hipStream_t s) const
 {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess)
         return fail(MAKO_EHIP, "%s: no current device", what), nullptr;
-    std::lock_guard<std::mutex> lock(ws_mu);
-    Held& ws = ws_all[{(int)purpose, dev, s}];
-    if (ws.bytes < bytes) {
+    StreamHeld* all;
+    {
+        std::lock_guard<std::mutex> lock(ws_mu);
+        all = &ws_all[stream_key(dev, s)];
+    }
+    if (!turn_.owns_lock())
+        turn_ = std::unique_lock<std::recursive_mutex>(all->turn);
+    auto& ws = all->buf[which];
+    if (ws.bytes < need) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(s, &cap) != hipSuccess)
             (void)hipGetLastError();
@@ -88,17 +106,17 @@ void* stream_workspace(WorkspacePurpose purpose, size_t bytes, hipStream_t s, co
             return fail(MAKO_EWORKSPACE,
                         "%s: the stream is capturing a graph and the library's workspace would grow to %zu bytes; "
                         "pass a workspace (the *_ws entry point) or make the call once before the capture",
-                        what, bytes), nullptr;
+                        what, need), nullptr;
         if (ws.ptr)
             (void)hipFreeAsync(ws.ptr, s);  // after the previous use on this stream
         ws.ptr = nullptr;
         ws.bytes = 0;
-        if (hipMallocAsync(&ws.ptr, bytes, s) != hipSuccess) {
+        if (hipMallocAsync(&ws.ptr, need, s) != hipSuccess) {
             (void)hipGetLastError();
             ws.ptr = nullptr;
-            return fail(MAKO_EHIP, "%s: no device memory for a workspace of %zu bytes", what, bytes), nullptr;
+            return fail(MAKO_EHIP, "%s: no device memory for a workspace of %zu bytes", what, need), nullptr;
         }
-        ws.bytes = bytes;
+        ws.bytes = need;
     }
     return ws.ptr;
 }
@@ -106,7 +124,7 @@ void* stream_workspace(WorkspacePurpose purpose, size_t bytes, hipStream_t s, co
 void* Workspace::get(size_t need, hipStream_t s) const
 {
     if (!given)
-        return stream_workspace(purpose, need, s, what);
+        return held(purpose, need, s);
     if (bytes < need || (need && !ptr))
         return fail(MAKO_EWORKSPACE, "%s: a workspace of %zu bytes, the call needs %zu", what, bytes, need), nullptr;
     return ptr;
@@ -116,20 +134,20 @@ void* Workspace::try_get(WorkspacePurpose optional, size_t need, hipStream_t s) 
 {
     if (given)
         return bytes >= need && reinterpret_cast<uintptr_t>(ptr) % 16 == 0 ? ptr : nullptr;
+    if (s == hipStreamPerThread)
+        return nullptr;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cap) != hipSuccess)
         (void)hipGetLastError();
-    return cap == hipStreamCaptureStatusNone ? stream_workspace(optional, need, s, what) : nullptr;
+    return cap == hipStreamCaptureStatusNone ? held(optional, need, s) : nullptr;
 }
 
 Workspace Workspace::at(size_t offset) const
 {
-    Workspace w = *this;
-    if (given) {
-        w.ptr = offset <= bytes ? static_cast<char*>(ptr) + offset : nullptr;
-        w.bytes = offset <= bytes ? bytes - offset : 0;
-    }
-    return w;
+    if (!given)
+        return library_workspace(purpose, what);
+    return offset <= bytes ? caller_workspace(static_cast<char*>(ptr) + offset, bytes - offset, what)
+                           : caller_workspace(nullptr, 0, what);
 }
 
 }  // namespace mako
@@ -143,18 +161,25 @@ extern "C" int mako_attn_release(void* stream)
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess)
         return fail(MAKO_EHIP, "release: no current device");
+    StreamHeld* all = nullptr;
+    {
+        std::lock_guard<std::mutex> lock(ws_mu);
+        const auto it = ws_all.find(stream_key(dev, s));
+        if (it != ws_all.end())
+            all = &it->second;
+    }
+    std::unique_lock<std::recursive_mutex> turn;
+    if (all)
+        turn = std::unique_lock<std::recursive_mutex>(all->turn);
     if (hipStreamSynchronize(s) != hipSuccess)
         return fail(MAKO_EHIP, "release: %s", hipGetErrorString(hipGetLastError()));
-    std::lock_guard<std::mutex> lock(ws_mu);
-    for (auto it = ws_all.begin(); it != ws_all.end();) {
-        if (std::get<1>(it->first) == dev && std::get<2>(it->first) == s) {
-            if (it->second.ptr && hipFree(it->second.ptr) != hipSuccess)
+    if (all)
+        for (auto& ws : all->buf) {
+            if (ws.ptr && hipFree(ws.ptr) != hipSuccess)
                 return fail(MAKO_EHIP, "release: %s", hipGetErrorString(hipGetLastError()));
-            it = ws_all.erase(it);
-        } else {
-            ++it;
+            ws.ptr = nullptr;
+            ws.bytes = 0;
         }
-    }
     return ok();
 }
 
@@ -167,8 +192,9 @@ extern "C" size_t mako_attn_held_bytes(void)
     std::lock_guard<std::mutex> lock(ws_mu);
     size_t n = 0;
     for (const auto& kv : ws_all)
-        if (std::get<1>(kv.first) == dev)
-            n += kv.second.bytes;
+        if (std::get<0>(kv.first) == dev)
+            for (const auto& ws : kv.second.buf)
+                n += ws.bytes;
     return n;
 }
 

@@ -3,6 +3,7 @@ launches and runs nothing (tests/cpp/fake_hip.cpp; 256 compute units). Pointers 
 import ctypes
 import os
 import subprocess
+import threading
 import types
 
 import pytest
@@ -91,3 +92,89 @@ def test_split_prefill_without_memory_keeps_the_other_workspaces(hip):
         hip.fake_alloc_limit(ctypes.c_size_t(-1).value)
     assert len(launches(hip)) == 1 and events(hip, "free") == []
     M.release(stream=s)
+
+
+def proj(t, stream, k=4096, n=4096):
+    M.proj_bf16(tensor(torch.bfloat16), tensor(torch.float32), tensor(torch.float32), t=t, k=k, n=n, stream=stream)
+
+
+def scan(tokens, stream):
+    x = tensor(torch.float32)
+    M.kda_scan(x, x, x, x, x, x, x, tokens=tokens, heads=4, stream=stream)
+
+
+# a call whose launches pass a workspace on, and one that needs more of it
+TWO_LAUNCHES = {
+    "proj": (lambda s: proj(256, s), lambda s: proj(512, s)),
+    "scan": (lambda s: scan(128, s), lambda s: scan(256, s)),
+    "prefill": (lambda s: attn(333, 9333, s), lambda s: attn(333, 20000, s)),
+    "few rows": (lambda s: attn(1, 4096, s), lambda s: attn(2, 40000, s)),
+    "rows": (lambda s: rows(300, 300, s), lambda s: rows(600, 600, s)),
+}
+
+
+@pytest.mark.parametrize("name", TWO_LAUNCHES)
+def test_threads_on_one_stream_take_turns(hip, name):
+    """Another thread's call on the stream, made between a call's two launches, neither launches in between nor frees
+    the buffer they share, and runs after it."""
+    first, second = TWO_LAUNCHES[name]
+    s = 0x53000
+    other = threading.Thread(target=second, args=(s,))
+    main = threading.get_ident()
+    seen = []
+
+    @ctypes.CFUNCTYPE(None, ctypes.c_char_p)
+    def hook(kernel):
+        seen.append(threading.get_ident() == main)
+        if len(seen) == 1:
+            other.start()
+            other.join(0.3)  # (time enough to come between)
+
+    hip.fake_launch_hook(hook)
+    try:
+        first(s)
+        other.join()
+    finally:
+        hip.fake_launch_hook(None)
+    n = seen.index(False)
+    assert n >= 2 and not any(seen[n:]), seen
+    kinds = [e[0] for e in events(hip, "launch", "free")]
+    assert "free" not in kinds[:n]
+    M.release(stream=s)
+
+
+PER_THREAD = 2  # hipStreamPerThread
+
+
+def test_per_thread_stream(hip):
+    """hipStreamPerThread is a stream of the calling thread: a workspace that has to be is the thread's own, and calls
+    that run without one do."""
+    for call in (TWO_LAUNCHES["proj"][0], TWO_LAUNCHES["scan"][0], TWO_LAUNCHES["prefill"][0]):
+        hip.fake_clear()
+        call(PER_THREAD)
+        assert events(hip, "alloc") == [] and len(launches(hip)) == 1, launches(hip)
+    hip.fake_clear()
+
+    def few_rows():
+        attn(1, 4096, PER_THREAD)
+        attn(1, 4096, PER_THREAD)
+        M.release(stream=PER_THREAD)
+
+    attn(1, 4096, PER_THREAD)
+    other = threading.Thread(target=few_rows)
+    other.start()
+    other.join()
+    attn(1, 4096, PER_THREAD)
+    allocs, frees = ([e[1] for e in events(hip, k)] for k in ("alloc", "free"))
+    assert len(allocs) == 2 and frees == allocs[1:]
+    M.release(stream=PER_THREAD)
+
+
+def test_release_frees_every_workspace_of_the_stream(hip):
+    s, before = 0x54000, M.held_bytes()
+    for first, _ in TWO_LAUNCHES.values():
+        first(s)
+    allocs = [e[1] for e in events(hip, "alloc")]
+    assert M.held_bytes() - before == sum(int(e[2]) for e in events(hip, "alloc"))
+    M.release(stream=s)
+    assert sorted(e[1] for e in events(hip, "free")) == sorted(allocs) and M.held_bytes() == before
