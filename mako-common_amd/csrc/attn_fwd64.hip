@@ -275,6 +275,9 @@ __global__ __launch_bounds__(256, 1) void flash_fwd_r64(const R64Params<SPLIT> p
 
 // The rows of items with more than one piece, from query row row0 on: the pieces' normalised rows weighted by
 // exp(their log-sum - the largest). D / 4 lanes a (row, head), four head dims each; bound by the read of the pieces.
+// A piece whose sum is not above 0 has a log-sum of -inf: zeros where every score was -inf, NaN where one was not a
+// number. Its row is added with weight 0, so NaN reaches the result whichever piece it is in; a row that is NaN
+// throughout makes the sum NaN too, and so the log-sum -inf, as in the call without pieces.
 template <class TO, int D>
 __global__ __launch_bounds__(256) void merge_pieces(const SplitParams p, uint32_t row0)
 {
@@ -294,27 +297,33 @@ __global__ __launch_bounds__(256) void merge_pieces(const SplitParams p, uint32_
         float l[U];
         f32x4 v[U];
         #pragma unroll
-        for (uint32_t u = 0; u < U; ++u) {  // (an empty piece wrote nothing)
+        for (uint32_t u = 0; u < U; ++u) {  // (an empty piece wrote nothing: zeros)
             const bool has = i0 + u < pc.np && pc.start(i0 + u) < pc.start(i0 + u + 1);
             l[u] = has ? pl[(i0 + u) * ls] : -INFINITY;
             v[u] = has ? *reinterpret_cast<const f32x4*>(po + (i0 + u) * os) : f32x4{};
         }
         #pragma unroll
         for (uint32_t u = 0; u < U; ++u) {
-            const float m = fmaxf(mx, l[u]);
-            if (m == -INFINITY)
+            if (l[u] == -INFINITY) {  // (the same in a row's lanes)
+                const uint64_t nan = __ballot(v[u][0] != v[u][0] && v[u][1] != v[u][1] && v[u][2] != v[u][2] && v[u][3] != v[u][3]);
+                const uint64_t row_lanes = ((1ull << (D / 4)) - 1) << (threadIdx.x & 63u & ~(D / 4 - 1));
+                acc += v[u] * 0.0f;
+                if ((nan & row_lanes) == row_lanes)
+                    sum = NAN;
                 continue;
+            }
+            const float m = fmaxf(mx, l[u]);
             const float a = exp2_fast((mx - m) * kLog2e), b = exp2_fast((l[u] - m) * kLog2e);
             sum = sum * a + b;
             acc = acc * a + v[u] * b;
             mx = m;
         }
     }
-    const float inv = sum != 0.0f ? 1.0f / sum : 0.0f;
+    const float inv = sum > 0.0f ? 1.0f / sum : 0.0f;
     store4<TO>(static_cast<TO*>(p.o) + (size_t)row * p.width + (size_t)h * D + d, acc[0] * inv, acc[1] * inv,
                acc[2] * inv, acc[3] * inv);
     if (p.lse && d == 0)
-        p.lse[(size_t)h * p.n_q + row] = sum != 0.0f ? mx + __log2f(sum) * kLn2 : -INFINITY;
+        p.lse[(size_t)h * p.n_q + row] = sum > 0.0f ? mx + __log2f(sum) * kLn2 : -INFINITY;
 }
 
 // Heads of 256 (Qwen3.5's gated attention): flash_fwd_d256. The parallelism of the usual shapes (16 query heads,

@@ -77,3 +77,35 @@ def test_split_prefill_under_capture():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(o, want)
+
+
+NONFINITE = [
+    # tensor, its first row changed, value; the calls below cut 1500 keys into pieces of at least six 64-key tiles
+    ("k", 5, "nan"), ("k", 1001, "nan"), ("k", 5, "inf"), ("k", 1001, "inf"), ("k", 1001, "-inf"),
+    ("v", 5, "nan"), ("v", 1001, "inf"), ("q", 0, "nan"), ("q", 69, "inf"),
+]
+
+
+@pytest.mark.parametrize("what,row,value", NONFINITE, ids=lambda x: str(x))
+@pytest.mark.parametrize("dim,dt,out", [(128, O.BF16, "same"), (64, O.F16, "f32")], ids=["d128", "d64"])
+def test_split_prefill_carries_non_finite_values(dim, dt, out, what, row, value):
+    """One value that is not finite, in the first piece's keys, a later one's or a query: the split call's outputs and
+    log-sums are not finite where the unsplit call's are not, and agree elsewhere (each side is within the tolerance of
+    the exact result, so they differ by twice it at most)."""
+    host, args, o, lse = inputs((dim, 8, 2, 70, 1500, 1430, U32, dt, out))
+    q, k, v = (G.to_dev(b, dt) for b in host)
+    {"q": q, "k": k, "v": v}[what][:, row, 3] = float(value)
+    need = M.attn_fwd_workspace(**args)
+    assert need > 0, "the call is not split"
+    M.attn_fwd(q, k, v, o, lse=lse, workspace=torch.empty(need, dtype=torch.uint8, device="cuda"), **args)
+    o1, lse1 = torch.full_like(o, float("nan")), torch.full_like(lse, float("nan"))
+    M.attn_fwd(q, k, v, o1, lse=lse1, workspace=None, **args)
+    torch.cuda.synchronize()
+    for got, want in ((o, o1), (lse, lse1)):
+        assert torch.equal(torch.isnan(got), torch.isnan(want))
+        inf = torch.isinf(want)
+        assert torch.equal(torch.isinf(got), inf) and torch.equal(got[inf], want[inf])
+        ok = torch.isfinite(want)
+        err = (got[ok].float() - want[ok].float()).abs()
+        assert bool((err <= 2 * (G.ATOL + G.RTOL * want[ok].float().abs())).all())
+    assert bool((~torch.isfinite(o1)).any())
