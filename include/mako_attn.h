@@ -364,8 +364,10 @@ int mako_kda_scan(const mako_scan_args* a, const float* q, const float* k, const
 /*
  * mako_kda_scan with the caller's workspace. Long runs are computed in chunks of 16 tokens whose operands take
  * mako_kda_scan_workspace(a) bytes (0: token by token; at most 64 MiB, or one chunk's); mako_kda_scan keeps them itself
- * per (device, stream) until mako_attn_release. With less or none, and in mako_kda_scan under capture, the tokens run one
- * by one.
+ * per (device, stream) until mako_attn_release. With less or none, in mako_kda_scan under capture, and with o over v or
+ * snap_state over state, the tokens run one by one: the same sums in another order, so the bits differ. A launch that
+ * meets a value that is not finite (an input, or decays that grow past f32 over a chunk) runs its tokens one by one too,
+ * so such a value reaches the same outputs on either route.
  */
 size_t mako_kda_scan_workspace(const mako_scan_args* a);
 int mako_kda_scan_ws(const mako_scan_args* a, const float* q, const float* k, const float* v, const float* g,

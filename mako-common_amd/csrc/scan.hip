@@ -65,17 +65,24 @@ __device__ __forceinline__ float row_sum(float x)
     return x;
 }
 
-// LANES lanes a state row, V = 128 / LANES values a lane in G = V / 4 runs of 4 channels: run r of lane l holds
-// channels 4 LANES r + 4 l .. + 3, so a run of the lanes of a row is 16 LANES contiguous bytes of a vector.
+// The LDS of the token-by-token scan: two batch buffers, the next batch's rows are fetched into registers while this
+// batch runs out of LDS.
 template <int LANES>
-__global__ __launch_bounds__(256) void kda_scan_rows(const ScanParams a)
+struct RowsLds {
+    float q[2][kBatch][kD], k[2][kBatch][kD], e[2][kBatch][kD];
+    float v[2][kBatch][256 / LANES], b[2][kBatch], o[2][kBatch][256 / LANES];
+};
+
+// LANES lanes a state row, V = 128 / LANES values a lane in G = V / 4 runs of 4 channels: run r of lane l holds
+// channels 4 LANES r + 4 l .. + 3, so a run of the lanes of a row is 16 LANES contiguous bytes of a vector. The work of
+// threads 0 .. 255 of workgroup (head, rows); lds 16-byte aligned.
+template <int LANES>
+__device__ __forceinline__ void scan_rows(const ScanParams& a, RowsLds<LANES>& lds)
 {
     constexpr int V = kD / LANES, G = V / 4, ROWS = 256 / LANES;
-    // two batch buffers: the next batch's rows are fetched into registers while this batch runs out of LDS
-    __shared__ __attribute__((aligned(16))) float qs[2][kBatch][kD];
-    __shared__ __attribute__((aligned(16))) float ks[2][kBatch][kD];
-    __shared__ __attribute__((aligned(16))) float es[2][kBatch][kD];
-    __shared__ float vs[2][kBatch][ROWS], bs[2][kBatch], os[2][kBatch][ROWS];
+    auto &qs = lds.q, &ks = lds.k, &es = lds.e;
+    auto &vs = lds.v, &os = lds.o;
+    auto& bs = lds.b;
     const uint32_t tid = threadIdx.x, h = blockIdx.x, j0 = blockIdx.y * ROWS, row = tid / LANES, l = tid % LANES;
     uint32_t ch[G];
     #pragma unroll
@@ -238,6 +245,15 @@ __global__ __launch_bounds__(256) void kda_scan_rows(const ScanParams a)
         *reinterpret_cast<f32x4*>(mg + ch[r]) = f32x4{m[4 * r], m[4 * r + 1], m[4 * r + 2], m[4 * r + 3]};
 }
 
+template <int LANES>
+__global__ __launch_bounds__(256) void kda_scan_rows(const ScanParams a)
+{
+    __shared__ __attribute__((aligned(16))) RowsLds<LANES> lds;
+    scan_rows<LANES>(a, lds);
+}
+
+constexpr int kScanLanes = 16;  // lanes a state row: 8 values a lane, one wave a SIMD at 32 heads
+
 // ---- long runs: chunks of 16 tokens ------------------------------------------------------------------------------
 //
 // Token by token the recurrence is a serial chain of ~400 cycles a token on a quarter of the issue slots (4096 tokens of
@@ -247,9 +263,16 @@ __global__ __launch_bounds__(256) void kda_scan_rows(const ScanParams a)
 //   A[t][s] = k_t . E(t, s) k_s (s < t),  B[t][s] = q_t . E(t, s) k_s (s <= t),  W = (1 + diag(beta) A)^-1 diag(beta)
 // (the delta rule's 16 rank-one updates solved at once), which is seven small matrix products. Products of decays are
 // formed one factor at a time as the recurrence forms them, never as exponentials of summed logarithms or as ratios:
-// no cancellation, no overflow where the recurrence has none. Everything is f32, on v_mfma_f32_16x16x4_f32; against 64
-// bits the outputs are within 1 % of the recurrence's error (1.65e-7 against 1.67e-7 over 97 to 3000 tokens), the state
-// closer (1.37e-7 and 1.53e-7: one rounding at its size a chunk).
+// no cancellation. Everything is f32, on v_mfma_f32_16x16x4_f32; against 64 bits the outputs are within 1 % of the
+// recurrence's error (1.65e-7 against 1.67e-7 over 97 to 3000 tokens), the state closer (1.37e-7 and 1.53e-7: one
+// rounding at its size a chunk).
+//
+// The products take terms the recurrence does not have, times zero: tokens after the output's (W and B above their
+// diagonals) and channels whose state is 0. Where all factors are finite that is exact. Where one is not (an input, or a
+// product of decays that grow past f32, which may meet a state of 0), the launch's tokens are left to the recurrence:
+// kda_chunk marks the chunk, or its d is not finite, and the workgroup, its state not yet stored, takes them by scan_rows.
+// A value that is not finite then reaches what it reaches token by token. The output wave looks, off the state's chain
+// (on it, a look at d and a way out of the loop took 5 to 9 %).
 //
 // kda_chunk: a workgroup a (chunk, head) makes everything of a chunk that needs no state, as the LDS image of the next
 // kernel's stage (28 KiB in the workspace): Gamma k, Gamma q, E(last, .) k, Gamma_last, W and B.
@@ -266,7 +289,8 @@ struct ChunkImage {
     float kg[kChunk][kCRow], qg[kChunk][kCRow], ke[kChunk][kCRow];
     float last[kD];
     float w[kChunk][kChunk], b[kChunk][kChunk];
-    float pad[192];
+    uint32_t bad;  // something above is not finite
+    float pad[191];
 };
 static_assert(sizeof(ChunkImage) == 28 * 1024, "whole DMA pieces");
 
@@ -288,6 +312,7 @@ __global__ __launch_bounds__(256) void kda_chunk(const ChunkParams a)
 {
     __shared__ __attribute__((aligned(16))) float ks[kChunk][kD], qs[kChunk][kD], es[kChunk][kD];
     __shared__ float as[kChunk][kChunk + 1], bs[kChunk][kChunk + 1], beta[kChunk];
+    __shared__ uint32_t bad;
     const uint32_t tid = threadIdx.x, h = blockIdx.x, c = a.c0 + blockIdx.y;
     uint32_t t0, np;
     chunk_of(a, c, t0, np);
@@ -309,6 +334,8 @@ __global__ __launch_bounds__(256) void kda_chunk(const ChunkParams a)
     }
     if (tid < kChunk)
         beta[tid] = tid < np ? a.s.beta[(size_t)(t0 + tid) * a.s.heads + h] : 0.0f;
+    if (tid == 0)
+        bad = 0;
     __syncthreads();
     // Row s of 16 lanes, 8 channels a lane: p = E(t, s) k_s, one more factor a step.
     const uint32_t s = tid >> 4, l = tid & 15, first = __builtin_amdgcn_readfirstlane(s);
@@ -340,6 +367,7 @@ __global__ __launch_bounds__(256) void kda_chunk(const ChunkParams a)
         bs[t][s] = 0.0f;
     __syncthreads();
     ChunkImage& out = a.image[(size_t)blockIdx.y * a.s.heads + h];
+    float z = 0.0f;  // stays 0 while what is added, times 0, is finite
     {
         // the running products: 128 threads forward, 128 backward, a channel each
         const uint32_t i = tid & 127;
@@ -348,15 +376,20 @@ __global__ __launch_bounds__(256) void kda_chunk(const ChunkParams a)
             #pragma unroll
             for (uint32_t t = 0; t < kChunk; ++t) {
                 p *= es[t][i];
-                out.kg[t][i] = p * ks[t][i];
-                out.qg[t][i] = p * qs[t][i];
+                const float kg = p * ks[t][i], qg = p * qs[t][i];
+                out.kg[t][i] = kg;
+                out.qg[t][i] = qg;
+                z = fmaf(kg, 0.0f, fmaf(qg, 0.0f, z));
             }
             out.last[i] = p;
+            z = fmaf(p, 0.0f, z);
         } else {
             #pragma unroll
             for (uint32_t n = 0; n < kChunk; ++n) {
                 const uint32_t t = kChunk - 1 - n;
-                out.ke[t][i] = p * ks[t][i];
+                const float ke = p * ks[t][i];
+                out.ke[t][i] = ke;
+                z = fmaf(ke, 0.0f, z);
                 p *= es[t][i];
             }
         }
@@ -371,9 +404,16 @@ __global__ __launch_bounds__(256) void kda_chunk(const ChunkParams a)
                 x = fmaf(-as[t][r], w[r], x);
             w[t] = x * beta[t];
             out.w[t][tid] = w[t];
+            z = fmaf(w[t], 0.0f, z);
         }
     }
-    out.b[tid >> 4][tid & 15] = bs[tid >> 4][tid & 15];
+    const float b = bs[tid >> 4][tid & 15];
+    out.b[tid >> 4][tid & 15] = b;
+    if (fmaf(b, 0.0f, z) != 0.0f)  // (not a number is not equal to anything)
+        bad = 1;
+    __syncthreads();
+    if (tid == 0)
+        out.bad = bad;
 }
 
 __device__ __forceinline__ f32x4 mfma4(float x, float y, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, c, 0, 0, 0); }
@@ -396,6 +436,8 @@ __global__ __launch_bounds__(448) void kda_scan_chunks(const ChunkParams a)
         float v[kChunk][kChunk];
     };
     __shared__ __attribute__((aligned(1024))) Stage st[kSlots];
+    static_assert(sizeof(RowsLds<kScanLanes>) <= sizeof(st) && kD / (256 / kScanLanes) == kD / 16, "scan_rows' LDS and grid");
+    __shared__ uint32_t left;                  // the tokens are left to scan_rows
     __shared__ f32x4 pu[4][64], pq[2][4][64];  // the waves' shares of (Gamma k) S and (Gamma q) S
     __shared__ f32x4 pd[2][64];                // d
     const uint32_t tid = threadIdx.x, lane = tid & 63, h = blockIdx.x, j0 = blockIdx.y * 16;
@@ -403,11 +445,11 @@ __global__ __launch_bounds__(448) void kda_scan_chunks(const ChunkParams a)
     const size_t hq = (size_t)h * kD;
     const float scale = 0.08838834764831845f;  // 1 / sqrt(128)
     if (w == 4 || w == 5) {
-        // Chunk c into slot c % kSlots: pieces w - 4, w - 2, .. of the image, and v (both waves, the same bytes: lane 4 t
+        // Chunk n into slot n % kSlots: pieces w - 4, w - 2, .. of the image, and v (both waves, the same bytes: lane 4 t
         // + n takes columns 4 n .. of token t; past a part chunk's end the last token's, whose products are zeros'), so
         // each wave has the same number in flight. Past the last chunk the DMA reads it again (into slots not read).
-        const auto issue = [&](uint32_t c) __attribute__((always_inline)) {
-            const uint32_t slot = c % kSlots, cc = min(c, a.n - 1);
+        const auto issue = [&](uint32_t n) __attribute__((always_inline)) {
+            const uint32_t slot = n % kSlots, cc = min(n, a.n - 1);
             uint32_t t0, np;
             chunk_of(a, a.c0 + cc, t0, np);
             const uint32_t lds = __builtin_amdgcn_readfirstlane((uint32_t)reinterpret_cast<uintptr_t>(&st[slot]));
@@ -421,8 +463,8 @@ __global__ __launch_bounds__(448) void kda_scan_chunks(const ChunkParams a)
             dma16(__builtin_amdgcn_readfirstlane(lds + (uint32_t)sizeof(ChunkImage)), v,
                   min(lane >> 2, np - 1) * a.s.qkv_stride * 4 + 16 * (lane & 3));
         };
-        for (uint32_t c = 0; c < kSlots - 1; ++c)
-            issue(c);
+        for (uint32_t n = 0; n < kSlots - 1; ++n)
+            issue(n);
         // the oldest chunk in flight has landed: all but the kSlots - 2 after it
         const auto landed = [] { asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kSlots - 2) * (kPieces / 2 + 1)) : "memory"); };
         landed();
@@ -434,19 +476,21 @@ __global__ __launch_bounds__(448) void kda_scan_chunks(const ChunkParams a)
             __syncthreads();        // the end of chunk c
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        return;
-    }
-    if (w == 6) {
+    } else if (w == 6) {
         // The outputs, a chunk behind the state, so that they are not on its chain (taken by waves 0 - 3 in turn, they
         // were a quarter of a chunk's time).
         __syncthreads();
+        float z = 0.0f;  // stays 0 while every d, times 0, is finite
+        uint32_t marked = 0;
         for (uint32_t c = 0; c < a.n; ++c) {
             uint32_t t0, np;
             chunk_of(a, a.c0 + c, t0, np);
             const f32x4 br = *reinterpret_cast<const f32x4*>(&st[c % kSlots].x.b[c16][4 * g]);
+            marked |= st[c % kSlots].x.bad;
             __syncthreads();
             __syncthreads();  // the end of chunk c (pq and pd are rewritten two chunks on)
             const f32x4 d = pd[c & 1][lane];
+            z = fmaf(d[0], 0.0f, fmaf(d[1], 0.0f, fmaf(d[2], 0.0f, fmaf(d[3], 0.0f, z))));
             f32x4 o{};
             #pragma unroll
             for (int r = 0; r < 4; ++r)
@@ -458,89 +502,112 @@ __global__ __launch_bounds__(448) void kda_scan_chunks(const ChunkParams a)
                 if (4 * g + r < np)
                     at[(size_t)(4 * g + r) * a.s.inner] = o[r] * scale;
         }
-        return;
-    }
-    // Channel 32 w + 16 b + 4 g + r of column j0 + c16: state[h][j][i].
-    float* mg = a.s.state + ((size_t)h * kD + j0 + c16) * kD + 32 * w + 4 * g;
-    f32x4 m[2];
-    #pragma unroll
-    for (int b = 0; b < 2; ++b)
-        m[b] = *reinterpret_cast<const f32x4*>(mg + 16 * b);
-    __syncthreads();  // chunk 0 is staged
-    for (uint32_t c = 0; c < a.n; ++c) {
-        const Stage& s = st[c % kSlots];
-        uint32_t t0, np;
-        chunk_of(a, a.c0 + c, t0, np);
-        // this wave's shares of (Gamma k) S and (Gamma q) S, tokens 4 g + r of column c16: the second while the first
-        // goes through LDS
-        f32x4 u[2]{}, y[2]{}, kg[2], qg[2], last[2], v;
-        float ke[2][4];
-        #pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            kg[b] = *reinterpret_cast<const f32x4*>(&s.x.kg[c16][32 * w + 16 * b + 4 * g]);
-            qg[b] = *reinterpret_cast<const f32x4*>(&s.x.qg[c16][32 * w + 16 * b + 4 * g]);
-        }
-        const f32x4 wr = *reinterpret_cast<const f32x4*>(&s.x.w[c16][4 * g]);
-        #pragma unroll
-        for (int r = 0; r < 4; ++r)
-            v[r] = s.v[4 * g + r][c16];
-        #pragma unroll
-        for (int r = 0; r < 4; ++r)
-            #pragma unroll
-            for (int b = 0; b < 2; ++b)
-                u[b] = mfma4(kg[b][r], m[b][r], u[b]);
-        #pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            last[b] = *reinterpret_cast<const f32x4*>(&s.x.last[32 * w + 16 * b + 4 * g]);
-            #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                ke[b][r] = s.x.ke[4 * g + r][32 * w + 16 * b + c16];
-        }
-        pu[w][lane] = u[0] + u[1];
-        __builtin_amdgcn_sched_barrier(0);
-        #pragma unroll
-        for (int r = 0; r < 4; ++r)
-            #pragma unroll
-            for (int b = 0; b < 2; ++b)
-                y[b] = mfma4(qg[b][r], m[b][r], y[b]);
-        __syncthreads();
-        const f32x4 e = v - ((pu[0][lane] + pu[1][lane]) + (pu[2][lane] + pu[3][lane]));
-        pq[c & 1][w][lane] = y[0] + y[1];
-        f32x4 d{};
-        #pragma unroll
-        for (int r = 0; r < 4; ++r)
-            d = mfma4(wr[r], e[r], d);
-        // the update summed by itself: one rounding at the state's size a chunk
-        f32x4 n[2]{};
-        #pragma unroll
-        for (int r = 0; r < 4; ++r)
-            #pragma unroll
-            for (int b = 0; b < 2; ++b)
-                n[b] = mfma4(ke[b][r], d[r], n[b]);
-        if (w == 0)
-            pd[c & 1][lane] = d;
+        left = __ballot(marked || z != 0.0f) != 0;
+        // (scan_rows writes these outputs again)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    } else {
+        // Channel 32 w + 16 b + 4 g + r of column j0 + c16: state[h][j][i].
+        float* mg = a.s.state + ((size_t)h * kD + j0 + c16) * kD + 32 * w + 4 * g;
+        f32x4 m[2];
         #pragma unroll
         for (int b = 0; b < 2; ++b)
+            m[b] = *reinterpret_cast<const f32x4*>(mg + 16 * b);
+        __syncthreads();  // chunk 0 is staged
+        for (uint32_t c = 0; c < a.n; ++c) {
+            const Stage& s = st[c % kSlots];
+            uint32_t t0, np;
+            chunk_of(a, a.c0 + c, t0, np);
+            // this wave's shares of (Gamma k) S and (Gamma q) S, tokens 4 g + r of column c16: the second while the first
+            // goes through LDS
+            f32x4 u[2]{}, y[2]{}, kg[2], qg[2], last[2], v;
+            float ke[2][4];
+            #pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                kg[b] = *reinterpret_cast<const f32x4*>(&s.x.kg[c16][32 * w + 16 * b + 4 * g]);
+                qg[b] = *reinterpret_cast<const f32x4*>(&s.x.qg[c16][32 * w + 16 * b + 4 * g]);
+            }
+            const f32x4 wr = *reinterpret_cast<const f32x4*>(&s.x.w[c16][4 * g]);
             #pragma unroll
             for (int r = 0; r < 4; ++r)
-                m[b][r] = fmaf(m[b][r], last[b][r], n[b][r]);
-        if (a.s.snap && t0 + np == a.s.snap) {
-            float* sg = a.s.snap_state + ((size_t)h * kD + j0 + c16) * kD + 32 * w + 4 * g;
+                v[r] = s.v[4 * g + r][c16];
+            #pragma unroll
+            for (int r = 0; r < 4; ++r)
+                #pragma unroll
+                for (int b = 0; b < 2; ++b)
+                    u[b] = mfma4(kg[b][r], m[b][r], u[b]);
+            #pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                last[b] = *reinterpret_cast<const f32x4*>(&s.x.last[32 * w + 16 * b + 4 * g]);
+                #pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    ke[b][r] = s.x.ke[4 * g + r][32 * w + 16 * b + c16];
+            }
+            pu[w][lane] = u[0] + u[1];
+            __builtin_amdgcn_sched_barrier(0);
+            #pragma unroll
+            for (int r = 0; r < 4; ++r)
+                #pragma unroll
+                for (int b = 0; b < 2; ++b)
+                    y[b] = mfma4(qg[b][r], m[b][r], y[b]);
+            __syncthreads();
+            const f32x4 e = v - ((pu[0][lane] + pu[1][lane]) + (pu[2][lane] + pu[3][lane]));
+            pq[c & 1][w][lane] = y[0] + y[1];
+            f32x4 d{};
+            #pragma unroll
+            for (int r = 0; r < 4; ++r)
+                d = mfma4(wr[r], e[r], d);
+            // the update summed by itself: one rounding at the state's size a chunk
+            f32x4 n[2]{};
+            #pragma unroll
+            for (int r = 0; r < 4; ++r)
+                #pragma unroll
+                for (int b = 0; b < 2; ++b)
+                    n[b] = mfma4(ke[b][r], d[r], n[b]);
+            if (w == 0)
+                pd[c & 1][lane] = d;
             #pragma unroll
             for (int b = 0; b < 2; ++b)
-                *reinterpret_cast<f32x4*>(sg + 16 * b) = m[b];
+                #pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    m[b][r] = fmaf(m[b][r], last[b][r], n[b][r]);
+            if (a.s.snap && t0 + np == a.s.snap) {
+                float* sg = a.s.snap_state + ((size_t)h * kD + j0 + c16) * kD + 32 * w + 4 * g;
+                #pragma unroll
+                for (int b = 0; b < 2; ++b)
+                    *reinterpret_cast<f32x4*>(sg + 16 * b) = m[b];
+            }
+            __syncthreads();
         }
-        __syncthreads();
+        __syncthreads();  // wave 6 has seen the last chunk
+        if (!__builtin_amdgcn_readfirstlane(left)) {
+            #pragma unroll
+            for (int b = 0; b < 2; ++b)
+                *reinterpret_cast<f32x4*>(mg + 16 * b) = m[b];
+            return;
+        }
+        uint32_t t0, t1, np;
+        chunk_of(a, a.c0 + a.n - 1, t1, np);
+        t1 += np;
+        chunk_of(a, a.c0, t0, np);
+        ScanParams r = a.s;
+        r.q += (size_t)t0 * r.qkv_stride;
+        r.k += (size_t)t0 * r.qkv_stride;
+        r.v += (size_t)t0 * r.qkv_stride;
+        r.g += (size_t)t0 * r.inner;
+        r.o += (size_t)t0 * r.inner;
+        r.beta += (size_t)t0 * r.heads;
+        r.tokens = t1 - t0;
+        r.snap = r.snap > t0 && r.snap <= t1 ? r.snap - t0 : 0;
+        scan_rows<kScanLanes>(r, *reinterpret_cast<RowsLds<kScanLanes>*>(&st[0]));
+        return;
     }
-    #pragma unroll
-    for (int b = 0; b < 2; ++b)
-        *reinterpret_cast<f32x4*>(mg + 16 * b) = m[b];
+    __syncthreads();
 }
 
 // Token counts from which the chunks are the faster kernels (32 heads: 96 tokens 21.7 us token by token, 18.2 by chunks;
-// 200 40 and 27; 512 93 and 49; 4096 716 and 367), and the workspace a launch's images take at most: longer runs go in
-// several launches, whose images stay in the last-level cache (73 chunks of 32 heads: 29 us to make, bound by their
-// traffic, and 83 us to run, 1.1 us a chunk of LDS and barrier latencies around 28 MFMAs a wave).
+// 200 40 and 27; 512 93 and 49; 4096 716 and 356), and the workspace a launch's images take at most: longer runs go in
+// several launches, whose images stay in the last-level cache (73 chunks of 32 heads: 30 us to make, bound by their
+// traffic, and 81 us to run, 1.1 us a chunk of LDS and barrier latencies around 28 MFMAs a wave).
 constexpr uint32_t kChunkTokens = 96;
 constexpr size_t kChunkBytes = 64u << 20;
 
@@ -556,8 +623,6 @@ uint32_t chunks_a_launch(const mako_scan_args* a)
 {
     return (uint32_t)std::min<size_t>({chunks_of(a), std::max<size_t>(1, kChunkBytes / chunk_bytes(a)), 65535});
 }
-
-constexpr int kScanLanes = 16;  // lanes a state row: 8 values a lane, one wave a SIMD at 32 heads
 
 bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
@@ -592,10 +657,13 @@ int scan_core(const mako_scan_args* a, const float* q, const float* k, const flo
         return fail(MAKO_EINVAL, "kda_scan: %u heads exceed the grid", a->heads);
     ScanParams p{q, k, v, g, beta, state, o, snap_state, a->tokens, a->qkv_stride, a->inner, a->heads, a->snap};
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    // chunks, where there is a workspace to be had (a capture, no memory or a caller's shorter one: token by token) and
-    // v's rows suit 16-byte DMA from 32-bit offsets
+    // chunks, where there is a workspace to be had (a capture, no memory or a caller's shorter one: token by token), v's
+    // rows suit 16-byte DMA from 32-bit offsets, and v and the first state outlast a launch that is left to scan_rows
     const size_t bytes = scan_bytes(a);
-    if (bytes && al16(v) && a->qkv_stride < (1u << 25)) {
+    const size_t v_end = (size_t)(a->tokens - 1) * a->qkv_stride + (size_t)a->heads * kD,
+                 o_end = (size_t)(a->tokens - 1) * a->inner + (size_t)a->heads * kD;
+    if (bytes && al16(v) && a->qkv_stride < (1u << 25) && (o >= v + v_end || v >= o + o_end) &&
+        !(a->snap && snap_state == state)) {
         if (ChunkImage* ws = static_cast<ChunkImage*>(work.try_get(kWsScan, bytes, s))) {
             const uint32_t n = chunks_of(a), per = chunks_a_launch(a);
             for (uint32_t c = 0; c < n; c += per) {

@@ -341,16 +341,37 @@ def idx_dots(q, pooled, dots, *, tokens, heads, dim, pools, stride, stream=None)
     _check(lib().mako_idx_dots(ctypes.byref(a), tokens, _ptr(q), _ptr(pooled), _ptr(dots), _stream(stream)))
 
 
-def proj_bf16(w, x, y, *, t, k, n, ldx=0, ldy=0, split=0, stream=None):
-    """mako_proj_bf16: w bfloat16 [n][k], x float32 or bfloat16 [t][ldx], y float32 [t][ldy]."""
-    a = GemmArgs(t, k, n, 2 * k, ldy, ldx)
-    _check(lib().mako_proj_bf16(ctypes.byref(a), dtype_code(x), split, _ptr(w), _ptr(x), _ptr(y), _stream(stream)))
+def proj_bf16_workspace(*, t, k, n, x_dtype, ldx=0, ldy=0, split=0):
+    """mako_proj_bf16_workspace for the call proj_bf16 would make with x of x_dtype (F32 / BF16)."""
+    return lib().mako_proj_bf16_workspace(ctypes.byref(GemmArgs(t, k, n, 2 * k, ldy, ldx)), x_dtype, split)
+
+
+def proj_bf16(w, x, y, *, t, k, n, ldx=0, ldy=0, split=0, stream=None, workspace=LIBRARY):
+    """mako_proj_bf16: w bfloat16 [n][k], x float32 or bfloat16 [t][ldx], y float32 [t][ldy]; with workspace (a tensor,
+    or None), mako_proj_bf16_ws."""
+    args = [ctypes.byref(GemmArgs(t, k, n, 2 * k, ldy, ldx)), dtype_code(x), split, _ptr(w), _ptr(x), _ptr(y)]
+    if isinstance(workspace, str):
+        _check(lib().mako_proj_bf16(*args, _stream(stream)))
+    else:
+        _check(lib().mako_proj_bf16_ws(*args, _ptr(workspace), _nbytes(workspace), _stream(stream)))
+
+
+def _scan_args(tokens, heads, qkv_stride, inner, snap, head_dim):
+    return ScanArgs(head_dim, tokens, qkv_stride or heads * head_dim, inner or heads * head_dim, heads, snap)
+
+
+def kda_scan_workspace(*, tokens, heads, qkv_stride=None, inner=None, snap=0, head_dim=128):
+    """mako_kda_scan_workspace for the call kda_scan would make with these arguments."""
+    return lib().mako_kda_scan_workspace(ctypes.byref(_scan_args(tokens, heads, qkv_stride, inner, snap, head_dim)))
 
 
 def kda_scan(q, k, v, g, beta, state, o, *, tokens, heads, qkv_stride=None, inner=None, snap=0, snap_state=None,
-             head_dim=128, stream=None):
+             head_dim=128, stream=None, workspace=LIBRARY):
     """mako_kda_scan: float32 q, k, v rows qkv_stride apart, g and o rows inner apart, beta [tokens][heads], state
-    [heads][head_dim][head_dim] (transposed, updated in place)."""
-    a = ScanArgs(head_dim, tokens, qkv_stride or heads * head_dim, inner or heads * head_dim, heads, snap)
-    _check(lib().mako_kda_scan(ctypes.byref(a), _ptr(q), _ptr(k), _ptr(v), _ptr(g), _ptr(beta), _ptr(state), _ptr(o),
-                               _ptr(snap_state), _stream(stream)))
+    [heads][head_dim][head_dim] (transposed, updated in place); with workspace (a tensor, or None), mako_kda_scan_ws."""
+    args = [ctypes.byref(_scan_args(tokens, heads, qkv_stride, inner, snap, head_dim)), _ptr(q), _ptr(k), _ptr(v), _ptr(g),
+            _ptr(beta), _ptr(state), _ptr(o), _ptr(snap_state)]
+    if isinstance(workspace, str):
+        _check(lib().mako_kda_scan(*args, _stream(stream)))
+    else:
+        _check(lib().mako_kda_scan_ws(*args, _ptr(workspace), _nbytes(workspace), _stream(stream)))

@@ -182,3 +182,147 @@ def test_chunks_under_capture():
         torch.cuda.synchronize()
         assert_close(o.cpu().numpy(), want_o, "o")
         assert_close(st.cpu().numpy(), want_st, "state")
+
+
+def both_routes(host, *, T, H, snap=0):
+    """Outputs, state and snapshot by chunks, and token by token (a call without a workspace)."""
+    out = []
+    need = M.kda_scan_workspace(tokens=T, heads=H, snap=snap)
+    assert need > 0, "the call does not go by chunks"
+    for ws in (torch.empty(need, dtype=torch.uint8, device="cuda"), None):
+        q, k, v, g, beta, st = (dev(x) for x in host)
+        o = torch.full_like(v, 7.0)
+        sn = torch.full_like(st, 7.0)
+        print(f"kda_scan T={T} H={H} snap={snap} workspace={ws is not None}", flush=True)
+        M.kda_scan(q, k, v, g, beta, st, o, tokens=T, heads=H, snap=snap, snap_state=sn, workspace=ws)
+        torch.cuda.synchronize()
+        out.append([x.cpu().numpy() for x in (o, st, sn)])
+    return out
+
+
+def assert_same_where_finite(by_chunks, by_token):
+    """Not finite in the same places, and elsewhere within the tolerance of each other that each has of the oracle."""
+    for what, got, want in zip(("o", "state", "snapshot"), by_chunks, by_token):
+        fin = np.isfinite(want)
+        assert np.array_equal(np.isfinite(got), fin), f"{what}: {int((np.isfinite(got) != fin).sum())} places differ"
+        err = np.abs(got[fin].astype(np.float64) - want[fin])
+        assert np.all(err <= 2 * (ATOL + RTOL * np.abs(want[fin]))), f"{what}: worst {err.max():.3e}"
+
+
+@pytest.mark.parametrize("value", ["nan", "inf", "-inf"])
+@pytest.mark.parametrize("what,t", [("q", 72), ("k", 72), ("v", 72), ("v", 0), ("v", 129), ("g", 72), ("beta", 72),
+                                    ("state", 0)])
+def test_a_value_that_is_not_finite_stays_causal(what, t, value):
+    """One value of head 1 that is not finite, at a token inside a chunk, at the first or the last (in a part chunk):
+    by chunks it reaches the outputs, the state and the snapshot that it reaches token by token, and the outputs before
+    its token and the other heads are as without it."""
+    T, H, snap = 130, 3, 75
+    host = inputs(np.random.default_rng(80), T, H, scale_state=0.3)
+    clean = [x.copy() for x in host]
+    x = host[("q", "k", "v", "g", "beta", "state").index(what)]
+    if what == "state":
+        x[1, 4, 9] = float(value)  # column 4 of the state's transpose
+    elif what == "beta":
+        x[t, 1] = float(value)
+    else:
+        x[t, D + 9] = float(value)
+    by_chunks, by_token = both_routes(host, T=T, H=H, snap=snap)
+    assert_same_where_finite(by_chunks, by_token)
+    want, _, _ = O.kda_scan(*clean[:5], clean[5].astype(np.float64), tokens=T, heads=H)
+    assert_close(by_chunks[0][:t], want[:t], "o before the token")
+    for h in (0, 2):
+        assert_close(by_chunks[0][:, h * D:(h + 1) * D], want[:, h * D:(h + 1) * D], f"o of head {h}")
+
+
+def test_growth_past_f32_over_a_state_of_zero():
+    """A channel that no key and no state uses grows by e^12 a token: past f32 within a chunk (e^192), never by the
+    recurrence, whose state there stays 0."""
+    T, H = 130, 3
+    host = inputs(np.random.default_rng(81), T, H)
+    q, k, v, g, beta, state = host
+    g[:, 9] = 12.0
+    k[:, 9] = 0.0
+    by_chunks, by_token = both_routes(host, T=T, H=H)
+    assert_same_where_finite(by_chunks, by_token)
+    want_o, want_st, _ = O.kda_scan(q, k, v, g, beta, np.zeros((H, D, D)), tokens=T, heads=H)
+    assert_close(by_chunks[0], want_o, "o")
+    assert_close(by_chunks[1], want_st, "state")
+
+
+@pytest.mark.parametrize("snap", [1100, 1104, 1105, 1536])
+def test_chunks_in_several_launches(snap):
+    """64 heads' images of 16 tokens take 1.75 MiB, so 1600 tokens go in launches of 36 chunks, three of them: a snapshot
+    in the second launch (inside a chunk, at its edge, one token past it) and in the third; and a value that is not
+    finite in the second, which goes on token by token, with the third after it."""
+    T, H = 1600, 64
+    host = inputs(np.random.default_rng(snap), T, H, scale_state=0.3)
+    q, k, v, g, beta, state = host
+    image = 28 * 1024 * H
+    assert M.kda_scan_workspace(tokens=T, heads=H, snap=snap) == (64 << 20) // image * image and (64 << 20) // image == 36
+    o, st, sn = run(q, k, v, g, beta, state, T=T, H=H, snap=snap)
+    for h in (0, 31, 63):
+        sl = slice(h * D, (h + 1) * D)
+        want_o, want_st, want_sn = O.kda_scan(*(np.ascontiguousarray(x[:, sl]) for x in (q, k, v, g)),
+                                              np.ascontiguousarray(beta[:, h:h + 1]), state[h:h + 1].astype(np.float64),
+                                              tokens=T, heads=1, snap=snap)
+        assert_close(o[:, sl], want_o, f"o head {h}")
+        assert_close(st[h], want_st[0], f"state head {h}")
+        assert_close(sn[h], want_sn[0], f"snapshot head {h}")
+    v[1000, 31 * D + 3] = float("nan")
+    assert_same_where_finite(*both_routes(host, T=T, H=H, snap=snap))
+
+
+@pytest.mark.parametrize("cut", ["exact", "short", "misaligned", "none"])
+def test_scan_workspace(cut):
+    """The bytes asked for: the library's own result; one less, a start off 16 bytes or none: token by token."""
+    T, H, snap = 200, 2, 33
+    host = inputs(np.random.default_rng(82), T, H, scale_state=0.3)
+    need = M.kda_scan_workspace(tokens=T, heads=H, snap=snap)
+    buf = torch.zeros(need + 16, dtype=torch.uint8, device="cuda")
+    ws = {"exact": buf[:need], "short": buf[:need - 1], "misaligned": buf[8:], "none": None}[cut]
+    res = []
+    for w in (M.LIBRARY if cut == "exact" else None, ws):
+        q, k, v, g, beta, st = (dev(x) for x in host)
+        o, sn = torch.full_like(v, 7.0), torch.full_like(st, 7.0)
+        M.kda_scan(q, k, v, g, beta, st, o, tokens=T, heads=H, snap=snap, snap_state=sn, workspace=w)
+        torch.cuda.synchronize()
+        res.append((o, st, sn))
+    assert all(torch.equal(a, b) for a, b in zip(*res))
+    assert int(buf[need:].sum()) == 0 and (cut == "exact" or int(buf.sum()) == 0)
+
+
+def test_chunks_under_capture_with_a_workspace():
+    """With the caller's workspace a captured call goes by chunks, and each replay has the eager call's bits."""
+    rng = np.random.default_rng(83)
+    T, H = 130, 2
+    host = inputs(rng, T, H, scale_state=0.3)
+    q, k, v, g, beta, st = (dev(x) for x in host)
+    state0, o = st.clone(), torch.empty_like(v)
+    ws = torch.empty(M.kda_scan_workspace(tokens=T, heads=H), dtype=torch.uint8, device="cuda")
+    M.kda_scan(q, k, v, g, beta, st, o, tokens=T, heads=H, workspace=ws)
+    torch.cuda.synchronize()
+    want_o, want_st = o.clone(), st.clone()
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        M.kda_scan(q, k, v, g, beta, st, o, tokens=T, heads=H, stream=s.cuda_stream, workspace=ws)
+    for _ in range(3):
+        st.copy_(state0)
+        o.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(o, want_o) and torch.equal(st, want_st)
+
+
+def test_outputs_in_the_place_of_v():
+    """o in v's buffer, and the snapshot in the state's: as with buffers of their own, with a value that is not finite in
+    the middle too."""
+    T, H, snap = 130, 2, 40
+    host = inputs(np.random.default_rng(84), T, H, scale_state=0.3)
+    host[2][70, 3] = float("nan")
+    _, (want_o, want_st, _) = both_routes(host, T=T, H=H, snap=snap)
+    q, k, v, g, beta, st = (dev(x) for x in host)
+    M.kda_scan(q, k, v, g, beta, st, v, tokens=T, heads=H, snap=snap, snap_state=st)
+    torch.cuda.synchronize()
+    assert_same_where_finite((v.cpu().numpy(), st.cpu().numpy()), (want_o, want_st))

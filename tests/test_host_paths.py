@@ -99,8 +99,8 @@ def proj(t, stream, k=4096, n=4096):
 
 
 def scan(tokens, stream):
-    x = tensor(torch.float32)
-    M.kda_scan(x, x, x, x, x, x, x, tokens=tokens, heads=4, stream=stream)
+    x, o = tensor(torch.float32), tensor(torch.float32, 0x40000000)
+    M.kda_scan(x, x, x, x, x, x, o, tokens=tokens, heads=4, stream=stream)
 
 
 # a call whose launches pass a workspace on, and one that needs more of it
