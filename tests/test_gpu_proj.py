@@ -26,7 +26,7 @@ def abs_bits(b):
     return np.asarray(b, np.uint16) & np.uint16(0x7FFF)
 
 
-def run_proj(rng, t, k, n, x_dtype, split, ldx=0, ldy=0, scale=1.0):
+def run_proj(rng, t, k, n, x_dtype, split, ldx=0, ldy=0, scale=1.0, workspace=M.LIBRARY):
     ldx_, ldy_ = ldx or k, ldy or n
     w = O.to_bf16_bits(rng.standard_normal((n, k)) * 0.05)
     xf = (rng.standard_normal((t, ldx_)) * scale).astype(np.float32)
@@ -36,7 +36,7 @@ def run_proj(rng, t, k, n, x_dtype, split, ldx=0, ldy=0, scale=1.0):
     y = torch.full((t, ldy_), SENTINEL, dtype=torch.float32, device="cuda")
     print(f"proj t={t} k={k} n={n} x={'f32' if x_dtype == O.F32 else 'bf16'} split={split} ldx={ldx} ldy={ldy}",
           flush=True)
-    M.proj_bf16(wd, xd, y, t=t, k=k, n=n, ldx=ldx, ldy=ldy, split=split)
+    M.proj_bf16(wd, xd, y, t=t, k=k, n=n, ldx=ldx, ldy=ldy, split=split, workspace=workspace)
     torch.cuda.synchronize()
     got = y.cpu().numpy()
     want = O.proj_bf16(x, w, t=t, k=k, n=n, ldx=ldx, ldy=ldy, x_dtype=x_dtype, split=split,
@@ -62,7 +62,7 @@ CASES = [
     (1, 64, 1, O.F32, 0, 0, 0),
     (600, 512, 700, O.F32, 1, 520, 0),      # the split over several 128-row tiles
     (1100, 192, 2048, O.F32, 0, 0, 0),      # more tiles than the 8 XCDs take evenly
-    # bf16 activations with 2, 4 and 6 chunks of 32 (each of the prologue's and the tail's DMA waits), part tiles
+    # bf16 activations of one, two and three K stages, part tiles
     (200, 64, 130, O.BF16, 0, 0, 0),
     (129, 128, 200, O.BF16, 0, 136, 0),
     (70, 192, 257, O.BF16, 0, 0, 260),
@@ -131,16 +131,23 @@ def test_few_rows(t, k, n, ldx, ldy, xd, split):
     assert (got[:, n:] == SENTINEL).all(), "a column past n was written"
 
 
-@pytest.mark.parametrize("t,k,n,ldx,ldy", [
-    (100, 64, 130, 0, 0), (65, 576, 257, 584, 260),   # 64 x 64 tiles: fewer K stages than the ring, and more
-    (300, 192, 4100, 0, 0), (290, 448, 4090, 456, 0),  # 64 x 128
-    (900, 128, 4100, 0, 0), (1000, 320, 4090, 328, 4092),  # 128 x 128
-    (2000, 64, 4090, 0, 0), (1990, 256, 4100, 0, 0),   # 128 x 256
-])
+# Calls by the kernel that takes their bf16 rows (f32 rows after round_rows) on 256 compute units, which
+# tests/test_host_paths.py checks: t, k, n, ldx, ldy. Part tiles in both dimensions; K stages (64 values) fewer than the
+# ring has, as many and more; for proj_dma one, two and three (its prologue's and tail's waits), and a strided x.
+TILES = {
+    "proj_ring<64, 64, 8>": [(100, 64, 130, 0, 0), (65, 576, 257, 584, 260)],
+    "proj_ring<64, 128, 6>": [(300, 192, 4100, 0, 0), (290, 448, 4090, 456, 0)],
+    "proj_ring<128, 128, 4>": [(850, 128, 4100, 0, 0), (1000, 320, 4090, 328, 4092)],
+    "proj_ring<128, 256, 3>": [(900, 128, 4100, 0, 0), (2000, 64, 4090, 0, 0), (1990, 320, 4090, 328, 0)],
+    "proj_dma": [(1990, 256, 4100, 0, 0), (1990, 64, 4100, 0, 0), (1990, 128, 4100, 136, 0), (2500, 192, 4090, 0, 4092)],
+}
+
+
+@pytest.mark.parametrize("t,k,n,ldx,ldy", [c for calls in TILES.values() for c in calls])
 @pytest.mark.parametrize("xd,split", [(O.BF16, 0), (O.F32, 0), (O.F32, 1)], ids=["bf16", "f32", "split"])
 def test_ring_tiles(t, k, n, ldx, ldy, xd, split):
-    """proj_ring's tiles with part tiles in both dimensions, and the rounding pass before them for f32 rows; 40 rows
-    (the last one among them) against the oracle."""
+    """The DMA kernels' tiles, and the rounding pass before them for f32 rows; 40 rows (the last one among them) against
+    the oracle."""
     rng = np.random.default_rng(t + k)
     ld = ldx or k
     w = O.to_bf16_bits(rng.standard_normal((n, k)) * 0.05)
@@ -161,7 +168,63 @@ def test_ring_tiles(t, k, n, ldx, ldy, xd, split):
     assert_sum_close(got[rows][:, :n], want[:, :n], (4 if split else 2) * k * U * mag[:, :n], "proj")
 
 
-@pytest.mark.parametrize("t,split", [(60, 1), (300, 0)])
+# f32 rows of calls that are given no workspace, by kernel: t, k, n, split, ldx, ldy
+NO_WORKSPACE = {
+    "proj_few<4, true, true>": [(50, 192, 77, 1, 200, 80), (64, 64, 16, 1, 0, 0)],
+    "proj_few<4, true, false>": [(33, 576, 49, 0, 584, 60)],
+    "proj_tiles<128, true, true>": [(77, 128, 96, 1, 0, 0), (600, 512, 700, 1, 520, 0), (257, 64, 515, 1, 72, 520)],
+    "proj_tiles<256, true, false>": [(256, 4096, 256, 0, 0, 0), (300, 320, 330, 0, 328, 340), (1100, 192, 2048, 0, 0, 0),
+                                     (65, 64, 1, 0, 0, 0)],
+}
+
+
+@pytest.mark.parametrize("case", [c for calls in NO_WORKSPACE.values() for c in calls],
+                         ids=lambda c: "t{}k{}n{}{}".format(*c[:3], "s" if c[3] else ""))
+def test_f32_rows_without_a_workspace(case):
+    """The kernels that round f32 rows as they load them."""
+    t, k, n, split, ldx, ldy = case
+    got, want, mag = run_proj(np.random.default_rng(t + k + n), t, k, n, O.F32, split, ldx, ldy, scale=3.0, workspace=None)
+    assert_sum_close(got[:, :n], want[:, :n], (4 if split else 2) * k * U * mag[:, :n], "proj")
+    assert (got[:, n:] == SENTINEL).all(), "a column past n was written"
+
+
+@pytest.mark.parametrize("split", [0, 1])
+def test_proj_workspace(split):
+    """The bytes asked for: the library's own result, under capture too; one byte less or a start off 16 bytes: the call
+    without a workspace; nothing written past what was given."""
+    t, k, n = 300, 256, 320
+    rng = np.random.default_rng(split)
+    w = G.to_dev(O.to_bf16_bits(rng.standard_normal((n, k)) * 0.05), O.BF16)
+    x = torch.from_numpy(rng.standard_normal((t, k)).astype(np.float32)).to("cuda")
+    need = M.proj_bf16_workspace(t=t, k=k, n=n, x_dtype=M.F32, split=split)
+    assert need == t * k * 2 * (2 if split else 1)
+    buf = torch.zeros(need + 16, dtype=torch.uint8, device="cuda")
+
+    def call(workspace, stream=None, y=None):
+        y = torch.full((t, n), SENTINEL, dtype=torch.float32, device="cuda") if y is None else y
+        M.proj_bf16(w, x, y, t=t, k=k, n=n, split=split, workspace=workspace, stream=stream)
+        return y
+
+    unrounded = call(None)
+    for ws in (buf[:need - 1], buf[8:]):
+        assert torch.equal(call(ws), unrounded)
+    assert int(buf.sum()) == 0
+    want = call(M.LIBRARY)
+    assert torch.equal(call(buf[:need]), want) and int(buf[need:].sum()) == 0
+    y = torch.empty_like(want)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        call(buf[:need], stream=s.cuda_stream, y=y)
+    for _ in range(3):
+        y.fill_(SENTINEL)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("t,split", [(60, 1), (300, 0), (300, 1)])
 def test_f32_rows_under_capture(t, split):
     """A captured call on a stream the library holds no workspace for rounds in the tiles: each replay gives the bound."""
     k, n = 256, 320

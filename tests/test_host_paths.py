@@ -2,6 +2,7 @@
 launches and runs nothing (tests/cpp/fake_hip.cpp; 256 compute units). Pointers are never read."""
 import ctypes
 import os
+import re
 import subprocess
 import threading
 import types
@@ -13,6 +14,7 @@ torch = pytest.importorskip("torch")
 from conftest import PKG, ROOT  # noqa: E402
 
 import mako_attn as M  # noqa: E402
+import test_gpu_proj as P  # noqa: E402
 
 U32 = 0xFFFFFFFF
 FAKE_SO = os.path.join(ROOT, "tests", "cpp", "bin", "libmako_attn_fakehip.so")
@@ -178,3 +180,36 @@ def test_release_frees_every_workspace_of_the_stream(hip):
     assert M.held_bytes() - before == sum(int(e[2]) for e in events(hip, "alloc"))
     M.release(stream=s)
     assert sorted(e[1] for e in events(hip, "free")) == sorted(allocs) and M.held_bytes() == before
+
+
+def kernels(L):
+    """The projection's launches, as kernel<template arguments>."""
+    out = []
+    for name in launches(L):
+        kernel = re.search(r"proj_few|proj_ring|proj_dma|proj_tiles|round_rows", name).group()
+        args = [{"0": "false", "1": "true"}[v] if t == "b" else v for t, v in re.findall(r"L([ib])(\d+)E", name)]
+        out.append(f"{kernel}<{', '.join(args)}>" if args else kernel)
+    return out
+
+
+@pytest.mark.parametrize("kernel,call", [(k, c) for k, calls in P.TILES.items() for c in calls])
+def test_projection_tiles(hip, kernel, call):
+    t, k, n, ldx, ldy = call
+    for dtype, split, rounded in ((torch.bfloat16, 0, []), (torch.float32, 0, ["round_rows<false>"]),
+                                  (torch.float32, 1, ["round_rows<true>"])):
+        hip.fake_clear()
+        M.proj_bf16(tensor(torch.bfloat16), tensor(dtype), tensor(torch.float32), t=t, k=k, n=n, ldx=ldx, ldy=ldy,
+                    split=split, stream=0x55000)
+        assert kernels(hip) == rounded + [kernel]
+
+
+@pytest.mark.parametrize("kernel,call", [(k, c) for k, calls in P.NO_WORKSPACE.items() for c in calls])
+def test_projection_without_a_workspace(hip, kernel, call):
+    t, k, n, split, ldx, ldy = call
+    for stream, workspace in ((0x55000, None), (0x56000, M.LIBRARY)):
+        hip.fake_clear()
+        hip.fake_capture(0x56000, 1)
+        M.proj_bf16(tensor(torch.bfloat16), tensor(torch.float32), tensor(torch.float32), t=t, k=k, n=n, ldx=ldx, ldy=ldy,
+                    split=split, stream=stream, workspace=workspace)
+        hip.fake_capture(0x56000, 0)
+        assert kernels(hip) == [kernel] and events(hip, "alloc") == []
