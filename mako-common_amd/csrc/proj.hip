@@ -529,10 +529,7 @@ __global__ __launch_bounds__(256) void round_rows(const float* __restrict__ x, _
 // from L2 outweighs w's.
 constexpr int kFewWaves = 8;
 constexpr uint32_t kFewRows = 64;  // at most
-// Rows up to which proj_few is the faster one, at 4096 x 4096: bf16 15.6 us at 32 rows and 18.9 at 48 (64 x 64 tiles: 18
-// for both); f32 rows 21 at 24 and 24 at 32 (rounded first, then tiles: 20.5); with the split 24 at 32, 32 at 48 and 38
-// at 64 (36 from 28 on).
-constexpr uint32_t kFewBf16 = 32, kFewF32 = 24, kFewSplit = 48;
+constexpr uint32_t kFewBf16 = 32, kFewF32 = 24, kFewSplit = 48;  // where the tiles' kernels can take the rows too (few_takes)
 
 typedef __attribute__((address_space(1))) const u32x4 global_u32x4;
 
@@ -681,12 +678,25 @@ void launch_ring(ProjParams p, hipStream_t stream)
     hipLaunchKernelGGL((proj_ring<BM, BN, NST>), dim3(8 * p.per_xcd), dim3(256), 0, stream, p);
 }
 
+// What a call's routes are chosen by; planes: 2 with the split.
+struct Size {
+    uint32_t t, k, n, planes;
+    bool f32;
+    uint32_t cus;
+};
+
+// Workgroups in rounds over the CUs, and the share of the CUs that work in them.
+struct Rounds {
+    double n, share;
+    Rounds(uint64_t groups, uint32_t cus) : n((double)((groups + cus - 1) / cus)), share((double)groups / (n * cus)) {}
+};
+
 // bf16 rows: the tile by an estimate of each one's time, rounds of workgroups times the time of their K stages, which
 // grows with the share of the CUs that work (clock and L2), and kRoundUs a round. One round at 4096 x 4096 weights
 // (64 stages), alone and on every CU: 256 x 256 78 and 109 us, 128 x 256 48 and 64, 128 x 128 28 and 36, 64 x 128 23 and
 // 26, 64 x 64 18 and 19 (two rounds 36). So t = 128 takes 18 us (79 in 256 x 256 tiles), 512 26 (82), 1000 36 (83), 2048
 // 64 (84), 3000 and 4096 the large tiles' 91 and 109.
-void launch_bf16(ProjParams p, uint32_t cus, hipStream_t stream)
+int dma_tile(const Size& z, double& best_us)
 {
     struct Tile {
         uint32_t bm, bn;
@@ -696,17 +706,64 @@ void launch_bf16(ProjParams p, uint32_t cus, hipStream_t stream)
         {256, 256, 1.14, 0.50}, {128, 256, 0.68, 0.24}, {128, 128, 0.37, 0.12}, {64, 128, 0.28, 0.10}, {64, 64, 0.20, 0.05}};
     constexpr double kRoundUs = 3;
     int best = 0;
-    double best_us = 0;
     for (int i = 0; i < 5; ++i) {
         const Tile& c = kTiles[i];
-        const uint64_t n = (uint64_t)((p.t + c.bm - 1) / c.bm) * ((p.n + c.bn - 1) / c.bn);
-        const double rounds = (double)((n + cus - 1) / std::max(cus, 1u)), share = (double)n / (rounds * cus);
-        const double us = rounds * (kRoundUs + p.planes * p.k / kEK * (c.alone + c.full * share));
+        const Rounds r((uint64_t)((z.t + c.bm - 1) / c.bm) * ((z.n + c.bn - 1) / c.bn), z.cus);
+        const double us = r.n * (kRoundUs + z.planes * z.k / kEK * (c.alone + c.full * r.share));
         if (i == 0 || us < best_us) {
             best = i;
             best_us = us;
         }
     }
+    return best;
+}
+
+// The DMA kernels with what surrounds the tiles: memory (w, once a plane, and y) beside them, and the rounding of f32 rows.
+double dma_us(const Size& z)
+{
+    double tiles;
+    dma_tile(z, tiles);
+    const double memory = (2.0 * z.k * z.n * z.planes + 4.0 * z.t * z.n) / 4.7e6;
+    const double rounding = z.f32 ? 2 + (double)z.t * z.k * (4 + 2 * z.planes) / 5e6 : 0;
+    return std::max(tiles, memory) + 0.25 * std::min(tiles, memory) + 1 + rounding;
+}
+
+// proj_few: a wave loads its share of the K chunks by U, and U past it.
+double few_us(const Size& z)
+{
+    const uint32_t u = z.t <= 16 ? 4 : z.t <= 32 ? 2 : 1, per = kFewWaves * u;
+    const double chunks = ((z.k / 64 + per - 1) / per + 1) * u, each = z.f32 ? 0.72 + 0.05 * z.t : 0.75 + 0.02 * z.t;
+    const Rounds r((z.n + 15) / 16, z.cus);
+    return 2.2 + r.n * chunks * each * (0.75 + 0.25 * r.share);
+}
+
+// proj_tiles: 128 rows a tile with the split, 256 without.
+double tiles_us(const Size& z)
+{
+    const uint32_t bm = z.planes == 2 ? 128 : 256;
+    const Rounds r((uint64_t)((z.t + bm - 1) / bm) * ((z.n + kBN - 1) / kBN), z.cus);
+    return r.n * (z.planes == 2 ? 6 + z.k / 64 * (1.69 + 0.65 * r.share) : 10 + z.k / 64 * (1.75 + 0.55 * r.share));
+}
+
+// Whether proj_few takes the call; `rounded`: f32 rows can be rounded ahead. Its workgroups each read all of x, so its
+// time grows with n / 16 over the CUs, where the tiles' grows with the read of w: past a round or two the tiles win. us,
+// w from memory, few / tiles: bf16 rows at k = 4096, t = 1: n = 4096 11.8 / 19.0, 8192 21.4 / 22.3, 16384 39 / 33, 65536
+// 146 / 114; t = 32: 16.5 / 19.5, 31 / 23, 58 / 33, 225 / 116. f32 rows t = 16: 19 / 21, 37 / 25, 72 / 35, 279 / 115;
+// with the split 19 / 37, 36 / 38, 69 / 51, 275 / 178. k = 14336, n = 4096, bf16 t = 32 48 / 59; k = 2048, n = 151936 312
+// / 139. The estimates are within 15 % of these, the split's tiles up to a third above (the second plane's read of w comes
+// in part from the last-level cache). Past kFewBf16 / F32 / Split rows the tiles win at 4096 x 4096 too (bf16
+// rows 18 at 48, few 18.9; f32 20.5 at 32, few 24; split 36 at 64, few 38); without a workspace f32 rows compare with
+// proj_tiles (at 4096 x 4096 122 and 114 with the split, few 38 at 64 rows).
+bool few_takes(const Size& z, bool rounded)
+{
+    const uint32_t most = !z.f32 ? kFewBf16 : !rounded ? kFewRows : z.planes == 2 ? kFewSplit : kFewF32;
+    return z.t <= most && few_us(z) <= (z.f32 && !rounded ? tiles_us(z) : dma_us(z));
+}
+
+void launch_bf16(ProjParams p, uint32_t cus, hipStream_t stream)
+{
+    double us;
+    const int best = dma_tile(Size{p.t, p.k, p.n, p.planes, false, cus}, us);
     switch (best) {
     case 0:
         set_tiles(p, kBN, kBN);
@@ -745,10 +802,17 @@ using namespace mako;
 
 namespace {
 
+// (with no device the routes are the MI355X's)
+Size size_of(const mako_gemm_args* a, int x_dtype, int split)
+{
+    const uint32_t cus = device_cus();
+    return {a->t, a->k, a->n, split ? 2u : 1u, x_dtype == MAKO_F32, cus ? cus : 256u};
+}
+
 // The workspace f32 rows are rounded into (0: the call's kernels round as they load).
 size_t rounded_bytes(const mako_gemm_args* a, int x_dtype, int split)
 {
-    if (x_dtype != MAKO_F32 || a->t <= (split ? kFewSplit : kFewF32))
+    if (x_dtype != MAKO_F32 || !a->t || !a->n || few_takes(size_of(a, x_dtype, split), true))
         return 0;
     const uint64_t planes = split ? 2 : 1, bytes = planes * a->t * a->k * 2;
     return bytes <= kMaxRounded && span_fits(a->t, planes * a->k, planes * a->k) && span_fits(a->n, a->k, a->k) ? bytes : 0;
@@ -780,14 +844,15 @@ int proj_core(const mako_gemm_args* a, int x_dtype, int split, const void* w, co
         return ok();
     ProjParams p{static_cast<const __bf16*>(w), x, y, a->t, a->k, a->n, ldy, ldx, 0, 0, 0, 0, 1};
     const hipStream_t s = static_cast<hipStream_t>(stream);
+    const Size z = size_of(a, x_dtype, split);
     if (x_dtype == MAKO_BF16) {
         if (!span_fits(a->t, ldx, a->k) || !span_fits(a->n, a->k, a->k))
             return fail(MAKO_EINVAL, "proj: rows of %u (x) and %u (w) values are too long for 32-bit tile offsets", ldx,
                         a->k);
-        if (p.t <= kFewBf16)
+        if (few_takes(z, true))
             launch_few<false, false>(p, s);
         else
-            launch_bf16(p, device_cus(), s);
+            launch_bf16(p, z.cus, s);
         return check_launch("proj");
     }
     // f32 rows: rounded once into the workspace and then as bf16 rows; where it cannot be had (a capture, no memory, a
@@ -806,11 +871,11 @@ int proj_core(const mako_gemm_args* a, int x_dtype, int split, const void* w, co
             p.x = ws;
             p.ldx = (uint32_t)planes * a->k;
             p.planes = (uint32_t)planes;
-            launch_bf16(p, device_cus(), s);
+            launch_bf16(p, z.cus, s);
             return check_launch("proj");
         }
     }
-    if (p.t <= kFewRows)
+    if (few_takes(z, false))
         split ? launch_few<true, true>(p, s) : launch_few<true, false>(p, s);
     else if (split)
         launch_proj<128, true, true>(p, s);

@@ -143,6 +143,28 @@ TILES = {
 }
 
 
+# A few rows by kernel: x dtype, split, t, k, n. proj_few up to a round or two of its n / 16 workgroups over 256 compute
+# units, the tiles for wider weights.
+FEW = {
+    "proj_few<1, false, false>": [(O.BF16, 0, 1, 4096, 4096), (O.BF16, 0, 16, 14336, 4096), (O.BF16, 0, 1, 1024, 1024)],
+    "proj_few<2, false, false>": [(O.BF16, 0, 32, 4096, 4090)],
+    "proj_few<1, true, false>": [(O.F32, 0, 1, 4096, 8192)],
+    "proj_few<1, true, true>": [(O.F32, 1, 16, 4096, 4096), (O.F32, 1, 1, 4096, 12290)],
+    "proj_few<4, true, true>": [(O.F32, 1, 48, 4096, 4096)],
+    "proj_ring<64, 64, 8>": [(O.BF16, 0, 1, 1024, 16370), (O.BF16, 0, 32, 576, 16384), (O.F32, 0, 16, 1024, 16380),
+                             (O.F32, 1, 33, 4096, 8190)],
+    "proj_ring<64, 128, 6>": [(O.BF16, 0, 7, 256, 28670), (O.F32, 0, 24, 256, 28672), (O.F32, 1, 17, 256, 28674)],
+}
+
+
+@pytest.mark.parametrize("case", [c for calls in FEW.values() for c in calls],
+                         ids=lambda c: "{}{}t{}k{}n{}".format("f32" if c[0] == O.F32 else "bf16", "s" if c[1] else "", *c[2:]))
+def test_few_rows_by_width(case):
+    xd, split, t, k, n = case
+    got, want, mag = run_proj(np.random.default_rng(n), t, k, n, xd, split)
+    assert_sum_close(got, want, (4 if split else 2) * k * U * mag, "proj")
+
+
 @pytest.mark.parametrize("t,k,n,ldx,ldy", [c for calls in TILES.values() for c in calls])
 @pytest.mark.parametrize("xd,split", [(O.BF16, 0), (O.F32, 0), (O.F32, 1)], ids=["bf16", "f32", "split"])
 def test_ring_tiles(t, k, n, ldx, ldy, xd, split):
@@ -170,7 +192,7 @@ def test_ring_tiles(t, k, n, ldx, ldy, xd, split):
 
 # f32 rows of calls that are given no workspace, by kernel: t, k, n, split, ldx, ldy
 NO_WORKSPACE = {
-    "proj_few<4, true, true>": [(50, 192, 77, 1, 200, 80), (64, 64, 16, 1, 0, 0)],
+    "proj_few<4, true, true>": [(50, 192, 77, 1, 200, 80), (64, 192, 16, 1, 0, 0)],
     "proj_few<4, true, false>": [(33, 576, 49, 0, 584, 60)],
     "proj_tiles<128, true, true>": [(77, 128, 96, 1, 0, 0), (600, 512, 700, 1, 520, 0), (257, 64, 515, 1, 72, 520)],
     "proj_tiles<256, true, false>": [(256, 4096, 256, 0, 0, 0), (300, 320, 330, 0, 328, 340), (1100, 192, 2048, 0, 0, 0),

@@ -203,6 +203,14 @@ def test_projection_tiles(hip, kernel, call):
         assert kernels(hip) == rounded + [kernel]
 
 
+@pytest.mark.parametrize("kernel,call", [(k, c) for k, calls in P.FEW.items() for c in calls])
+def test_projection_of_a_few_rows(hip, kernel, call):
+    xd, split, t, k, n = call
+    M.proj_bf16(tensor(torch.bfloat16), tensor(torch.float32 if xd == P.O.F32 else torch.bfloat16), tensor(torch.float32),
+                t=t, k=k, n=n, split=split, stream=0x55000)
+    assert kernels(hip)[-1] == kernel
+
+
 @pytest.mark.parametrize("kernel,call", [(k, c) for k, calls in P.NO_WORKSPACE.items() for c in calls])
 def test_projection_without_a_workspace(hip, kernel, call):
     t, k, n, split, ldx, ldy = call
