@@ -718,14 +718,17 @@ int dma_tile(const Size& z, double& best_us)
     return best;
 }
 
-// The DMA kernels with what surrounds the tiles: memory (w, once a plane, and y) beside them, and the rounding of f32 rows.
+// The DMA kernels with what surrounds the tiles: the read of w and the writing of y, beside the tiles or, with the split
+// (w is read twice), in part after them, and the rounding of f32 rows.
 double dma_us(const Size& z)
 {
     double tiles;
     dma_tile(z, tiles);
-    const double memory = (2.0 * z.k * z.n * z.planes + 4.0 * z.t * z.n) / 4.7e6;
+    const double bytes = 2.0 * z.k * z.n + 4.0 * z.t * z.n;
     const double rounding = z.f32 ? 2 + (double)z.t * z.k * (4 + 2 * z.planes) / 5e6 : 0;
-    return std::max(tiles, memory) + 0.25 * std::min(tiles, memory) + 1 + rounding;
+    if (z.planes == 2)
+        return 1.7 + 0.91 * tiles + 0.14e-6 * bytes + rounding;
+    return 1 + std::max(tiles, bytes / 4.7e6) + 0.25 * std::min(tiles, bytes / 4.7e6) + rounding;
 }
 
 // proj_few: a wave loads its share of the K chunks by U, and U past it.
@@ -742,7 +745,21 @@ double tiles_us(const Size& z)
 {
     const uint32_t bm = z.planes == 2 ? 128 : 256;
     const Rounds r((uint64_t)((z.t + bm - 1) / bm) * ((z.n + kBN - 1) / kBN), z.cus);
-    return r.n * (z.planes == 2 ? 6 + z.k / 64 * (1.69 + 0.65 * r.share) : 10 + z.k / 64 * (1.75 + 0.55 * r.share));
+    if (z.planes == 1)
+        return r.n * (10 + z.k / 64 * (1.75 + 0.55 * r.share));
+    const double tiles = r.n * (5.8 + z.k / 64 * (1.64 + 0.27 * r.share)), memory = (2.0 * z.k * z.n + 4.0 * z.t * z.n) / 3.9e6;
+    return 1.4 + std::max(tiles, memory) + 0.12 * std::min(tiles, memory);
+}
+
+// Whether the DMA kernels take f32 rows, rounded ahead, before proj_tiles. Without the split always; with it they read w
+// twice, and proj_tiles, which reads it once, is the faster one where w is large and the rows are few, and where its
+// tiles come out at whole rounds and K is short. us, rounded ahead / proj_tiles: t = 65, k = 4096, n = 4096 37 / 113, 28672
+// 83 / 117, 65536 233 / 156; k = 2048, n = 151936 245 / 211; t = 2000, k = n = 4096 134 / 132, k = 512 29 / 24; t = 4096, k
+// = n = 4096 235 / 260. Over 415 such calls (t 48 to 4096, k 64 to 14336, n 1024 to 151936) the estimates are within 8 %
+// and 4 % on the average; the slower one is taken in 15, by 5 % to 14 % in seven.
+bool dma_takes(const Size& z)
+{
+    return z.planes == 1 || dma_us(z) <= 1.02 * tiles_us(z);
 }
 
 // Whether proj_few takes the call; `rounded`: f32 rows can be rounded ahead. Its workgroups each read all of x, so its
@@ -756,8 +773,9 @@ double tiles_us(const Size& z)
 // proj_tiles (at 4096 x 4096 122 and 114 with the split, few 38 at 64 rows).
 bool few_takes(const Size& z, bool rounded)
 {
-    const uint32_t most = !z.f32 ? kFewBf16 : !rounded ? kFewRows : z.planes == 2 ? kFewSplit : kFewF32;
-    return z.t <= most && few_us(z) <= (z.f32 && !rounded ? tiles_us(z) : dma_us(z));
+    const bool dma = !z.f32 || (rounded && dma_takes(z));
+    const uint32_t most = !dma ? kFewRows : !z.f32 ? kFewBf16 : z.planes == 2 ? kFewSplit : kFewF32;
+    return z.t <= most && few_us(z) <= (dma ? dma_us(z) : tiles_us(z));
 }
 
 void launch_bf16(ProjParams p, uint32_t cus, hipStream_t stream)
@@ -812,7 +830,8 @@ Size size_of(const mako_gemm_args* a, int x_dtype, int split)
 // The workspace f32 rows are rounded into (0: the call's kernels round as they load).
 size_t rounded_bytes(const mako_gemm_args* a, int x_dtype, int split)
 {
-    if (x_dtype != MAKO_F32 || !a->t || !a->n || few_takes(size_of(a, x_dtype, split), true))
+    const Size z = size_of(a, x_dtype, split);
+    if (x_dtype != MAKO_F32 || !a->t || !a->n || !dma_takes(z) || few_takes(z, true))
         return 0;
     const uint64_t planes = split ? 2 : 1, bytes = planes * a->t * a->k * 2;
     return bytes <= kMaxRounded && span_fits(a->t, planes * a->k, planes * a->k) && span_fits(a->n, a->k, a->k) ? bytes : 0;

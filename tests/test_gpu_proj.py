@@ -131,16 +131,20 @@ def test_few_rows(t, k, n, ldx, ldy, xd, split):
     assert (got[:, n:] == SENTINEL).all(), "a column past n was written"
 
 
-# Calls by the kernel that takes their bf16 rows (f32 rows after round_rows) on 256 compute units, which
-# tests/test_host_paths.py checks: t, k, n, ldx, ldy. Part tiles in both dimensions; K stages (64 values) fewer than the
+# Calls by the kernel that takes their bf16 rows (f32 rows after round_rows, but for SPLIT_TILES) on 256 compute units,
+# which tests/test_host_paths.py checks: t, k, n, ldx, ldy. Part tiles in both dimensions; K stages (64 values) fewer than the
 # ring has, as many and more; for proj_dma one, two and three (its prologue's and tail's waits), and a strided x.
 TILES = {
     "proj_ring<64, 64, 8>": [(100, 64, 130, 0, 0), (65, 576, 257, 584, 260)],
     "proj_ring<64, 128, 6>": [(300, 192, 4100, 0, 0), (290, 448, 4090, 456, 0)],
     "proj_ring<128, 128, 4>": [(850, 128, 4100, 0, 0), (1000, 320, 4090, 328, 4092)],
-    "proj_ring<128, 256, 3>": [(900, 128, 4100, 0, 0), (2000, 64, 4090, 0, 0), (1990, 320, 4090, 328, 0)],
+    "proj_ring<128, 256, 3>": [(900, 128, 4100, 0, 0), (2000, 64, 4090, 0, 0), (1990, 320, 4090, 328, 0),
+                               (1000, 320, 4100, 328, 0)],
     "proj_dma": [(1990, 256, 4100, 0, 0), (1990, 64, 4100, 0, 0), (1990, 128, 4100, 136, 0), (2500, 192, 4090, 0, 4092)],
 }
+
+# those that proj_tiles takes with the split
+SPLIT_TILES = [(900, 128, 4100, 0, 0), (2000, 64, 4090, 0, 0), (1990, 320, 4090, 328, 0)]
 
 
 # A few rows by kernel: x dtype, split, t, k, n. proj_few up to a round or two of its n / 16 workgroups over 256 compute
@@ -154,6 +158,7 @@ FEW = {
     "proj_ring<64, 64, 8>": [(O.BF16, 0, 1, 1024, 16370), (O.BF16, 0, 32, 576, 16384), (O.F32, 0, 16, 1024, 16380),
                              (O.F32, 1, 33, 4096, 8190)],
     "proj_ring<64, 128, 6>": [(O.BF16, 0, 7, 256, 28670), (O.F32, 0, 24, 256, 28672), (O.F32, 1, 17, 256, 28674)],
+    "proj_tiles<128, true, true>": [(O.F32, 1, 33, 128, 65536), (O.F32, 1, 65, 256, 40962)],
 }
 
 
