@@ -673,13 +673,23 @@ uint32_t item_tiles(const mako_attn_args* a, uint32_t rows_wg, uint32_t qb)
     return ((last >= a->block ? a->n_k : std::min(a->n_k, last + 1)) + 63) / 64;
 }
 
+// The keys query row `row` sees.
+uint32_t first_keys(const mako_attn_args* a, uint32_t row)
+{
+    const uint32_t pos = a->q_pos0 + row;
+    return pos >= a->block ? a->n_k : std::min(a->n_k, pos + 1);
+}
+
 // An estimate in microseconds, from this kernel's times: a workgroup takes kTileUs a tile of 64 keys on an otherwise
 // idle chip and kFullUs more where every CU works (the clock drops), kWgUs around them (dispatch, prologue, epilogue)
 // and kTurnUs for each further piece; the merge kMergeUs and its read of the pieces. A plan must gain 15 %.
 // Measured at 32 / 8 heads of 128, unsplit and split: 333 rows over 9333 keys 174 -> 61 us, 100 over 32868 591 -> 70,
-// 17 over 3017 61 -> 20, 1000 over 10000 188 -> 140; 8 / 2 heads, causal 2048 rows 43 -> 28. Not split: causal 1531
-// rows of 32 heads (192 items of 1 to 24 tiles: the chip's clock and the merge take back what the shorter path gives);
-// causal 4096 rows (512 items, heavy and light in turn).
+// 17 over 3017 61 -> 20, 1000 over 10000 188 -> 140; 8 / 2 heads, causal 2048 rows 43 -> 28. Over 5090 calls of random
+// sizes that it splits (chunks, causal, bidirectional and prefix-causal rows) the time is 0.40 of the unsplit call's on
+// the average and more than 1.02 of it in 11 (1.11 at most). Not split: prefix-causal calls whose item across
+// `block` keeps most of its keys in one piece (445 rows over 1125 keys from position 3, block 59: 33 us, split 45), causal 1531
+// rows of 32 heads (192 items of 1 to 24 tiles, at most a piece a CU: by the estimate the chip's clock and the merge take
+// back most of what the shorter path gives), causal 4096 rows (512 items, heavy and light in turn).
 template <int D>
 SplitPlan split_plan(const mako_attn_args* a, uint32_t cus)
 {
@@ -703,12 +713,12 @@ SplitPlan split_plan(const mako_attn_args* a, uint32_t cus)
     uint64_t total = 0;
     for (uint32_t qb = 0; qb < n_qblk; ++qb)
         total += (uint64_t)n_hg * tiles(qb);
-    // the busiest CU's tiles: whole rounds of equal items, or a CU's share
-    const auto path = [&](uint64_t n, double longest) {
-        return even ? (double)((n + cus - 1) / cus) * longest : std::max(longest, (double)total / cus);
+    // the busiest CU's tiles: whole rounds of equal items with the longest among them, or a CU's share or the longest
+    const auto path = [&](uint64_t n, double equal, double longest) {
+        return even ? (double)((n - 1) / cus) * equal + longest : std::max(longest, (double)total / cus);
     };
     const double full_us = kFullUs * total / cus;
-    double best_us = 0.85 * (kTileUs * path(n_items, nt) + full_us + kWgUs);
+    double best_us = 0.85 * (kTileUs * path(n_items, nt, nt) + full_us + kWgUs);
     if (kTileUs * total / cus + full_us + kWgUs + kMergeUs >= best_us)
         return best;  // an even share and a merge are no shorter
     for (uint32_t np = 2; np <= 16 && nt / np >= kMinTiles; ++np) {
@@ -720,19 +730,21 @@ SplitPlan split_plan(const mako_attn_args* a, uint32_t cus)
         if (s.bytes > kMaxBytes)
             break;
         uint64_t n = 0, merged = 0;  // pieces; pieces' rows the merge reads
+        uint32_t longest = 0;        // tiles: an item with rows on both sides of `block` has a long last piece (Pieces)
         s.row0 = a->n_q;
         for (uint32_t qb = 0; qb < n_qblk; ++qb) {
-            const uint32_t k = (tiles(qb) + s.piece_tiles - 1) / s.piece_tiles;
-            n += (uint64_t)n_hg * k;
-            if (k > 1) {
-                merged += (uint64_t)k * rows_wg * a->heads;
+            const Pieces pc(tiles(qb), first_keys(a, qb * rows_wg), s.piece_tiles);
+            n += (uint64_t)n_hg * pc.np;
+            longest = std::max(longest, pc.nt - pc.start(pc.np - 1));
+            if (pc.np > 1) {
+                merged += (uint64_t)pc.np * rows_wg * a->heads;
                 s.row0 = std::min(s.row0, qb * rows_wg);
             }
         }
         // (the lists deal equal pieces evenly; of unequal ones a second round would put two long ones on a CU)
         if (!even && n > cus)
             continue;
-        const double us = kTileUs * path(n, s.piece_tiles) + full_us + kWgUs + kTurnUs * (double)((n - 1) / cus) +
+        const double us = kTileUs * path(n, s.piece_tiles, std::max(longest, s.piece_tiles)) + full_us + kWgUs + kTurnUs * (double)((n - 1) / cus) +
                           kMergeUs + merged * D * 4.0 / 4.5e6;
         if (us < best_us) {
             best_us = us;

@@ -116,7 +116,7 @@ def test_split_prefill_carries_non_finite_values(dim, dt, out, what, row, value)
 LISTS = [
     (128, 32, 8, 70, 1500, 1430, U32, O.BF16, "same", 8, 64),
     (128, 64, 16, 33, 1200, 1167, U32, O.F16, "f32", 16, 48),     # two head groups an XCD
-    (128, 32, 8, 200, 2100, 700, 800, O.BF16, "f32", 8, 136),     # prefix-causal rows: pieces of several lengths
+    (128, 32, 8, 200, 2100, 1700, 1800, O.BF16, "f32", 8, 152),     # prefix-causal rows: pieces of several lengths
     (64, 16, 16, 2048, 2048, 0, U32, O.BF16, "same", 16, 192),    # causal rows from 0, items of one piece and of two
     (64, 32, 8, 700, 4000, 3300, U32, O.F16, "same", 8, 504),     # two rounds of the XCDs' lists
     (64, 48, 12, 500, 6000, 5500, U32, O.BF16, "f32", 12, 480),   # two rounds of one list

@@ -223,3 +223,14 @@ def test_projection_without_a_workspace(hip, kernel, call):
                     split=split, stream=stream, workspace=workspace)
         hip.fake_capture(0x56000, 0)
         assert kernels(hip) == [kernel] and events(hip, "alloc") == []
+
+
+@pytest.mark.parametrize("heads,kv,n_q,n_k,q_pos0,block,split", [
+    # rows on both sides of `block` in one item of query rows: its keys past the first row's stay in one piece
+    (32, 8, 445, 1125, 3, 59, False), (16, 8, 867, 1563, 9, 99, False), (24, 24, 806, 7685, 186, 263, False),
+    (32, 8, 200, 2100, 700, 800, False), (8, 2, 200, 2100, 700, 800, True), (32, 8, 200, 2100, 1700, 1800, True),
+    (32, 8, 333, 9333, 9000, U32, True), (32, 8, 333, 9333, 0, 0, True), (32, 8, 1531, 1531, 0, U32, False),
+])
+def test_prefill_is_split_where_its_longest_piece_is_shorter(hip, heads, kv, n_q, n_k, q_pos0, block, split):
+    assert (M.attn_fwd_workspace(n_q=n_q, q_pad=n_q, n_k=n_k, k_pad=n_k, heads=heads, kv_heads=kv, q_pos0=q_pos0,
+                                 block=block, dim=128) > 0) == split
