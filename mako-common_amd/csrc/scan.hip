@@ -22,6 +22,7 @@
 // the VALU (no packed FP32 here): 7 flops a channel a row a token. This is the kernel of short runs, and of calls with no
 // workspace; long runs go by chunks of 16 tokens (below).
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "device.hpp"
@@ -604,10 +605,9 @@ __global__ __launch_bounds__(448) void kda_scan_chunks(const ChunkParams a)
     __syncthreads();
 }
 
-// Token counts from which the chunks are the faster kernels (32 heads: 96 tokens 21.7 us token by token, 18.2 by chunks;
-// 200 40 and 27; 512 93 and 49; 4096 716 and 356), and the workspace a launch's images take at most: longer runs go in
-// several launches, whose images stay in the last-level cache (73 chunks of 32 heads: 30 us to make, bound by their
-// traffic, and 81 us to run, 1.1 us a chunk of LDS and barrier latencies around 28 MFMAs a wave).
+// The workspace a launch's images take at most: longer runs go in several launches, whose images stay in the last-level
+// cache (73 chunks of 32 heads: 30 us to make, bound by their traffic, and 81 us to run, 1.1 us a chunk of LDS and barrier
+// latencies around 28 MFMAs a wave).
 constexpr uint32_t kChunkTokens = 96;
 constexpr size_t kChunkBytes = 64u << 20;
 
@@ -633,10 +633,23 @@ using namespace mako;
 
 namespace {
 
-size_t scan_bytes(const mako_scan_args* a)
+// Whether the chunks are the faster kernels, by estimates in us of both: an image 0.0124, a chunk 1.1 and a launch 2.3 for
+// each round of heads x 8 workgroups over the CUs, against 0.175 a token while those workgroups have a CU each and 0.00375
+// a token and head past that (two or three of them share a CU then, and the chunks' one a CU gains less). us, token by
+// token / by chunks: 32 heads, 96 tokens 21.2 / 17.1, 200 39 / 26, 1024 182 / 90, 4096 716 / 356; 64 heads, 96 27.1 /
+// 26.5, 100 28.1 / 28.9, 1024 245 / 186; 256 heads, 100 98 / 102, 1024 1027 / 918; 512 heads, 200 376 / 452; 1024 heads,
+// 100 396 / 632.
+bool chunks_take(const mako_scan_args* a)
 {
-    return a->heads && a->tokens >= kChunkTokens && a->snap <= a->tokens ? chunks_a_launch(a) * chunk_bytes(a) : 0;
+    if (!a->heads || a->tokens < kChunkTokens || a->snap > a->tokens)
+        return false;
+    const uint32_t cus = device_cus(), n = chunks_of(a), per = chunks_a_launch(a);
+    const double groups = 8.0 * a->heads, rounds = std::ceil(groups / (cus ? cus : 256));
+    const double chunks = 0.0124 * n * a->heads + rounds * (2.3 * ((n + per - 1) / per) + 1.1 * n);
+    return chunks <= a->tokens * std::max(0.175, 0.00375 * a->heads);
 }
+
+size_t scan_bytes(const mako_scan_args* a) { return chunks_take(a) ? chunks_a_launch(a) * chunk_bytes(a) : 0; }
 
 int scan_core(const mako_scan_args* a, const float* q, const float* k, const float* v, const float* g,
               const float* beta, float* state, float* o, float* snap_state, const Workspace& work, void* stream)

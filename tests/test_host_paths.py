@@ -234,3 +234,16 @@ def test_projection_without_a_workspace(hip, kernel, call):
 def test_prefill_is_split_where_its_longest_piece_is_shorter(hip, heads, kv, n_q, n_k, q_pos0, block, split):
     assert (M.attn_fwd_workspace(n_q=n_q, q_pad=n_q, n_k=n_k, k_pad=n_k, heads=heads, kv_heads=kv, q_pos0=q_pos0,
                                  block=block, dim=128) > 0) == split
+
+
+@pytest.mark.parametrize("heads,tokens,snap,chunks", [
+    (1, 95, 0, False), (1, 96, 0, True), (32, 96, 0, True), (32, 4096, 0, True), (64, 96, 0, True), (64, 96, 51, False),
+    (64, 100, 0, False), (64, 200, 0, True), (256, 100, 0, False), (256, 1024, 0, True), (512, 200, 0, False),
+    (1024, 100, 53, False), (1024, 200, 0, False), (4000, 1024, 0, False),
+])
+def test_scan_goes_by_chunks_where_they_are_faster(hip, heads, tokens, snap, chunks):
+    assert (M.kda_scan_workspace(tokens=tokens, heads=heads, snap=snap) > 0) == chunks
+    x, o, st = (tensor(torch.float32, a) for a in (0x100000, 1 << 44, 1 << 45))
+    M.kda_scan(x, x, x, x, x, x, o, tokens=tokens, heads=heads, snap=snap, snap_state=st, stream=0x57000)
+    assert any("kda_scan_chunks" in k for k in launches(hip)) == chunks
+    M.release(stream=0x57000)
