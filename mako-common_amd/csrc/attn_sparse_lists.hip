@@ -26,10 +26,13 @@
 // Padding is not computed. Cubes cut by the video's edge hold few valid rows in runs of 16 (the last frame layer: one
 // run of four), so a tile of 32 keys is two groups of 16 consecutive keys with a valid one, from anywhere in the
 // sequence, and a workgroup's query rows are those with an output, packed. 56 heads, 9 frames of 34 x 60 patches, 948
-// dense rows: 53 -> 43 thousand tiles a head, 4.33 -> 3.6 ms; one frame (16 of 64 rows valid) 901 -> 511 us with the
-// selection; no padding (4 frames of 32 x 32) 273 -> 276 us. Groups of 8 keys would save another 6 % of the first
-// case's tiles, at four sources a tile. The loop is bound by its chain of barrier, scores, softmax and P V (MFMA a
-// third busy at two waves a SIMD).
+// dense rows: 53 -> 43 thousand tiles a head, 4.33 -> 3.5 ms; one frame (16 of 64 rows valid) 901 -> 511 us with the
+// selection. Without padding the list costs up to 4 % over tiles of 32 keys in a row: 16 heads, 256 cubes in lists of 32
+// and 128 dense rows 612 -> 625 us, 24 heads, 100 cubes in all lists and 2000 dense rows 1128 -> 1148, 16 heads of 3000
+// dense rows 106 -> 110 (a scan before the first tile), causal lists of 32 of 256 cubes 417 -> 434. (The list's next pair
+// is read a tile ahead and the DMA's offsets are taken before the barrier: 642 -> 625, 1164 -> 1148 of these.) Groups of 8
+// keys would save another 6 % of the first case's tiles, at four sources a tile. The loop is bound by its chain of barrier,
+// scores, softmax and P V (MFMA a third busy at two waves a SIMD).
 #include "fwd64_common.hpp"
 
 namespace mako {
@@ -146,7 +149,8 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     using E = Elem<_Float16>;
     using V8 = f16x8;
     __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kLBuf];
-    __shared__ __attribute__((aligned(8))) uint32_t lst[kLList];  // the groups visited, in order: K / V byte offsets
+    // the groups visited, in order: K / V byte offsets (and a pair past them, read and not used)
+    __shared__ __attribute__((aligned(8))) uint32_t lst[kLList + 2];
     __shared__ uint32_t lcnt[2], lcut;  // lcut: the last group crosses the end of the dense rows
 
     const uint32_t tid = threadIdx.x, lane = tid & 63;
@@ -223,20 +227,23 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const bool second = 1024 * 4 + 16 * lane >= kLGroup * kLKRow;  // piece 4's lane is the second group's
     const uint32_t lbase = __builtin_amdgcn_readfirstlane((uint32_t)reinterpret_cast<uintptr_t>(lds));
     // A tile's K image and validity bytes, and its V image, into buffer buf.
-    // (ta, tb: the tile's groups; the wave's own is ta for wave 0 and tb for wave 1)
-    auto dma_k = [&](uint32_t ta, uint32_t tb, uint32_t buf) __attribute__((always_inline)) {
+    // (ta, tb: the tile's groups; the wave's own is ta for wave 0 and tb for wave 1; ko: dma_k_off, taken ahead of the
+    // barrier that the DMA waits for)
+    auto dma_k_off = [&](uint32_t ta, uint32_t tb) __attribute__((always_inline)) {
+        uint32_t ko = w == 0 ? (lane ? tb : ta) / (2 * kLD) : kd[0] + (second ? tb : ta);
+        asm volatile("" : "+v"(ko));
+        return ko;
+    };
+    auto dma_k = [&](uint32_t ta, uint32_t tb, uint32_t ko, uint32_t buf) __attribute__((always_inline)) {
         const uint32_t kb = lbase + buf * kLBuf;
         const uint32_t so = w == 0 ? ta : tb;
-        if (w == 0)
-            dma16_at(kb, kd[0], so, krs);
-        else
-            dma16_at(kb + 1024 * 4, kd[0] + (second ? tb : ta), 0, krs);
+        dma16_at(kb + 1024 * 4 * w, w == 0 ? kd[0] : ko, w == 0 ? ta : 0u, krs);
 #pragma unroll
         for (int m = 1; m < 4; ++m)
             dma16_at(kb + 1024 * (4 * w + m), kd[m], so, krs);
         dma16_at(kb + 1024 * 8, kd[4], tb, krs);
         if (w == 0 && lane < 2)
-            dma16_at(kb + kLKImg + kLVImg, (lane ? tb : ta) / (2 * kLD), 0, brs);
+            dma16_at(kb + kLKImg + kLVImg, ko, 0, brs);
     };
     auto dma_v = [&](uint32_t ta, uint32_t tb, uint32_t buf) __attribute__((always_inline)) {
         const uint32_t vb = lbase + buf * kLBuf + kLKImg;
@@ -329,19 +336,22 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // The next tile's groups; both waves make the same calls, so they scan together. When the last tile is taken,
     // last_mask gets the keys it has (an odd tile's second group, and past the end of the dense rows, none).
     uint32_t last_mask = 0xffffffffu;
+    u32x2 pair{};  // lst[used], lst[used + 1], read a tile ahead
     if (tid == 0)
         lcut = 0;
     auto next_tile = [&](uint32_t& ja, uint32_t& jb) __attribute__((always_inline)) {
         if (used + 2 >= held) {
-            while (held - used < 2 && blk < n_blk)
+            while (held - used < 2 && blk < n_blk) {
                 scan();
+                pair = *reinterpret_cast<const u32x2*>(lst);
+            }
             if (used >= held)
                 return false;
         }
-        const u32x2 pair = *reinterpret_cast<const u32x2*>(lst + used);  // (used is even)
         ja = __builtin_amdgcn_readfirstlane(pair[0]);
         jb = __builtin_amdgcn_readfirstlane(pair[1]);
         used += 2;
+        pair = *reinterpret_cast<const u32x2*>(lst + used);  // (used is even)
         if (used >= held && blk >= n_blk) {
             const bool odd = used > held;
             if (odd)
@@ -412,11 +422,11 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int kk = 0; kk < 8; ++kk)
         settle(qreg[kk]);
     if (ta) {
-        dma_k(a0, a1, 0);
+        dma_k(a0, a1, dma_k_off(a0, a1), 0);
         dma_v(a0, a1, 0);
     }
     if (tb)
-        dma_k(b0, b1, 1);
+        dma_k(b0, b1, dma_k_off(b0, b1), 1);
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
     // A wave with no row to compute (tiles of at most 32 rows with an output) stages its share of each tile and keeps
     // the barriers of the other wave's loop, then leaves.
@@ -425,9 +435,10 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (bool have_l = ta; have_l;) {
             uint32_t c0 = 0, c1 = 0;
             const bool tc = tb && next_tile(c0, c1);
+            const uint32_t ko = dma_k_off(c0, c1);
             asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
             if (tc)
-                dma_k(c0, c1, bl);
+                dma_k(c0, c1, ko, bl);
             if (tb)
                 dma_v(b0, b1, bl ^ 1);
             have_l = tb;
@@ -445,11 +456,12 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     while (have) {
         uint32_t c0 = 0, c1 = 0;
         const bool tc = tb && next_tile(c0, c1);
+        const uint32_t ko = dma_k_off(c0, c1);
         // this wave's DMAs of K(t + 1) and V(t) have landed; past the barrier, the other wave's too, and neither
         // reads the slots of K(t) and V(t - 1) any more
         asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
         if (tc)
-            dma_k(c0, c1, b);
+            dma_k(c0, c1, ko, b);
         if (tb)
             dma_v(b0, b1, b ^ 1);
         // tile t's row maxima and the rescale decision
