@@ -19,7 +19,7 @@ share of the host), timed on the whole S512 case and on a bounded random sample 
 configuration, scaled to the metric's unit by the sample's share of the algorithmic work; the same sampled rows are
 the parity check of the GPU output against the oracle.
 
-  python bench.py [--steps K] [--warmup W] [--gpus 1] [--no-cpu]
+  python bench.py [--steps K] [--warmup W] [--gpus 1] [--no-cpu] [--detail FILE]
                   [--only prefill,s512,decode,bidir,sparse,h3_sparse,h3_bidir,heads,step,gather,proj,scan,copy]
 """
 import argparse
@@ -580,10 +580,14 @@ def bench_h3_sparse(torch, M, steps, warmup, with_cpu):
     cnt64 = cnt_h.astype(np.int64)
     kvalid = np.where(np.arange(topk)[None, None, :] < ns[:, :, None], cnt64[sl], 0).sum(-1) + dense
     pairs = float((cnt64[None, :] * kvalid).sum() + H * (rows - n * 64) * int(valid_h.sum()))
-    # the tiles the kernel computes: 32-key halves of the listed cubes that hold a valid key, the dense rows
-    halves = valid_h[:n * 64].reshape(n, 2, 32).any(-1).sum(-1).astype(np.int64)
-    n_halves = np.where(np.arange(topk)[None, None, :] < ns[:, :, None], halves[sl], 0).sum(-1)
-    visited = float(64 * (32 * n_halves + dense).sum() + H * (rows - n * 64) * rows)
+    # the tiles the kernel computes: two groups of 16 keys with a valid one (of the listed cubes and the dense rows, or of
+    # all keys) by the tile's rows that have an output, 32 a wave
+    groups = np.add.reduceat(np.pad(valid_h, (0, -rows % 16)), np.arange(0, rows, 16)) > 0
+    per_cube = groups[:n * 4].reshape(n, 4).sum(-1).astype(np.int64)
+    n_dense = int(groups[n * 4:].sum())
+    keys = 32 * ((np.where(np.arange(topk)[None, None, :] < ns[:, :, None], per_cube[sl], 0).sum(-1) + n_dense + 1) // 2)
+    waves = lambda r: 32 * ((r + 31) // 32)  # noqa: E731
+    visited = float((waves(cnt64)[None, :] * keys).sum() + H * waves(rows - n * 64) * 32 * ((int(groups.sum()) + 1) // 2))
     flop = 4.0 * D * pairs
     ms_sel, kms_sel = time_launches(torch, select, steps, warmup)
     ms_att, kms_att = time_launches(torch, attend, steps, warmup)
@@ -815,8 +819,8 @@ def bench_gather(torch, M, steps, warmup):
 def bench_proj(torch, M, steps, warmup):
     """The output projection after attention at Qwen3-8B's prefill shape (src/models/qwen_text.cpp:312): 4096
     tokens x 4096 -> 4096, bf16 weights, f32 output. Three forms: bf16 activations as the attention writes them (the
-    headline of this leg), f32 activations rounded in the GEMM's loads, and f32 with the bf16 split (twice the
-    MFMA work). TFLOP/s count 2 t k n (4 t k n with the split)."""
+    headline of this leg), f32 activations (rounded by a pass of their own, part of the call), and f32 with the bf16
+    split (twice the MFMA work). TFLOP/s count 2 t k n (4 t k n with the split)."""
     t = k = n = 4096
     gen = torch.Generator(device="cuda").manual_seed(312)
     w = (torch.randn((n, k), generator=gen, device="cuda") * 0.02).to(torch.bfloat16)
@@ -841,9 +845,9 @@ def bench_proj(torch, M, steps, warmup):
 def bench_scan(torch, M, steps, warmup):
     """The gated delta rule (kda_scan) at the shape of Qwen3.5's linear-attention layers: 32 heads of 128 over 4096
     tokens, f32, q and k unit-norm per head, g a log-decay in [-0.5, 0], beta in (0, 1), the state zeroed before
-    each call. VALU work: 896 flops a (token, head, state row) (the decay, and three 128-term fused multiply-add
-    sums); the roofline is the vector f32 peak (157.3 TFLOP/s counts packed FP32, which these kernels do not use:
-    78.6 without it)."""
+    each call. Work: the recurrence's 896 flops a (token, head, state row) (the decay, and three 128-term fused
+    multiply-add sums), which the kernels of long runs do as products of 16-token chunks on the f32 matrix unit; the
+    roofline is that unit's peak, also the vector unit's with packed FP32 (157.3 TFLOP/s; 78.6 without it)."""
     T, H, D = 4096, 32, 128
     gen = torch.Generator(device="cuda").manual_seed(459)
     unit = lambda x: x / x.norm(dim=-1, keepdim=True)
@@ -884,6 +888,7 @@ def main():
                          "few_rows:N runs the n_q = N "
                          "case alone, dims:NAME one head width (d256_causal, d64_bidir)")
     ap.add_argument("--cpu", action="store_true", help="with --only: run the legs' CPU-baseline and parity parts")
+    ap.add_argument("--detail", default=None, help="write every leg's full object to this file")
     args = ap.parse_args()
     if args.gpus != 1:
         print(f"bench.py measures one GPU; --gpus {args.gpus} is not supported (the attention path is built and "
@@ -993,7 +998,7 @@ def main():
         "config": {"workload": "Qwen3-8B o_proj after a 4096-token prefill: 4096 x 4096 bf16 weights over the "
                                "attention's bf16 rows [4096][32 * 128], f32 output"}}
     line["linear_attention"] = {
-        "value": scn["tflops"], "unit": "TFLOP/s", "kernel_ms": scn["kernel_ms"], "bound": "valu",
+        "value": scn["tflops"], "unit": "TFLOP/s", "kernel_ms": scn["kernel_ms"], "bound": "mfma",
         "frac": scn["frac_of_157"], "frac_without_packed_fp32": scn["frac_of_78_6_unpacked"],
         "config": {"workload": "gated delta rule (kda_scan), 32 heads of 128 over 4096 tokens, f32, state zeroed"}}
     line["latent_decode"]["config"] = {"workload": "sparse latent decode helpers: 65536-row cache of 512-wide f16 "
@@ -1007,38 +1012,62 @@ def main():
         line["decode"]["cpu_baseline"] = dec["cpu_baseline"]
         line["decode"]["parity"] = dec["parity"]
     line["configs"] = configs_summary(line, pre, dec, few)
-    print(json.dumps(line), flush=True)
+    if args.detail:
+        with open(args.detail, "w") as f:
+            json.dump(line, f, indent=1)
+    print(json.dumps(short_line(line)), flush=True)
+
+
+def short_line(line):
+    """The printed line: the headline with its roofline, CPU baseline and parity whole, the other workloads in a few
+    numbers each. A record that keeps 8 KB of output holds all of it; --detail writes the rest."""
+    def brief(d, *keys):
+        return {k: d[k] for k in keys if k in d}
+
+    out = {k: v for k, v in line.items() if not isinstance(v, dict)}
+    out.update(brief(line, "config", "roofline", "cpu_baseline"))
+    if "parity" in line:
+        out["parity"] = {k: v for k, v in line["parity"].items() if not isinstance(v, dict)}
+    out["others"] = {
+        **{name: brief(line[name], "value", "unit", "kernel_ms", "frac", "same_bits_as_separate")
+           for name in ("head_tiles", "prefill_step_from_rows", "output_projection", "linear_attention")},
+        "latent_decode": {name: brief(v, "kernel_ms", "frac") for name, v in line["latent_decode"].items()
+                          if name != "config"}}
+    out["configs"] = line["configs"]
+    return out
 
 
 def configs_summary(line, pre, dec, few):
     """The five configurations, the other head widths and the few-row route in a few numbers each, last in the JSON
     line (so a record that keeps only the line's tail still holds them): value, unit, kernel ms, fraction of the
-    roofline, and the parity of the sampled rows (within tolerance, max abs error)."""
+    roofline, the parity of the sampled rows (within tolerance, max abs error) and the CPU baseline's value in the
+    same unit."""
     def par(p):
         return {} if not p else {"within_tolerance": p["within_tolerance"], "max_abs_err": round(p["max_abs_err"], 6)}
 
-    def entry(value, unit, kernel_ms, frac, parity):
+    def entry(value, unit, kernel_ms, frac, of):
+        cpu = of.get("cpu_baseline")
         return dict({"value": round(value, 2), "unit": unit, "kernel_ms": round(kernel_ms, 4),
-                     "frac": round(frac, 4)}, **par(parity))
+                     "frac": round(frac, 4)}, **par(of.get("parity")), **({"cpu": round(cpu["value"], 5)} if cpu else {}))
     s512, bid, spa = line["prefill_s512"], line["bidirectional"], line["block_sparse"]
     h3s, h3d = line["h3_block_sparse"], line["h3_bidirectional"]
     f1 = few["n_q=1"]
     return {
         "C1_causal_s512_f16": entry(s512["value"], "TFLOP/s", s512["roofline"]["kernel_ms"], s512["roofline"]["frac"],
-                                    s512.get("parity")),
+                                    s512),
         "C2_causal_s4096_bf16": entry(pre["tflops"], "TFLOP/s", pre["kernel_ms"], pre["roofline"]["frac"],
-                                      pre.get("parity")),
-        "C3_decode_b16": entry(dec["gbps"], "GB/s", dec["kernel_ms"], dec["roofline"]["frac"], dec.get("parity")),
+                                      pre),
+        "C3_decode_b16": entry(dec["gbps"], "GB/s", dec["kernel_ms"], dec["roofline"]["frac"], dec),
         "C4_block_sparse_s16384": entry(spa["value"], "TFLOP/s", spa["kernel_ms"], spa["roofline"]["frac"],
-                                        spa.get("parity")),
-        "C5_bidirectional_s16384": entry(bid["value"], "TFLOP/s", bid["kernel_ms"], bid["frac"], bid.get("parity")),
-        **{f"heads_{name}": entry(h["value"], "TFLOP/s", h["kernel_ms"], h["frac"], h.get("parity"))
+                                        spa),
+        "C5_bidirectional_s16384": entry(bid["value"], "TFLOP/s", bid["kernel_ms"], bid["frac"], bid),
+        **{f"heads_{name}": entry(h["value"], "TFLOP/s", h["kernel_ms"], h["frac"], h)
            for name, h in line["other_head_widths"].items() if isinstance(h, dict) and "kernel_ms" in h},
-        "few_rows_n_q1": entry(f1["gbps"], "GB/s", f1["kernel_ms"], f1["roofline"]["frac"], f1.get("parity")),
+        "few_rows_n_q1": entry(f1["gbps"], "GB/s", f1["kernel_ms"], f1["roofline"]["frac"], f1),
         "h3_sparse_per_head_lists": entry(h3s["attention"]["tflops"], "TFLOP/s", h3s["attention"]["kernel_ms"],
-                                          h3s["roofline"]["frac"], h3s.get("parity")),
+                                          h3s["roofline"]["frac"], h3s),
         "h3_bidirectional_s19308_f16_f32": dict(entry(h3d["value"], "TFLOP/s", h3d["kernel_ms"], h3d["frac"],
-                                                      h3d.get("parity")),
+                                                      h3d),
                                                 vs_baseline=h3d["vs_baseline"],
                                                 baseline="302 ms on an Apple GPU (reference's published figure)"),
     }
