@@ -67,23 +67,20 @@ __device__ __forceinline__ float row_sum(float x)
 }
 
 // The LDS of the token-by-token scan: two batch buffers, the next batch's rows are fetched into registers while this
-// batch runs out of LDS.
+// batch runs out of LDS. (kda_scan_rows has them as arrays of their own: members of one struct cost it 1-2 %.)
+using RowsVectors = float[2][kBatch][kD];
 template <int LANES>
-struct RowsLds {
-    float q[2][kBatch][kD], k[2][kBatch][kD], e[2][kBatch][kD];
-    float v[2][kBatch][256 / LANES], b[2][kBatch], o[2][kBatch][256 / LANES];
-};
+using RowsValues = float[2][kBatch][256 / LANES];
+using RowsBetas = float[2][kBatch];
 
 // LANES lanes a state row, V = 128 / LANES values a lane in G = V / 4 runs of 4 channels: run r of lane l holds
 // channels 4 LANES r + 4 l .. + 3, so a run of the lanes of a row is 16 LANES contiguous bytes of a vector. The work of
-// threads 0 .. 255 of workgroup (head, rows); lds 16-byte aligned.
+// threads 0 .. 255 of workgroup (head, rows); the vectors 16-byte aligned.
 template <int LANES>
-__device__ __forceinline__ void scan_rows(const ScanParams& a, RowsLds<LANES>& lds)
+__device__ __forceinline__ void scan_rows(const ScanParams& a, RowsVectors& qs, RowsVectors& ks, RowsVectors& es,
+                                          RowsValues<LANES>& vs, RowsBetas& bs, RowsValues<LANES>& os)
 {
     constexpr int V = kD / LANES, G = V / 4, ROWS = 256 / LANES;
-    auto &qs = lds.q, &ks = lds.k, &es = lds.e;
-    auto &vs = lds.v, &os = lds.o;
-    auto& bs = lds.b;
     const uint32_t tid = threadIdx.x, h = blockIdx.x, j0 = blockIdx.y * ROWS, row = tid / LANES, l = tid % LANES;
     uint32_t ch[G];
     #pragma unroll
@@ -249,8 +246,11 @@ __device__ __forceinline__ void scan_rows(const ScanParams& a, RowsLds<LANES>& l
 template <int LANES>
 __global__ __launch_bounds__(256) void kda_scan_rows(const ScanParams a)
 {
-    __shared__ __attribute__((aligned(16))) RowsLds<LANES> lds;
-    scan_rows<LANES>(a, lds);
+    __shared__ __attribute__((aligned(16))) RowsVectors qs, ks, es;
+    __shared__ RowsValues<LANES> vs;
+    __shared__ RowsBetas bs;
+    __shared__ RowsValues<LANES> os;
+    scan_rows<LANES>(a, qs, ks, es, vs, bs, os);
 }
 
 constexpr int kScanLanes = 16;  // lanes a state row: 8 values a lane, one wave a SIMD at 32 heads
@@ -437,7 +437,12 @@ __global__ __launch_bounds__(448) void kda_scan_chunks(const ChunkParams a)
         float v[kChunk][kChunk];
     };
     __shared__ __attribute__((aligned(1024))) Stage st[kSlots];
-    static_assert(sizeof(RowsLds<kScanLanes>) <= sizeof(st) && kD / (256 / kScanLanes) == kD / 16, "scan_rows' LDS and grid");
+    struct RowsLds {
+        RowsVectors q, k, e;
+        RowsValues<kScanLanes> v, o;
+        RowsBetas b;
+    };
+    static_assert(sizeof(RowsLds) <= sizeof(st) && kD / (256 / kScanLanes) == kD / 16, "scan_rows' LDS and grid");
     __shared__ uint32_t left;                  // the tokens are left to scan_rows
     __shared__ f32x4 pu[4][64], pq[2][4][64];  // the waves' shares of (Gamma k) S and (Gamma q) S
     __shared__ f32x4 pd[2][64];                // d
@@ -503,9 +508,10 @@ __global__ __launch_bounds__(448) void kda_scan_chunks(const ChunkParams a)
                 if (4 * g + r < np)
                     at[(size_t)(4 * g + r) * a.s.inner] = o[r] * scale;
         }
-        left = __ballot(marked || z != 0.0f) != 0;
-        // (scan_rows writes these outputs again)
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        const bool leave = __ballot(marked || z != 0.0f) != 0;
+        left = leave;
+        if (leave)  // (scan_rows writes these outputs again)
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     } else {
         // Channel 32 w + 16 b + 4 g + r of column j0 + c16: state[h][j][i].
         float* mg = a.s.state + ((size_t)h * kD + j0 + c16) * kD + 32 * w + 4 * g;
@@ -599,7 +605,8 @@ __global__ __launch_bounds__(448) void kda_scan_chunks(const ChunkParams a)
         r.beta += (size_t)t0 * r.heads;
         r.tokens = t1 - t0;
         r.snap = r.snap > t0 && r.snap <= t1 ? r.snap - t0 : 0;
-        scan_rows<kScanLanes>(r, *reinterpret_cast<RowsLds<kScanLanes>*>(&st[0]));
+        RowsLds& lds = *reinterpret_cast<RowsLds*>(&st[0]);
+        scan_rows<kScanLanes>(r, lds.q, lds.k, lds.e, lds.v, lds.b, lds.o);
         return;
     }
     __syncthreads();
