@@ -695,7 +695,8 @@ struct Rounds {
 // grows with the share of the CUs that work (clock and L2), and kRoundUs a round. One round at 4096 x 4096 weights
 // (64 stages), alone and on every CU: 256 x 256 78 and 109 us, 128 x 256 48 and 64, 128 x 128 28 and 36, 64 x 128 23 and
 // 26, 64 x 64 18 and 19 (two rounds 36). So t = 128 takes 18 us (79 in 256 x 256 tiles), 512 26 (82), 1000 36 (83), 2048
-// 64 (84), 3000 and 4096 the large tiles' 91 and 109.
+// 64 (84), 3000 and 4096 the large tiles' 91 and 109. A tile of 128 columns must be estimated 3 % shorter than one of
+// 256: about equal, the wider one was the faster (t = 3000, k = 12288, n = 4096: 256 x 256 288, 128 x 128 306).
 int dma_tile(const Size& z, double& best_us)
 {
     struct Tile {
@@ -710,13 +711,15 @@ int dma_tile(const Size& z, double& best_us)
         const Tile& c = kTiles[i];
         const Rounds r((uint64_t)((z.t + c.bm - 1) / c.bm) * ((z.n + c.bn - 1) / c.bn), z.cus);
         const double us = r.n * (kRoundUs + z.planes * z.k / kEK * (c.alone + c.full * r.share));
-        if (i == 0 || us < best_us) {
+        if (i == 0 || us * (c.bn < 256 && kTiles[best].bn == 256 ? 1.03 : 1) < best_us) {
             best = i;
             best_us = us;
         }
     }
     return best;
 }
+
+double rounding_us(const Size& z) { return z.f32 ? 2 + (double)z.t * z.k * (4 + 2 * z.planes) / 5e6 : 0; }
 
 // The DMA kernels with what surrounds the tiles: the read of w and the writing of y, beside the tiles or, with the split
 // (w is read twice), in part after them, and the rounding of f32 rows.
@@ -725,10 +728,9 @@ double dma_us(const Size& z)
     double tiles;
     dma_tile(z, tiles);
     const double bytes = 2.0 * z.k * z.n + 4.0 * z.t * z.n;
-    const double rounding = z.f32 ? 2 + (double)z.t * z.k * (4 + 2 * z.planes) / 5e6 : 0;
     if (z.planes == 2)
-        return 1.7 + 0.91 * tiles + 0.14e-6 * bytes + rounding;
-    return 1 + std::max(tiles, bytes / 4.7e6) + 0.25 * std::min(tiles, bytes / 4.7e6) + rounding;
+        return 1.7 + 0.91 * tiles + 0.14e-6 * bytes + rounding_us(z);
+    return 1 + std::max(tiles, bytes / 4.7e6) + 0.25 * std::min(tiles, bytes / 4.7e6) + rounding_us(z);
 }
 
 // proj_few: a wave loads its share of the K chunks by U, and U past it.
@@ -741,25 +743,36 @@ double few_us(const Size& z)
 }
 
 // proj_tiles: 128 rows a tile with the split, 256 without.
-double tiles_us(const Size& z)
+Rounds tiles_rounds(const Size& z)
 {
     const uint32_t bm = z.planes == 2 ? 128 : 256;
-    const Rounds r((uint64_t)((z.t + bm - 1) / bm) * ((z.n + kBN - 1) / kBN), z.cus);
-    if (z.planes == 1)
-        return r.n * (10 + z.k / 64 * (1.75 + 0.55 * r.share));
-    const double tiles = r.n * (5.8 + z.k / 64 * (1.64 + 0.27 * r.share)), memory = (2.0 * z.k * z.n + 4.0 * z.t * z.n) / 3.9e6;
+    return Rounds((uint64_t)((z.t + bm - 1) / bm) * ((z.n + kBN - 1) / kBN), z.cus);
+}
+
+double tiles_us(const Size& z)
+{
+    const Rounds r = tiles_rounds(z);
+    const double tiles = r.n * (z.planes == 2 ? 5.8 + z.k / 64 * (1.64 + 0.27 * r.share) : 8.6 + z.k / 64 * (1.75 + 0.55 * r.share));
+    const double memory = (2.0 * z.k * z.n + 4.0 * z.t * z.n) / 3.9e6;
     return 1.4 + std::max(tiles, memory) + 0.12 * std::min(tiles, memory);
 }
 
-// Whether the DMA kernels take f32 rows, rounded ahead, before proj_tiles. Without the split always; with it they read w
-// twice, and proj_tiles, which reads it once, is the faster one where w is large and the rows are few, and where its
-// tiles come out at whole rounds and K is short. us, rounded ahead / proj_tiles: t = 65, k = 4096, n = 4096 37 / 113, 28672
-// 83 / 117, 65536 233 / 156; k = 2048, n = 151936 245 / 211; t = 2000, k = n = 4096 134 / 132, k = 512 29 / 24; t = 4096, k
-// = n = 4096 235 / 260. Over 415 such calls (t 48 to 4096, k 64 to 14336, n 1024 to 151936) the estimates are within 8 %
-// and 4 % on the average; the slower one is taken in 15, by 5 % to 14 % in seven.
+// Whether the DMA kernels take f32 rows, rounded ahead, before proj_tiles.
+// With the split they read w twice, and proj_tiles, which reads it once, is the faster one where w is large and the rows
+// are few, and where its tiles come out at whole rounds and K is short. us, rounded ahead / proj_tiles: t = 65, k = 4096, n
+// = 4096 37 / 113, 28672 83 / 117, 65536 233 / 156; k = 2048, n = 151936 245 / 211; t = 2000, k = n = 4096 134 / 132, k =
+// 512 29 / 24; t = 4096, k = n = 4096 235 / 260. Over 415 such calls (t 48 to 4096, k 64 to 14336, n 1024 to 151936) the
+// estimates are within 8 % and 4 % on the average; the slower one is taken in 15, by 5 % to 14 % in seven.
+// Without it they gain 3 to 15 % of a round that proj_tiles fills by more than half, the more the longer K, which must pay
+// for the rounding: n = 4096, t = 4096, k = 256 24.5 / 22.1, 512 32.8 / 30.1, 1024 46.1 / 46.6. Where proj_tiles leaves
+// half the chip idle, or takes several rounds, they are always faster (k = 512, t = 2000 21.5 / 28.8, n = 16384, t = 4096
+// 112 / 122), and for up to 128 rows, half of its tile.
 bool dma_takes(const Size& z)
 {
-    return z.planes == 1 || dma_us(z) <= 1.02 * tiles_us(z);
+    if (z.planes == 2)
+        return dma_us(z) <= 1.02 * tiles_us(z);
+    const Rounds r = tiles_rounds(z);
+    return r.n > 1 || r.share <= 0.5 || z.t <= 128 || rounding_us(z) <= tiles_us(z) * (0.03 + 0.12 * z.k / 1024);
 }
 
 // Whether proj_few takes the call; `rounded`: f32 rows can be rounded ahead. Its workgroups each read all of x, so its

@@ -131,7 +131,7 @@ def test_few_rows(t, k, n, ldx, ldy, xd, split):
     assert (got[:, n:] == SENTINEL).all(), "a column past n was written"
 
 
-# Calls by the kernel that takes their bf16 rows (f32 rows after round_rows, but for SPLIT_TILES) on 256 compute units,
+# Calls by the kernel that takes their bf16 rows (f32 rows after round_rows, but for the next two) on 256 compute units,
 # which tests/test_host_paths.py checks: t, k, n, ldx, ldy. Part tiles in both dimensions; K stages (64 values) fewer than the
 # ring has, as many and more; for proj_dma one, two and three (its prologue's and tail's waits), and a strided x.
 TILES = {
@@ -140,8 +140,11 @@ TILES = {
     "proj_ring<128, 128, 4>": [(850, 128, 4100, 0, 0), (1000, 320, 4090, 328, 4092)],
     "proj_ring<128, 256, 3>": [(900, 128, 4100, 0, 0), (2000, 64, 4090, 0, 0), (1990, 320, 4090, 328, 0),
                                (1000, 320, 4100, 328, 0)],
-    "proj_dma": [(1990, 256, 4100, 0, 0), (1990, 64, 4100, 0, 0), (1990, 128, 4100, 136, 0), (2500, 192, 4090, 0, 4092)],
+    "proj_dma": [(1990, 256, 4100, 0, 0), (1990, 64, 4100, 0, 0), (1990, 128, 4100, 136, 0), (2500, 192, 4090, 0, 4092),
+                 (1990, 1088, 4100, 1096, 0)],
 }
+# those whose f32 rows proj_tiles takes without the split (K too short to pay for the rounding)
+SHORT_K = [(1990, 256, 4100, 0, 0), (1990, 64, 4100, 0, 0), (1990, 128, 4100, 136, 0), (2500, 192, 4090, 0, 4092)]
 
 # those that proj_tiles takes with the split
 SPLIT_TILES = [(900, 128, 4100, 0, 0), (2000, 64, 4090, 0, 0), (1990, 320, 4090, 328, 0)]

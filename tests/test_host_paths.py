@@ -195,14 +195,16 @@ def kernels(L):
 @pytest.mark.parametrize("kernel,call", [(k, c) for k, calls in P.TILES.items() for c in calls])
 def test_projection_tiles(hip, kernel, call):
     t, k, n, ldx, ldy = call
-    for dtype, split, rounded in ((torch.bfloat16, 0, []), (torch.float32, 0, ["round_rows<false>"]),
-                                  (torch.float32, 1, ["round_rows<true>"])):
+    f32, split = ["round_rows<false>", kernel], ["round_rows<true>", kernel]
+    if call in P.SHORT_K:
+        f32 = ["proj_tiles<256, true, false>"]
+    if call in P.SPLIT_TILES:
+        split = ["proj_tiles<128, true, true>"]
+    for dtype, split, want in ((torch.bfloat16, 0, [kernel]), (torch.float32, 0, f32), (torch.float32, 1, split)):
         hip.fake_clear()
         M.proj_bf16(tensor(torch.bfloat16), tensor(dtype), tensor(torch.float32), t=t, k=k, n=n, ldx=ldx, ldy=ldy,
                     split=split, stream=0x55000)
-        if split and call in P.SPLIT_TILES:
-            rounded, kernel = [], "proj_tiles<128, true, true>"
-        assert kernels(hip) == rounded + [kernel]
+        assert kernels(hip) == want
 
 
 @pytest.mark.parametrize("kernel,call", [(k, c) for k, calls in P.FEW.items() for c in calls])
