@@ -485,7 +485,7 @@ __global__ __launch_bounds__(64) void cube_topk(const double* __restrict__ sc, u
     best_of<P>(v, lane, n, bv, bi);
     // Up to 64 picks at once: a score that exactly `need` scores exceed is found by bisection between the largest and
     // the least, and the scores past it are packed into LDS and ranked, a lane each, by counting the better ones: about
-    // 900 instructions for 48 picks of 405 where a pick at a time takes 130 each (56 heads: 258 -> 67 us). When no such
+    // 900 instructions for 48 picks of 405 where a pick at a time takes 130 each (56 heads: 258 -> 53 us). When no such
     // score is found (ties across the last pick, scores that are infinite or not numbers, or so close that the bisection
     // runs out), and for the few picks that take fewer instructions so, the picks are made one at a time.
     const uint32_t need = kk - it;
