@@ -1,6 +1,6 @@
 """ctypes binding of the CPU oracle (oracle/attn_oracle.c): test infrastructure only.
 
-Only the tests, the smoke check and the benchmark's CPU-baseline leg use this module, and only as the checker or
+Only the tests, the smoke check and the benchmark's CPU-baseline leg use this module, and only as the reference results or
 the timed CPU baseline. Inputs are numpy arrays of float32, or uint16 bit patterns of float16 / bfloat16; outputs
 are float64.
 """
